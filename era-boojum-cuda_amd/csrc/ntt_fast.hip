@@ -8,32 +8,22 @@ namespace bc {
 namespace {
 using namespace pass;
 
-// Register bounds of three workgroups per CU for the DIF (n2b) variants and
-// two for the DIT (b2n) ones, except four for the plain and n^-1 12-bit b2n
-// kernels.  With their LDS slots addressed as one base plus immediate
-// offsets, the 12-bit n2b kernels need 124 VGPRs without spills and run 4
-// workgroups per CU (LDS allows 4).  The 12-bit b2n kernels need 142 (3 per
-// CU); held to 128 they spill 14 dwords and still ran 1.5-2% faster at 4 per
-// CU on 2^16-2^21 columns.  Their coset variants spill 20-26 dwords at 128
-// and were not faster, so they keep the bound of two.
+// Register bounds: three workgroups per CU for the n2b variants and the
+// 12-bit b2n ones (160-168 VGPRs, no spills in the plain forms), two for the
+// shorter b2n ones, some of which need more.  Four per CU spills 18-20 dwords
+// in the 12-bit kernels and ran 4-5% slower.
 template <int LH, bool INV, bool DIT, int MODE, bool MC>
-__global__ __launch_bounds__(NT, DIT && LH == 12 && !MC && (MODE == MODE_NONE || MODE == MODE_NINV) ? 4
-                                 : DIT                                                           ? 2
-                                                                                                 : 3) void
+__global__ __launch_bounds__(NT, DIT && LH != 12 ? 2 : 3) void
     ntt_contig_kernel(FastArgs a) {
   __shared__ PassLds sh;
   contig_run<LH, INV, DIT, MODE, MC>(a, sh, blockIdx.x, a.tiles, gridDim.x);
 }
 
-// Three workgroups per CU as well (the coset-scaling variants included: their
-// factors live in the pass and level twists and a 16-entry LDS table, not in
-// per-thread registers), except where 168 VGPRs spill heavily: h = 6 (four
-// radix-4 groups per thread in the second level; 70-76 spilled dwords at
-// three per CU, 28-38% slower on 512 x 2^18 and 8 x 2^24 n2b calls) and b2n
-// h = 5 (16-22 dwords, 3-4% slower).  The other b2n variants spill 4-8
-// dwords at three per CU and still ran faster there than at two.
+// Three workgroups per CU for n2b h = 7 and 8 (2-6 spilled dwords; two per CU
+// was 5-6% slower on 256 x 2^20), two for the others, which spill 10-84 dwords
+// at three (b2n h = 8 runs the same at both: 0.97 ms on 256 x 2^20).
 template <int LH, bool INV, bool DIT, int MODE>
-__global__ __launch_bounds__(NT, LH == 6 || (LH == 5 && DIT) ? 2 : 3) void ntt_strided_kernel(FastArgs a) {
+__global__ __launch_bounds__(NT, LH >= 7 && !DIT ? 3 : 2) void ntt_strided_kernel(FastArgs a) {
   __shared__ PassLds sh;
   const uint64_t total = (uint64_t)a.num_cols << (a.log_n - a.log_N);
   const uint64_t p_begin = (uint64_t)blockIdx.y * a.blocks_per_wg;
@@ -88,11 +78,12 @@ hipError_t strided_dir(const FastArgs &a, bool inv, bool dit, int mode, dim3 gri
   return dit ? strided_mode<LH, false, true>(a, mode, grid, s) : strided_mode<LH, false, false>(a, mode, grid, s);
 }
 
-// Default grid of the contiguous pass: two whole rounds of resident
-// workgroups.  The tile loop is grid-strided, so a grid that is a whole
-// number of rounds leaves no partly filled last round (2048 workgroups on the
-// 768 slots of 256 CUs x 3 ran 2.67 rounds and were 4% slower on 256 x 2^20).
-// Queried once per device and direction: the n2b and b2n 12-bit kernels
+// Default grid of the contiguous pass: eight whole rounds of resident
+// workgroups.  The tile loop is grid-strided, and a SIMD with three waves
+// issues from them unevenly (two share an issue slot that the third has to
+// itself), so the work has to be handed out in several rounds: two rounds
+// were 3-8% slower on 256 x 2^20, a part-filled last round 4%.
+// Queried once per device and direction: the n2b and b2n 12-bit kernels may
 // differ in register use and so in workgroups per CU.
 constexpr int MAX_DEVICES = 64;
 std::mutex g_grid_mu;
@@ -100,7 +91,7 @@ uint32_t g_grid[MAX_DEVICES][2] = {};
 
 uint32_t default_contig_grid(bool dit) {
   int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= MAX_DEVICES) return 2048;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= MAX_DEVICES) return 6144;
   std::lock_guard<std::mutex> lk(g_grid_mu);
   uint32_t &g = g_grid[dev][dit ? 1 : 0];
   if (!g) {
@@ -112,7 +103,7 @@ uint32_t default_contig_grid(bool dit) {
              : hipOccupancyMaxActiveBlocksPerMultiprocessor(
                    &per_cu, ntt_contig_kernel<12, false, false, MODE_NONE, false>, NT, 0)) == hipSuccess &&
         cus > 0 && per_cu > 0;
-    g = ok ? (uint32_t)(2 * cus * per_cu) : 2048u;
+    g = ok ? (uint32_t)(8 * cus * per_cu) : 6144u;
   }
   return g;
 }

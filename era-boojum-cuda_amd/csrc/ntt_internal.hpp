@@ -117,7 +117,7 @@ int describe_fast_passes(const Tables &tab, const uint64_t *inputs, uint64_t *ou
 constexpr uint64_t STRIDED_MAX_GROUPS = 65535;
 uint32_t strided_groups(uint64_t pairs, uint64_t positions, uint32_t tuned_bpw, uint32_t *bpw);
 
-// max_wgs: grid cap of a contiguous pass (0: built-in 2048).
+// max_wgs: grid cap of a contiguous pass (0: built-in, whole rounds of resident workgroups).
 hipError_t launch_contig(const FastArgs &a, int log_h, bool inverse, bool dit, int mode, uint32_t max_wgs,
                          hipStream_t stream);
 hipError_t launch_strided(const FastArgs &a, int log_h, bool inverse, bool dit, int mode, uint32_t positions,

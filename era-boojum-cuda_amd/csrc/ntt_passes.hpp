@@ -28,6 +28,7 @@
 // that share it and computes it once.  n2b runs levels top-down (DIF), b2n
 // bottom-up (DIT) as the transpose.
 #pragma once
+#include "gl_lazy.hpp"
 #include "ntt_device.hpp"
 
 namespace bc {
@@ -53,11 +54,21 @@ template <int LM, bool INV> __device__ __forceinline__ void stage_level_twists(u
 }
 
 // x[i] *= tw[(i - 1) * S + rp] for i = 1..15 (tw in LDS).
-template <int LM>
-__device__ __forceinline__ void level_twist_lds(uint64_t *x, const uint64_t *tw, uint32_t rp) {
+template <int LM, gl::Reduce R>
+__device__ __forceinline__ void level_twist_lds(uint64_t *x, const uint64_t *tw, uint32_t rp, int32_t *e = nullptr) {
   constexpr uint32_t S = 1u << (LM - 4);
-#pragma unroll
-  for (int i = 1; i < 16; ++i) x[i] = gl::mul(x[i], tw[(i - 1) * S + rp]);
+  gl::mul_each<1, 15, R>(x, [&](int i) { return tw[(i - 1) * S + rp]; }, e);
+}
+
+// x[i] *= base * part[i] for all 16 points.
+template <gl::Reduce R> __device__ __forceinline__ void coset_twist(uint64_t *x, uint64_t base, const uint64_t *part) {
+  gl::unroll<4>([&](auto r) {
+    constexpr int B = 4 * decltype(r)::value;
+    uint64_t f[4] = {part[B], part[B + 1], part[B + 2], part[B + 3]};
+    const uint64_t b[4] = {base, base, base, base};
+    gl::mul_row<4, gl::ANY>(f, f, b);
+    gl::mul_row<4, R>(x + B, x + B, f);
+  });
 }
 
 // -------------------------------------------------------------------------
@@ -100,6 +111,33 @@ __device__ __forceinline__ void stage_level_twists_coset(uint64_t *dst, uint64_t
   if (threadIdx.x < S) dst0[threadIdx.x] = coset_scale_pow<MODE>(a, threadIdx.x << log_r);
 }
 
+// Column values are loaded and stored through buffer descriptors: a wave-
+// uniform base, a 32-bit per-thread offset that does not change, and the rest
+// of the address in a scalar offset, so that the 16 accesses of a tile need no
+// vector address arithmetic (three instructions and a wait state per pair of
+// loads before).  Accesses are non-temporal.
+__device__ __forceinline__ uint64_t uniform64(uint64_t v) {
+  return gl::pair64(__builtin_amdgcn_readfirstlane((uint32_t)v), __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32)));
+}
+struct Buf {
+  static constexpr int RAW_32 = 0x00020000;  // word 3: raw buffer, 32-bit data format
+  static constexpr int NT = 2;               // cache policy: non-temporal
+  using V2 = uint32_t __attribute__((ext_vector_type(2)));
+  __amdgpu_buffer_rsrc_t r;
+  __device__ __forceinline__ Buf(const uint64_t *base, uint32_t bytes)
+      : r(__builtin_amdgcn_make_buffer_rsrc((void *)uniform64((uint64_t)base), 0, (int)bytes, RAW_32)) {}
+  __device__ __forceinline__ uint64_t load(uint32_t voff, uint32_t soff) const {
+    const V2 v = __builtin_amdgcn_raw_buffer_load_b64(r, (int)voff, (int)soff, NT);
+    return gl::pair64(v.x, v.y);
+  }
+  __device__ __forceinline__ void store(uint64_t x, uint32_t voff, uint32_t soff) const {
+    V2 v;
+    v.x = (uint32_t)x;
+    v.y = (uint32_t)(x >> 32);
+    __builtin_amdgcn_raw_buffer_store_b64(v, r, (int)voff, (int)soff, NT);
+  }
+};
+
 // Column addressing: one matrix (base + c * stride) for the standalone
 // launches, or a per-column pointer table (CT) for ragged job groups.
 template <bool CT> __device__ __forceinline__ const uint64_t *in_col(const FastArgs &a, uint64_t c) {
@@ -111,37 +149,23 @@ template <bool CT> __device__ __forceinline__ uint64_t *out_col(const FastArgs &
   else return a.out + c * a.stride_out;
 }
 
-// Addressing of a contiguous-pass tile: 4096 consecutive points of one column,
-// or (MC: single-pass transforms shorter than 4096) 2^(12-h) whole columns.
-template <int LH, bool MC, bool CT> struct ContigTile {
-  const uint64_t *in;  // !MC: the tile's first input point
-  uint64_t *out;       // !MC: the tile's first output point
+// Addressing of a contiguous-pass tile: 4096 consecutive points of one column
+// (position pos0 of column col), or (MC: single-pass transforms shorter than
+// 4096) 2^(12-h) whole columns from col0 on.
+template <int LH, bool MC> struct ContigTile {
+  uint64_t col;
   uint32_t pos0, col0;
   __device__ __forceinline__ ContigTile(const FastArgs &a, uint32_t tile) {
     if constexpr (!MC) {
       const uint32_t sh = a.log_n - TILE_LOG;
-      const uint64_t col = tile >> sh;
+      col = tile >> sh;
       pos0 = (tile & ((1u << sh) - 1u)) << TILE_LOG;
-      in = in_col<CT>(a, col) + pos0;
-      out = out_col<CT>(a, col) + pos0;
       col0 = 0;
     } else {
       col0 = tile << (12 - LH);
+      col = 0;
       pos0 = 0;
-      in = nullptr;
-      out = nullptr;
     }
-  }
-  // element e of the tile; nullptr for MC slots past the last column
-  __device__ __forceinline__ const uint64_t *src(const FastArgs &a, uint32_t e) const {
-    if constexpr (!MC) return in + e;
-    const uint32_t c = col0 + (e >> LH);
-    return c < a.num_cols ? in_col<CT>(a, c) + (e & ((1u << LH) - 1u)) : nullptr;
-  }
-  __device__ __forceinline__ uint64_t *dst(const FastArgs &a, uint32_t e) const {
-    if constexpr (!MC) return out + e;
-    const uint32_t c = col0 + (e >> LH);
-    return c < a.num_cols ? out_col<CT>(a, c) + (e & ((1u << LH) - 1u)) : nullptr;
   }
   __device__ __forceinline__ uint32_t pos(uint32_t e) const {
     if constexpr (MC) return e & ((1u << LH) - 1u);
@@ -175,11 +199,38 @@ __device__ __forceinline__ void wave_lds_sync() {
 // consecutive points), or (ROW) in the wl_row mapping.
 template <int LH, bool MC, bool CT, bool ROW = false>
 __device__ __forceinline__ void contig_load(const FastArgs &a, uint32_t tile, uint32_t t, uint64_t *x) {
-  const ContigTile<LH, MC, CT> ct(a, tile);
+  const ContigTile<LH, MC> ct(a, tile);
+  if constexpr (!MC) {
+    const Buf in(in_col<CT>(a, ct.col) + ct.pos0, TILE * 8);
+    const uint32_t v = (ROW ? wl_row(t, 0) : celem<LH, 0, 4>(t, 0, 0)) * 8;
+    constexpr uint32_t STEP = ROW ? 64 * 8 : 8u << (LH - 4);
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const uint64_t *q = ct.src(a, ROW ? wl_row(t, i) : celem<LH, 0, 4>(t, 0, i));
-    x[i] = q ? __builtin_nontemporal_load(q) : 0ull;
+    for (uint32_t i = 0; i < 16; ++i) x[i] = in.load(v + i * STEP % 4096, i * STEP / 4096 * 4096);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const uint32_t e = celem<LH, 0, 4>(t, 0, i), c = ct.col0 + (e >> LH);
+      x[i] = c < a.num_cols ? __builtin_nontemporal_load(in_col<CT>(a, c) + (e & ((1u << LH) - 1u))) : 0ull;
+    }
+  }
+}
+
+// Stores a tile's 16 values per thread from the level-0 mapping.
+template <int LH, bool MC, bool CT>
+__device__ __forceinline__ void contig_store(const FastArgs &a, const ContigTile<LH, MC> &ct, uint32_t t,
+                                             const uint64_t *x) {
+  if constexpr (!MC) {
+    const Buf out(out_col<CT>(a, ct.col) + ct.pos0, TILE * 8);
+    const uint32_t v = celem<LH, 0, 4>(t, 0, 0) * 8;
+    constexpr uint32_t STEP = 8u << (LH - 4);
+#pragma unroll
+    for (uint32_t i = 0; i < 16; ++i) out.store(x[i], v + i * STEP % 4096, i * STEP / 4096 * 4096);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const uint32_t e = celem<LH, 0, 4>(t, 0, i), c = ct.col0 + (e >> LH);
+      if (c < a.num_cols) __builtin_nontemporal_store(x[i], out_col<CT>(a, c) + (e & ((1u << LH) - 1u)));
+    }
   }
 }
 
@@ -229,9 +280,19 @@ __device__ __forceinline__ void contig_run(const FastArgs &a, PassLds &sh, uint3
   auto srun = [&](int k) -> uint64_t & { return srunb[k]; };
   auto srow = [&](int i) -> uint64_t & { return srowb[i * 68]; };
 
-  // level-0 twists: 15 per thread, read from the (cache-resident) level table
-  // at each use, which keeps 30 VGPRs free
+  // level-0 twists: 15 per thread.  The plain n2b pass keeps them in
+  // registers: read at each use they wait, in order, behind the prefetch of
+  // the next tile (5-9% slower on 256 x 2^20).  b2n uses them last, when the
+  // prefetch has landed, and the coset and multi-column forms would spill;
+  // these read the (cache-resident) level table each time, which keeps 30
+  // VGPRs free.
   const uint64_t *tw0 = lvl_table<LH, INV>(a.tab) + (t & ((1u << (LH - 4)) - 1u));
+  constexpr bool TW_REGS = WL && !DIT;
+  uint64_t twr[16];
+  if constexpr (TW_REGS) {
+#pragma unroll
+    for (int i = 1; i < 16; ++i) twr[i] = tw0[(i - 1) << (LH - 4)];
+  }
   // level-1 twists (at most 240 entries) in LDS
   if constexpr (NL == 3) stage_level_twists<LH - 4, INV>(tw1, a.tab);
   const uint32_t rp1 = t & ((1u << (LH - 8)) - 1u);
@@ -249,13 +310,14 @@ __device__ __forceinline__ void contig_run(const FastArgs &a, PassLds &sh, uint3
 
   // b2n with WL loads in the wl_row mapping, everything else in level 0's
   constexpr bool ROW_LOAD = WL && DIT;
-  uint32_t tile = tile_begin;
+  uint32_t tile = __builtin_amdgcn_readfirstlane(tile_begin);
+  tile_end = __builtin_amdgcn_readfirstlane(tile_end);
   uint64_t pf[16];
   if (tile < tile_end) contig_load<LH, MC, CT, ROW_LOAD>(a, tile, t, pf);
   __syncthreads();  // tw1 and coset part factors staged
 
   for (; tile < tile_end; tile += step) {
-    const ContigTile<LH, MC, CT> ct(a, tile);
+    const ContigTile<LH, MC> ct(a, tile);
     uint64_t x[16];
 #pragma unroll
     for (int i = 0; i < 16; ++i) x[i] = pf[i];
@@ -268,48 +330,46 @@ __device__ __forceinline__ void contig_run(const FastArgs &a, PassLds &sh, uint3
       const uint32_t pos = ct.pos(celem<LH, 0, 4>(t, 0, 0));
       cfb = coset_scale_pow<MODE>(a, SC_BREV ? brev_bits(pos, a.log_n) : pos);
     }
-    if constexpr (MODE == MODE_LDE_IN) {
-#pragma unroll
-      for (int i = 0; i < 16; ++i) x[i] = gl::mul(x[i], gl::mul(cfb, sh.cf[i]));
-    } else {
-      if (a.first) {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) x[i] = gl::canon(x[i]);  // field ops take canonical values
-      }
-    }
+    if constexpr (MODE == MODE_LDE_IN) coset_twist<gl::ANY>(x, cfb, sh.cf);
 
+    // Values between levels are any u64; the pass's last operation on each
+    // makes it canonical (this pass writes the caller's outputs in n2b, and in
+    // single-pass b2n calls).
+    constexpr bool SCALE_OUT = MODE == MODE_NINV || MODE == MODE_LDE_OUT;
+    constexpr gl::Reduce LAST = SCALE_OUT ? gl::ANY : gl::CANON;
+    auto scale_out = [&](uint64_t *v) {
+      if constexpr (MODE == MODE_NINV) gl::mul_each<0, 16, gl::CANON>(v, [&](int) { return a.n_inv; });
+      if constexpr (MODE == MODE_LDE_OUT) coset_twist<gl::CANON>(v, cfb, sh.cf);
+    };
+    auto tw0_at = [&](int i) { return TW_REGS ? twr[i] : tw0[(i - 1) << (LH - 4)]; };
     if constexpr (!DIT) {
-      dft_dif<4, INV>(x);
-#pragma unroll
-      for (int i = 1; i < 16; ++i) x[i] = gl::mul(x[i], tw0[(i - 1) << (LH - 4)]);
+      gl::dft_lazy<4, INV, false, gl::ANY>(x);
+      gl::mul_each<1, 15, gl::ANY>(x, tw0_at);
 #pragma unroll
       for (int i = 0; i < 16; ++i) s0(i) = x[i];
       __syncthreads();
 #pragma unroll
       for (int i = 0; i < 16; ++i) x[i] = s1(i);
-      dft_dif<4, INV>(x);
       if constexpr (WL) {
-        level_twist_lds<LH - 4>(x, tw1, rp1);
+        gl::dft_lazy<4, INV, false, gl::ANY>(x);
+        level_twist_lds<LH - 4, gl::ANY>(x, tw1, rp1);
         // each thread rewrites the slots it read, inside its wave's region
 #pragma unroll
         for (int i = 0; i < 16; ++i) s1(i) = x[i];
         wave_lds_sync();
 #pragma unroll
         for (int k = 0; k < 16; ++k) x[k] = srun(k);
-#pragma unroll
-        for (int g = 0; g < G2; ++g) dft_dif<A2, INV>(x + g * (1 << A2));
+        gl::dft_lazy<A2, INV, false, LAST>(x);
 #pragma unroll
         for (int k = 0; k < 16; ++k) srun(k) = x[k];
         __syncthreads();  // the level-0 mapping crosses waves
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          const uint32_t e = celem<LH, 0, 4>(t, 0, i);
-          uint64_t v = s0(i);
-          if constexpr (MODE == MODE_NINV) v = gl::mul(v, a.n_inv);
-          __builtin_nontemporal_store(v, ct.dst(a, e));
-        }
+        for (int i = 0; i < 16; ++i) x[i] = s0(i);
+        scale_out(x);
+        contig_store<LH, MC, CT>(a, ct, t, x);
       } else if constexpr (NL == 3) {
-        level_twist_lds<LH - 4>(x, tw1, rp1);
+        gl::dft_lazy<4, INV, false, gl::ANY>(x);
+        level_twist_lds<LH - 4, gl::ANY>(x, tw1, rp1);
 #pragma unroll
         for (int i = 0; i < 16; ++i) s1(i) = x[i];
         __syncthreads();
@@ -317,8 +377,9 @@ __device__ __forceinline__ void contig_run(const FastArgs &a, PassLds &sh, uint3
         for (int g = 0; g < G2; ++g)
 #pragma unroll
           for (int i = 0; i < (1 << A2); ++i) x[g * (1 << A2) + i] = lds[pidx(celem<LH, 2, A2>(t, g, i))];
-#pragma unroll
-        for (int g = 0; g < G2; ++g) dft_dif<A2, INV>(x + g * (1 << A2));
+        gl::dft_lazy<A2, INV, false, LAST>(x);
+      } else {
+        gl::dft_lazy<4, INV, false, LAST>(x);
       }
       // regroup the last level's runs into the coalesced level-0 mapping
       // through LDS (each thread rewrites the slots it read, so no barrier
@@ -330,86 +391,62 @@ __device__ __forceinline__ void contig_run(const FastArgs &a, PassLds &sh, uint3
           for (int i = 0; i < (1 << AL); ++i) lds[pidx(celem<LH, LL, AL>(t, g, i))] = x[g * (1 << AL) + i];
         __syncthreads();
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          const uint32_t e = celem<LH, 0, 4>(t, 0, i);
-          uint64_t v = s0(i);
-          if constexpr (MODE == MODE_NINV) v = gl::mul(v, a.n_inv);
-          if constexpr (MODE == MODE_LDE_OUT) v = gl::mul(v, gl::mul(cfb, sh.cf[i]));
-          uint64_t *q = ct.dst(a, e);
-          if (q) __builtin_nontemporal_store(v, q);
+        for (int i = 0; i < 16; ++i) x[i] = s0(i);
+        scale_out(x);
+        contig_store<LH, MC, CT>(a, ct, t, x);
+      }
+    } else {
+      int32_t e[16];
+      e[0] = 0;  // point 0 of a level takes no twist
+      if constexpr (WL) {
+        // loaded in the wl_row mapping: regroup into runs inside the wave's region
+#pragma unroll
+        for (int i = 0; i < 16; ++i) srow(i) = x[i];
+        wave_lds_sync();
+#pragma unroll
+        for (int k = 0; k < 16; ++k) x[k] = srun(k);
+        gl::dft_lazy<A2, INV, true, gl::ANY>(x);
+#pragma unroll
+        for (int k = 0; k < 16; ++k) srun(k) = x[k];
+        wave_lds_sync();
+#pragma unroll
+        for (int i = 0; i < 16; ++i) x[i] = s1(i);
+        level_twist_lds<LH - 4, gl::LAZY>(x, tw1, rp1, e);
+        gl::dft_lazy<4, INV, true, gl::ANY, true>(x, e);
+      } else {
+        // regroup the coalesced load into the last level's runs through LDS
+#pragma unroll
+        for (int i = 0; i < 16; ++i) s0(i) = x[i];
+        __syncthreads();
+#pragma unroll
+        for (int g = 0; g < GL; ++g)
+#pragma unroll
+          for (int i = 0; i < (1 << AL); ++i) x[g * (1 << AL) + i] = lds[pidx(celem<LH, LL, AL>(t, g, i))];
+        if constexpr (NL == 3) {
+          gl::dft_lazy<A2, INV, true, gl::ANY>(x);
+#pragma unroll
+          for (int g = 0; g < G2; ++g)
+#pragma unroll
+            for (int i = 0; i < (1 << A2); ++i) lds[pidx(celem<LH, 2, A2>(t, g, i))] = x[g * (1 << A2) + i];
+          __syncthreads();
+#pragma unroll
+          for (int i = 0; i < 16; ++i) x[i] = s1(i);
+          level_twist_lds<LH - 4, gl::LAZY>(x, tw1, rp1, e);
+          gl::dft_lazy<4, INV, true, gl::ANY, true>(x, e);
+        } else {
+          gl::dft_lazy<4, INV, true, gl::ANY>(x);
         }
       }
-    } else if constexpr (WL) {
-      // loaded in the wl_row mapping: regroup into runs inside the wave's region
-#pragma unroll
-      for (int i = 0; i < 16; ++i) srow(i) = x[i];
-      wave_lds_sync();
-#pragma unroll
-      for (int k = 0; k < 16; ++k) x[k] = srun(k);
-#pragma unroll
-      for (int g = 0; g < G2; ++g) dft_dit<A2, INV>(x + g * (1 << A2));
-#pragma unroll
-      for (int k = 0; k < 16; ++k) srun(k) = x[k];
-      wave_lds_sync();
-#pragma unroll
-      for (int i = 0; i < 16; ++i) x[i] = s1(i);
-      level_twist_lds<LH - 4>(x, tw1, rp1);
-      dft_dit<4, INV>(x);
       // each thread rewrites the slots it read; the level-0 mapping crosses waves
 #pragma unroll
       for (int i = 0; i < 16; ++i) s1(i) = x[i];
       __syncthreads();
 #pragma unroll
       for (int i = 0; i < 16; ++i) x[i] = s0(i);
-#pragma unroll
-      for (int i = 1; i < 16; ++i) x[i] = gl::mul(x[i], tw0[(i - 1) << (LH - 4)]);
-      dft_dit<4, INV>(x);
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const uint32_t e = celem<LH, 0, 4>(t, 0, i);
-        uint64_t v = x[i];
-        if constexpr (MODE == MODE_NINV) v = gl::mul(v, a.n_inv);
-        __builtin_nontemporal_store(v, ct.dst(a, e));
-      }
-    } else {
-      // regroup the coalesced load into the last level's runs through LDS
-#pragma unroll
-      for (int i = 0; i < 16; ++i) s0(i) = x[i];
-      __syncthreads();
-#pragma unroll
-      for (int g = 0; g < GL; ++g)
-#pragma unroll
-        for (int i = 0; i < (1 << AL); ++i) x[g * (1 << AL) + i] = lds[pidx(celem<LH, LL, AL>(t, g, i))];
-      if constexpr (NL == 3) {
-#pragma unroll
-        for (int g = 0; g < G2; ++g) dft_dit<A2, INV>(x + g * (1 << A2));
-#pragma unroll
-        for (int g = 0; g < G2; ++g)
-#pragma unroll
-          for (int i = 0; i < (1 << A2); ++i) lds[pidx(celem<LH, 2, A2>(t, g, i))] = x[g * (1 << A2) + i];
-        __syncthreads();
-#pragma unroll
-        for (int i = 0; i < 16; ++i) x[i] = s1(i);
-        level_twist_lds<LH - 4>(x, tw1, rp1);
-      }
-      dft_dit<4, INV>(x);
-#pragma unroll
-      for (int i = 0; i < 16; ++i) s1(i) = x[i];
-      __syncthreads();
-#pragma unroll
-      for (int i = 0; i < 16; ++i) x[i] = s0(i);
-#pragma unroll
-      for (int i = 1; i < 16; ++i) x[i] = gl::mul(x[i], tw0[(i - 1) << (LH - 4)]);
-      dft_dit<4, INV>(x);
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const uint32_t e = celem<LH, 0, 4>(t, 0, i);
-        uint64_t v = x[i];
-        if constexpr (MODE == MODE_NINV) v = gl::mul(v, a.n_inv);
-        if constexpr (MODE == MODE_LDE_OUT) v = gl::mul(v, gl::mul(cfb, sh.cf[i]));
-        uint64_t *q = ct.dst(a, e);
-        if (q) __builtin_nontemporal_store(v, q);
-      }
+      gl::mul_each<1, 15, gl::LAZY>(x, tw0_at, e);
+      gl::dft_lazy<4, INV, true, LAST, true>(x, e);
+      scale_out(x);
+      contig_store<LH, MC, CT>(a, ct, t, x);
     }
     __syncthreads();  // LDS is reused by the next tile
   }
@@ -433,6 +470,7 @@ __device__ __forceinline__ void strided_run(const FastArgs &a, PassLds &sh, uint
   uint64_t *tw0 = sh.tw;
   const uint32_t t = threadIdx.x;
   const uint32_t log_r = a.log_N - LH;
+  rho = __builtin_amdgcn_readfirstlane(rho);
   const uint32_t r0 = rho << LT;
 
   // level-0 mapping: q = t % T, rp = t / T, j = i * 2^LS0 + rp
@@ -448,9 +486,8 @@ __device__ __forceinline__ void strided_run(const FastArgs &a, PassLds &sh, uint
   };
   // Element offsets from the block base (r0 included).  Level-0 mapping:
   // base0 + i * step0; last-level mapping: basel(g) + i * stepl.
-  const uint64_t step0 = 1ull << (LS0 + log_r);
+  const uint32_t log_step0 = LS0 + log_r, log_stepl = NL == 2 ? log_r : log_step0;
   const uint64_t base0 = ((uint64_t)rp0 << log_r) + q0;
-  const uint64_t stepl = NL == 2 ? (1ull << log_r) : step0;
   auto basel = [&](int g) -> uint64_t {
     if constexpr (NL == 2) return ((uint64_t)lastj(g, 0) << log_r) + lastq(g);
     else return base0;
@@ -474,23 +511,35 @@ __device__ __forceinline__ void strided_run(const FastArgs &a, PassLds &sh, uint
     if (t < 16) sh.cf[t] = coset_scale_pow<MODE>(a, t << (a.log_N - 4));
   }
 
-  // pass twist omega_N^((r0 + q) * brev_h(j)) in the last-level mapping, with
-  // n^-1 folded in when this pass carries the inverse scaling
+  // pass twist omega_N^(r brev_h(j)) in the last-level mapping, with n^-1 and
+  // the coset factor of r folded in.  T <= 256, so r = r0 + q is the same for
+  // all of a thread's values, and their j differ in four bits: register k =
+  // (g, i) has bits i at the bottom of j and bits g at its top.  So the 16
+  // twists are the thread's own power times the subset products of four
+  // powers omega_N^(r 2^m): five table powers and 15 products a workgroup
+  // instead of 16 powers and up to 48 products.
   uint64_t pt[16];
-#pragma unroll
-  for (int g = 0; g < G1; ++g) {
-    uint64_t cq = 0;
-    if constexpr (SC) cq = coset_scale_pow<MODE>(a, r0 + lastq(g));
-#pragma unroll
-    for (int i = 0; i < (1 << A1); ++i) {
-      const uint32_t j = lastj(g, i);
-      uint32_t e = ((r0 + lastq(g)) * brev_bits(j, LH)) << (32u - a.log_N);
-      if (INV) e = 0u - e;
-      uint64_t w = pow_w(a.tab, e);
-      if constexpr (MODE == MODE_NINV || MODE == MODE_LDE_OUT) w = gl::mul(w, a.n_inv);
-      if constexpr (SC) w = gl::mul(w, cq);
-      pt[g * (1 << A1) + i] = w;
-    }
+  {
+    const uint32_t r = r0 + lastq(0);
+    auto power = [&](uint32_t k) {  // omega_N^(+-r k)
+      const uint32_t e = (r * k) << (32u - a.log_N);
+      return pow_w(a.tab, INV ? 0u - e : e);
+    };
+    pt[0] = power(brev_bits(lastj(0, 0), LH));
+    if constexpr (MODE == MODE_NINV || MODE == MODE_LDE_OUT) pt[0] = gl::mul(pt[0], a.n_inv);
+    if constexpr (SC) pt[0] = gl::mul(pt[0], coset_scale_pow<MODE>(a, r));
+    // register bit m is bit m of j (m < A1: i; h = 4: the slot's bit m + LS0)
+    // or, for g, bit h - 4 + m
+    gl::unroll<4>([&](auto m) {
+      constexpr int B = decltype(m)::value, N = 1 << B;
+      constexpr int JBIT = NL == 2 ? (B < A1 ? B : LH - 4 + B) : LS0 + B;
+      const uint64_t f = power(1u << (LH - 1 - JBIT));
+      const uint64_t fs[4] = {f, f, f, f};
+      gl::unroll<(N + 3) / 4>([&](auto c) {
+        constexpr int C = 4 * decltype(c)::value, R = N < 4 ? N : 4;
+        gl::mul_row<R, gl::ANY>(pt + N + C, pt + C, fs);
+      });
+    });
   }
 
   const uint32_t blocks_per_col_log = a.log_n - a.log_N;
@@ -498,23 +547,64 @@ __device__ __forceinline__ void strided_run(const FastArgs &a, PassLds &sh, uint
   auto pair_pos = [&](uint64_t p) -> uint64_t {
     return ((p & ((1ull << blocks_per_col_log) - 1ull)) << a.log_N) + r0;
   };
-  // loads one pair's 16 values in the first level's mapping
+  // One pair's 16 values in the level-0 (DIF loads, DIT stores) or last-level
+  // mapping.  Blocks of up to 2^28 points (2 GiB) are addressed through a
+  // buffer descriptor, longer ones, whose offsets pass 32 bits, with pointers.
+  const bool buffered = a.log_N <= 28;
+  const uint32_t block_bytes = buffered ? (uint32_t)(((1ull << a.log_N) - r0) * 8) : 0u;
   auto load = [&](uint64_t p, uint64_t *v) {
     const uint64_t *in = in_col<CT>(a, p >> blocks_per_col_log) + pair_pos(p);
-    if constexpr (!DIT) {
-      const uint64_t *q = in + base0;
+    if (buffered) {
+      const Buf b(in, block_bytes);
+      if constexpr (!DIT) {
 #pragma unroll
-      for (int k = 0; k < 16; ++k, q += step0) v[k] = __builtin_nontemporal_load(q);
+        for (uint32_t k = 0; k < 16; ++k) v[k] = b.load((uint32_t)base0 * 8, k << (log_step0 + 3));
+      } else {
+#pragma unroll
+        for (int g = 0; g < G1; ++g)
+#pragma unroll
+          for (uint32_t i = 0; i < (1u << A1); ++i)
+            v[g * (1 << A1) + i] = b.load((uint32_t)basel(g) * 8, i << (log_stepl + 3));
+      }
+    } else if constexpr (!DIT) {
+#pragma unroll
+      for (uint64_t k = 0; k < 16; ++k) v[k] = __builtin_nontemporal_load(in + base0 + (k << log_step0));
     } else {
 #pragma unroll
-      for (int g = 0; g < G1; ++g) {
-        const uint64_t *q = in + basel(g);
+      for (int g = 0; g < G1; ++g)
 #pragma unroll
-        for (int i = 0; i < (1 << A1); ++i, q += stepl) v[g * (1 << A1) + i] = __builtin_nontemporal_load(q);
+        for (uint64_t i = 0; i < (1u << A1); ++i)
+          v[g * (1 << A1) + i] = __builtin_nontemporal_load(in + basel(g) + (i << log_stepl));
+    }
+  };
+  auto store = [&](uint64_t p, const uint64_t *v) {
+    uint64_t *out = out_col<CT>(a, p >> blocks_per_col_log) + pair_pos(p);
+    if (buffered) {
+      const Buf b(out, block_bytes);
+      if constexpr (DIT) {
+#pragma unroll
+        for (uint32_t k = 0; k < 16; ++k) b.store(v[k], (uint32_t)base0 * 8, k << (log_step0 + 3));
+      } else {
+#pragma unroll
+        for (int g = 0; g < G1; ++g)
+#pragma unroll
+          for (uint32_t i = 0; i < (1u << A1); ++i)
+            b.store(v[g * (1 << A1) + i], (uint32_t)basel(g) * 8, i << (log_stepl + 3));
       }
+    } else if constexpr (DIT) {
+#pragma unroll
+      for (uint64_t k = 0; k < 16; ++k) __builtin_nontemporal_store(v[k], out + base0 + (k << log_step0));
+    } else {
+#pragma unroll
+      for (int g = 0; g < G1; ++g)
+#pragma unroll
+        for (uint64_t i = 0; i < (1u << A1); ++i)
+          __builtin_nontemporal_store(v[g * (1 << A1) + i], out + basel(g) + (i << log_stepl));
     }
   };
 
+  p_begin = uniform64(p_begin);
+  p_end = uniform64(p_end);
   uint64_t pf[16];
   if (p_begin < p_end) load(p_begin, pf);
   __syncthreads();  // tw0 and coset factors staged
@@ -523,19 +613,11 @@ __device__ __forceinline__ void strided_run(const FastArgs &a, PassLds &sh, uint
 #pragma unroll
     for (int i = 0; i < 16; ++i) x[i] = pf[i];
     if (p + 1 < p_end) load(p + 1, pf);  // prefetch: in flight during this pair's math
-    uint64_t *out = out_col<CT>(a, p >> blocks_per_col_log) + pair_pos(p);
     if constexpr (!DIT) {
-      if constexpr (MODE == MODE_LDE_IN) {
-        if (a.first) x[0] = gl::canon(x[0]);  // field ops take canonical values
-#pragma unroll
-        for (int i = 1; i < 16; ++i) x[i] = gl::mul_uniform(x[i], sh.cf[i]);
-      } else if (a.first) {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) x[i] = gl::canon(x[i]);  // field ops take canonical values
-      }
-      dft_dif<4, INV>(x);
+      if constexpr (MODE == MODE_LDE_IN) gl::mul_each<1, 15, gl::ANY, true>(x, [&](int i) { return sh.cf[i]; });
+      gl::dft_lazy<4, INV, false, gl::ANY>(x);
       if constexpr (NL == 2) {
-        level_twist_lds<LH>(x, tw0, rp0);
+        level_twist_lds<LH, gl::ANY>(x, tw0, rp0);
         if constexpr (SC) x[0] = gl::mul(x[0], sh.cr[rp0]);
         // LDS row-major by j: element (q, j) at j * T + q
 #pragma unroll
@@ -546,25 +628,18 @@ __device__ __forceinline__ void strided_run(const FastArgs &a, PassLds &sh, uint
 #pragma unroll
           for (int i = 0; i < (1 << A1); ++i) x[g * (1 << A1) + i] = lds[(lastj(g, i) << LT) + lastq(g)];
         __syncthreads();  // the next iteration rewrites LDS
-#pragma unroll
-        for (int g = 0; g < G1; ++g) dft_dif<A1, INV>(x + g * (1 << A1));
+        gl::dft_lazy<A1, INV, false, gl::ANY>(x);
       }
-#pragma unroll
-      for (int g = 0; g < G1; ++g) {
-        uint64_t *q = out + basel(g);
-#pragma unroll
-        for (int i = 0; i < (1 << A1); ++i, q += stepl) {
-          const int k = g * (1 << A1) + i;
-          __builtin_nontemporal_store(gl::mul(x[k], pt[k]), q);
-        }
-      }
+      // a later pass reads these, so any u64 will do
+      gl::mul_each<0, 16, gl::ANY>(x, [&](int k) { return pt[k]; });
+      store(p, x);
     } else {
-      // the pass twist makes every value canonical
-#pragma unroll
-      for (int k = 0; k < 16; ++k) x[k] = gl::mul(x[k], pt[k]);
+      // outputs are canonical: this may be the call's last pass
+      constexpr gl::Reduce LAST = MODE == MODE_LDE_OUT ? gl::ANY : gl::CANON;
+      int32_t e[16];
+      gl::mul_each<0, 16, gl::LAZY>(x, [&](int k) { return pt[k]; }, e);
       if constexpr (NL == 2) {
-#pragma unroll
-        for (int g = 0; g < G1; ++g) dft_dit<A1, INV>(x + g * (1 << A1));
+        gl::dft_lazy<A1, INV, true, gl::ANY, true>(x, e);
 #pragma unroll
         for (int g = 0; g < G1; ++g)
 #pragma unroll
@@ -573,19 +648,16 @@ __device__ __forceinline__ void strided_run(const FastArgs &a, PassLds &sh, uint
 #pragma unroll
         for (int i = 0; i < 16; ++i) x[i] = lds[((((uint32_t)i << LS0) + rp0) << LT) + q0];
         __syncthreads();
-        level_twist_lds<LH>(x, tw0, rp0);
+        level_twist_lds<LH, gl::LAZY>(x, tw0, rp0, e);
+        e[0] = 0;
         if constexpr (SC) x[0] = gl::mul(x[0], sh.cr[rp0]);
       }
-      dft_dit<4, INV>(x);
-      uint64_t *q = out + base0;
-#pragma unroll
-      for (int i = 0; i < 16; ++i, q += step0) {
-        uint64_t v = x[i];
-        if constexpr (MODE == MODE_LDE_OUT) {
-          if (i > 0) v = gl::mul_uniform(v, sh.cf[i]);
-        }
-        __builtin_nontemporal_store(v, q);
+      gl::dft_lazy<4, INV, true, LAST, true>(x, e);
+      if constexpr (MODE == MODE_LDE_OUT) {
+        x[0] = gl::canon(x[0]);
+        gl::mul_each<1, 15, gl::CANON, true>(x, [&](int i) { return sh.cf[i]; });
       }
+      store(p, x);
     }
   }
   __syncthreads();  // LDS (tile and staged twists) is reused by the caller's next unit
