@@ -114,6 +114,7 @@ using Mask = uint64_t;
 #define GL_S_ONESK(i) "v_cndmask_b32_e64 %[t" #i "], 0, -1, %[k" #i "]\n\t"
 #define GL_S_FLO(i) "v_addc_co_u32_e64 %[lo" #i "], %[k" #i "], %[xl" #i "], %[t" #i "], %[w" #i "]\n\t"
 #define GL_S_FHI(i) "v_addc_co_u32_e64 %[hi" #i "], %[k" #i "], %[xh" #i "], 0, %[k" #i "]\n\t"
+#define GL_S_ADD(i) "v_add_co_u32_e64 %[r" #i "], %[c" #i "], %[a" #i "], %[b" #i "]\n\t"
 #define GL_S_LAZY_E(i) "v_subb_co_u32_e64 %[n" #i "], %[c" #i "], %[t" #i "], 0, %[m" #i "]\n\t"
 
 template <int N> struct Rows;
@@ -129,6 +130,11 @@ template <int N> struct Rows;
     }                                                                                                                  \
     GL_FN static void mad_eps(uint64_t *z, Mask *c, const uint32_t *f, const uint64_t *d) {                            \
       asm(GL_CAT##N(GL_S_EPS) : GL_LIST##N(GL_O_z), GL_LIST##N(GL_O_c) : GL_LIST##N(GL_I_f), GL_LIST##N(GL_I_d));      \
+    }                                                                                                                  \
+    GL_FN static void add_bit(uint32_t *r, uint32_t *t, const uint32_t *a, const uint32_t *b) {                        \
+      Mask c[N];                                                                                                       \
+      asm(GL_CAT##N(GL_S_ADD) GL_WAIT##N GL_CAT##N(GL_S_BIT)                                                           \
+          : GL_LIST##N(GL_O_r), GL_LIST##N(GL_O_t), GL_LIST##N(GL_O_c) : GL_LIST##N(GL_I_a), GL_LIST##N(GL_I_b));      \
     }                                                                                                                  \
     GL_FN static void mad_eps_carry(uint64_t *z, uint32_t *n, const uint32_t *f, const uint64_t *d,                    \
                                     const uint32_t *b) {                                                               \
@@ -239,6 +245,12 @@ template <int N> struct Rows {
   static void mad_s(uint64_t *r, Mask *c, const uint32_t *a, const uint32_t *b, const uint64_t *d) { mad(r, c, a, b, d); }
   static void mad_eps(uint64_t *z, Mask *c, const uint32_t *f, const uint64_t *d) {
     for (int i = 0; i < N; ++i) z[i] = mad1(f[i], 0xFFFFFFFFu, d[i], c[i]);
+  }
+  static void add_bit(uint32_t *r, uint32_t *t, const uint32_t *a, const uint32_t *b) {
+    for (int i = 0; i < N; ++i) {
+      r[i] = a[i] + b[i];
+      t[i] = r[i] < a[i];
+    }
   }
   static void mad_eps_carry(uint64_t *z, uint32_t *n, const uint32_t *f, const uint64_t *d, const uint32_t *b) {
     Mask c[N];

@@ -30,10 +30,16 @@
 //
 // One thread hashes one leaf or node: the permutation is a serial chain of
 // field products with no data shared between hashes, and 12 state words fit
-// in registers at full occupancy.  Bound: VALU issue (about 25k VALU per
-// permutation against 64 bytes absorbed).
+// in 128 registers, four waves per SIMD.  Bound: VALU issue (86% busy, at a
+// clock the load holds to 2.05 GHz): about 15.9k VALU instructions per
+// Poseidon permutation, 38% of them S-box products and 28% multiply-adds of
+// the partial rounds' dot products, and 13.0k per Poseidon2 permutation,
+// against 64 bytes absorbed.  With every word reduced to [0, p) in every step,
+// products one at a time and sparse partial rounds it was 24.8k and 16.4k;
+// 128 columns x 2^20 rows: 10.8 -> 8.9 ms a Poseidon tree, 2^18 leaves of
+// 2 x 93 values: 3.30 -> 2.32 ms a Poseidon2 tree.
 #include "../../include/boojum_ntt.h"
-#include "gl_field.hpp"
+#include "gl_lazy.hpp"
 
 #include <hip/hip_runtime.h>
 
@@ -65,14 +71,62 @@ struct PosTable {
 
 __device__ PosTable pos_table;
 
+// Constants of the one-lane-per-state permutations (permute, permute2).
+//
+// A constant factor b of a dot product is kept as three limbs, b = c0 +
+// c1 2^24 + c2 2^48 (c0, c1 < 2^24, c2 < 2^16), so that products with a
+// 32-bit half of a state word can be summed in 64 bits without carries.
+constexpr int LIMBS = 3;
+constexpr int BLOCK = 11, BLOCKS = PARTIAL / BLOCK;  // partial rounds are run in blocks of 11
+// 2^DOT_BIAS_LOG is added to the low accumulator of every dot product (see
+// Dot::value) and taken out of its constant.
+constexpr int DOT_BIAS_LOG = 54;
+
+struct DotConst {
+  uint32_t k[2];  // constant term, low and high half, less the bias
+};
+// Partial rounds in blocks.  With z_j the S-box output of round j of a block
+// and s_1..s_11 the other words at the block's start, the words at round r
+// are s_i + sum_{j<r} w_j,i z_j, so element 0 after round r is
+//   z_r + vs_r . s + sum_{j<r} (vs_r . w_j) z_j + constant,
+// and the words 1..11 are only formed at the block's end, with one reduction
+// per word instead of one per word and round.
+struct PosBlock {
+  struct {
+    DotConst k;
+    uint32_t s[PT - 1][LIMBS];
+    uint32_t z[BLOCK][LIMBS];  // j < r used
+  } round[BLOCK];
+  struct {
+    DotConst k;
+    uint32_t z[BLOCK][LIMBS];
+  } update[PT - 1];
+};
+struct PosFast {
+  uint64_t first[PT];        // constants of round 0
+  uint64_t after[7][PT][2];  // added behind each MDS, halves in 64 bits: rounds 1-3, then 27-29 and none
+  struct {
+    DotConst k;
+    uint32_t c[PT][LIMBS];
+  } dense[PT];
+  PosBlock block[BLOCKS];
+  // Poseidon2: behind the first external matrix and behind each full round's
+  // (the constants of the round that follows; element 0 alone before a
+  // partial round), and behind each internal matrix (element 0; all of the
+  // first closing full round's behind the last)
+  uint64_t p2_ext[1 + 2 * HALF_FULL][PT][2];
+  uint64_t p2_int[PARTIAL][2];
+  uint64_t p2_last[PT][2];
+};
+
+__device__ PosFast pos_fast;
+
 // The table, through an address the optimizer cannot see through: a kernel
 // that permutes in a loop then reloads the constants it needs in each pass
 // (scalar-cache hits) instead of hoisting them all into more SGPRs than a
-// wave has, which spilled 490 of them to VGPR lanes in the Poseidon leaf
-// kernel (5% faster leaves without; Poseidon2, with fewer constants, keeps
-// the direct table, 1% faster that way).
-__device__ __forceinline__ const PosTable &table() {
-  const PosTable *p = &pos_table;
+// wave has, which spilled them to VGPR lanes.
+__device__ __forceinline__ const PosFast &table() {
+  const PosFast *p = &pos_fast;
   asm volatile("" : "+s"(p));
   return *p;
 }
@@ -84,71 +138,193 @@ __device__ __forceinline__ uint64_t sbox(uint64_t x) {
   return gl::mul(x3, x4);
 }
 
-// y_r = sum_i 2^e_i x_((r + i) mod 12): the shifted words summed into 96
-// bits (12 terms below 2^80) and reduced once.
-__device__ __forceinline__ void mds(uint64_t (&s)[PT]) {
-  uint64_t y[PT];
+// x^7 of N words, any u64 in and out.
+template <int N> __device__ __forceinline__ void sbox_row(uint64_t *x) {
+  uint64_t x2[N], x3[N], x4[N];
+  gl::mul_row<N, gl::ANY>(x2, x, x);
+  gl::mul_row<N, gl::ANY>(x3, x2, x);
+  gl::mul_row<N, gl::ANY>(x4, x2, x2);
+  gl::mul_row<N, gl::ANY>(x, x3, x4);
+}
+__device__ __forceinline__ void sbox_all(uint64_t (&s)[PT]) {
+  sbox_row<4>(s);
+  sbox_row<4>(s + 4);
+  sbox_row<4>(s + 8);
+}
+
+// A power of two in an SGPR the optimizer does not know the value of, so that
+// a product with it stays one multiply-add into a 64-bit sum (a shift of a
+// widened word and an addition otherwise).
+__device__ __forceinline__ uint32_t opaque(uint32_t v) {
+  asm("" : "+s"(v));
+  return v;
+}
+
+// s[i] = lo[i] + hi[i] 2^32 for lo, hi < 2^62 (any u64): hi = h0 + h1 2^32
+// gives lo + h1 EPS + h0 2^32, one multiply-add, one addition into the high
+// word and its carry.
+template <int N> __device__ __forceinline__ void join_halves(uint64_t *s, const uint64_t *lo, const uint64_t *hi) {
+  uint32_t z1[N], h0[N], r[N], up[N];
+  uint64_t z[N];
+  gl::row::Mask drop[N];
+  gl::unroll<N>([&](auto k) {
+    constexpr int i = decltype(k)::value;
+    z[i] = (hi[i] >> 32) * gl::EPS + lo[i];
+    z1[i] = gl::hi32(z[i]);
+    h0[i] = gl::lo32(hi[i]);
+  });
+  gl::row::Rows<N>::add_bit(r, up, z1, h0);
+  gl::unroll<N>([&](auto k) {
+    constexpr int i = decltype(k)::value;
+    z[i] = gl::pair64(gl::lo32(z[i]), r[i]);
+  });
+  gl::row::Rows<N>::mad_eps(s, drop, up, z);
+}
+
+// MDS rows R0..R0+N-1: y_r = sum_i 2^e_i x_((r + i) mod 12) + k_r with the two
+// 32-bit halves of the words summed apart (12 terms below 2^48, one
+// multiply-add each): 24 multiply-adds and 4 instructions a row.
+template <int R0, int N>
+__device__ __forceinline__ void mds_rows(uint64_t *y, const uint64_t (&s)[PT], const uint64_t (*k)[2]) {
+  uint32_t c[PT];
 #pragma unroll
-  for (int r = 0; r < PT; ++r) {
-    uint64_t lo = 0;
-    uint32_t hi = 0;
+  for (int i = 0; i < PT; ++i) c[i] = opaque(1u << MDS_EXPS[i]);
+  gl::unroll<N / 4>([&](auto g) {
+    constexpr int G = 4 * decltype(g)::value;
+    uint64_t lo[4], hi[4];
 #pragma unroll
-    for (int i = 0; i < PT; ++i) {
-      const uint64_t v = s[(r + i) % PT];
-      const unsigned e = MDS_EXPS[i];
-      const uint64_t t = e ? v << e : v;
-      lo += t;
-      hi += (e ? (uint32_t)(v >> (64 - e)) : 0u) + (lo < t ? 1u : 0u);
+    for (int r = 0; r < 4; ++r) {
+      lo[r] = k[R0 + G + r][0];
+      hi[r] = k[R0 + G + r][1];
+#pragma unroll
+      for (int i = 0; i < PT; ++i) {
+        const uint64_t v = s[(R0 + G + r + i) % PT];
+        lo[r] += (uint64_t)gl::lo32(v) * c[i];
+        hi[r] += (uint64_t)gl::hi32(v) * c[i];
+      }
     }
-    y[r] = gl::reduce_limbs((uint32_t)lo, (uint32_t)(lo >> 32), hi, 0u);
+    join_halves<4>(y + G, lo, hi);
+  });
+}
+
+__device__ __forceinline__ void mds(uint64_t (&s)[PT], const uint64_t (*k)[2]) {
+  uint64_t y[PT];
+  mds_rows<0, PT>(y, s, k);
+#pragma unroll
+  for (int i = 0; i < PT; ++i) s[i] = y[i];
+}
+
+// A dot product of state words with table constants: six 64-bit sums, one
+// multiply-add per word half and limb.  At most 22 terms, so the sums stay
+// below 2^61 (limbs of 24 bits) and 2^53 (16 bits).
+struct Dot {
+  uint64_t p0, p1 = 0, p2 = 0, q0, q1 = 0, q2 = 0;
+  __device__ __forceinline__ explicit Dot(const DotConst &k)
+      : p0(gl::pair64(k.k[0], 1u << (DOT_BIAS_LOG - 32))), q0(k.k[1]) {}
+  __device__ __forceinline__ void mac(uint64_t a, const uint32_t *c) {
+    const uint64_t a0 = gl::lo32(a), a1 = gl::hi32(a);
+    p0 += a0 * c[0];
+    p1 += a0 * c[1];
+    p2 += a0 * c[2];
+    q0 += a1 * c[0];
+    q1 += a1 * c[1];
+    q2 += a1 * c[2];
   }
-#pragma unroll
-  for (int r = 0; r < PT; ++r) s[r] = y[r];
+  __device__ __forceinline__ void add(uint64_t a, uint32_t one) {  // one: opaque(1)
+    p0 += (uint64_t)gl::lo32(a) * one;
+    q0 += (uint64_t)gl::hi32(a) * one;
+  }
+  // p0 + p1 2^24 + p2 2^48 + (q0 + q1 2^24 + q2 2^48) 2^32, by weight:
+  // l + u 2^32 + v 2^64 + w 2^96 = (l - v - w) + (u + v) 2^32.  The bias in p0
+  // keeps l - v - w >= 0 (v < 2^53, w < 2^37).  lo < 2^62, hi < 2^62.
+  __device__ __forceinline__ void halves(uint64_t &lo, uint64_t &hi, uint32_t c24, uint32_t c16) const {
+    const uint64_t l = p0 + (uint64_t)gl::lo32(p1) * c24;
+    const uint64_t u = q0 + (uint64_t)gl::hi32(p1) * c24 + (uint64_t)gl::lo32(p2) * c16 + (uint64_t)gl::lo32(q1) * c24;
+    const uint64_t v = (uint64_t)gl::hi32(q1) * c24 + (uint64_t)gl::hi32(p2) * c16 + (uint64_t)gl::lo32(q2) * c16;
+    const uint64_t w = (uint64_t)gl::hi32(q2) * c16 + v;
+    lo = l - w;
+    hi = u + v;
+  }
+};
+
+// One dot product's value (any u64).
+__device__ __forceinline__ uint64_t dot_value(const Dot &d, uint32_t c24, uint32_t c16) {
+  uint64_t lo, hi, r;
+  d.halves(lo, hi, c24, c16);
+  join_halves<1>(&r, &lo, &hi);
+  return r;
 }
 
-__device__ __forceinline__ void full_round(uint64_t (&s)[PT], const uint64_t *rc) {
+// The permutation on any u64 words, giving any u64 words.  Only the four words
+// read next are formed by the last MDS: the capacity (capacity_out; a sponge
+// overwrites the rate), else words 0..3, the digest.
+__device__ __forceinline__ void permute(uint64_t (&s)[PT], bool capacity_out) {
+  const PosFast &t = table();
 #pragma unroll
-  for (int i = 0; i < PT; ++i) s[i] = sbox(rc ? gl::add(s[i], rc[i]) : s[i]);
-}
-
-__device__ __forceinline__ void permute(uint64_t (&s)[PT]) {
-  const PosTable &t = table();
+  for (int i = 0; i < PT; ++i) {
+    // s + constant: the constant is below p, so one carry is all there can be
+    const uint64_t v = s[i] + t.first[i];
+    s[i] = v + (v < s[i] ? gl::EPS : 0ull);
+  }
 #pragma unroll 1
   for (int r = 0; r < HALF_FULL - 1; ++r) {
-    full_round(s, t.rc_full[r]);
-    mds(s);
+    sbox_all(s);
+    mds(s, t.after[r]);
   }
-  full_round(s, t.rc_full[HALF_FULL - 1]);
+  sbox_all(s);
+  const uint32_t c24 = opaque(1u << 24), c16 = opaque(1u << 16), one = opaque(1u);
   {
     uint64_t v[PT];
 #pragma unroll
-    for (int i = 0; i < PT; ++i) v[i] = gl::add(s[i], t.rcf[i]);
+    for (int i = 0; i < PT; ++i) v[i] = s[i];
 #pragma unroll
     for (int r = 0; r < PT; ++r) {
-      gl::Acc acc;
+      Dot d(t.dense[r].k);
 #pragma unroll
-      for (int c = 0; c < PT; ++c) gl::mac(acc, v[c], t.dense[r][c]);
-      s[r] = gl::acc_reduce(acc);
+      for (int c = 0; c < PT; ++c) d.mac(v[c], t.dense[r].c[c]);
+      s[r] = dot_value(d, c24, c16);
     }
   }
 #pragma unroll 1
-  for (int k = 0; k < PARTIAL; ++k) {
-    const uint64_t s0 = gl::add(sbox(s[0]), t.sbox_c[k]);
-    gl::Acc acc;
-    acc.l0 = (uint32_t)s0;
-    acc.l1 = (uint32_t)(s0 >> 32);
+  for (int b = 0; b < BLOCKS; ++b) {
+    const PosBlock &blk = t.block[b];
+    uint64_t z[BLOCK];
 #pragma unroll
-    for (int i = 1; i < PT; ++i) gl::mac(acc, s[i], t.vs[k][i - 1]);
+    for (int r = 0; r < BLOCK; ++r) {
+      z[r] = s[0];
+      sbox_row<1>(z + r);
+      Dot d(blk.round[r].k);
 #pragma unroll
-    for (int i = 1; i < PT; ++i) s[i] = gl::add(gl::mul(s0, t.w_hats[k][i - 1]), s[i]);
-    s[0] = gl::acc_reduce(acc);
+      for (int i = 1; i < PT; ++i) d.mac(s[i], blk.round[r].s[i - 1]);
+#pragma unroll
+      for (int j = 0; j < r; ++j) d.mac(z[j], blk.round[r].z[j]);
+      d.add(z[r], one);
+      s[0] = dot_value(d, c24, c16);
+    }
+#pragma unroll
+    for (int i = 1; i < PT; ++i) {
+      Dot d(blk.update[i - 1].k);
+#pragma unroll
+      for (int j = 0; j < BLOCK; ++j) d.mac(z[j], blk.update[i - 1].z[j]);
+      d.add(s[i], one);
+      s[i] = dot_value(d, c24, c16);
+    }
   }
-  full_round(s, nullptr);
-  mds(s);
 #pragma unroll 1
   for (int r = 0; r < 3; ++r) {
-    full_round(s, t.rc_full[HALF_FULL + r]);
-    mds(s);
+    sbox_all(s);
+    mds(s, t.after[3 + r]);
+  }
+  sbox_all(s);
+  uint64_t y[CAP];
+  if (capacity_out) {
+    mds_rows<RATE, CAP>(y, s, t.after[6]);
+#pragma unroll
+    for (int i = 0; i < CAP; ++i) s[RATE + i] = y[i];
+  } else {
+    mds_rows<0, CAP>(y, s, t.after[6]);
+#pragma unroll
+    for (int i = 0; i < CAP; ++i) s[i] = y[i];
   }
 }
 
@@ -157,83 +333,103 @@ __device__ __forceinline__ void permute(uint64_t (&s)[PT]) {
 // M4, M4) over the three 4-tiles, internal matrix M_I = J + diag(2^mu_i).
 constexpr unsigned P2_MU[PT] = {4, 14, 11, 8, 0, 5, 2, 9, 13, 6, 3, 12};
 
-// M4 = [[5,7,1,3],[4,6,1,1],[1,3,5,7],[1,1,4,6]] on one tile, by the
-// addition chain of eprint 2023/323 Appendix B (8 additions, 4 doublings).
+// M4 = [[5,7,1,3],[4,6,1,1],[1,3,5,7],[1,1,4,6]] on one tile of 64-bit sums, by
+// the addition chain of eprint 2023/323 Appendix B (8 shifted additions).
 __device__ __forceinline__ void m4_tile(uint64_t *x) {
-  const uint64_t t0 = gl::add(x[0], x[1]);
-  const uint64_t t1 = gl::add(x[2], x[3]);
-  const uint64_t t2 = gl::add(gl::add(x[1], x[1]), t1);
-  const uint64_t t3 = gl::add(gl::add(x[3], x[3]), t0);
-  const uint64_t t1x2 = gl::add(t1, t1), t0x2 = gl::add(t0, t0);
-  const uint64_t t4 = gl::add(gl::add(t1x2, t1x2), t3);
-  const uint64_t t5 = gl::add(gl::add(t0x2, t0x2), t2);
-  x[0] = gl::add(t3, t5);
+  const uint64_t t0 = x[0] + x[1];
+  const uint64_t t1 = x[2] + x[3];
+  const uint64_t t2 = (x[1] << 1) + t1;
+  const uint64_t t3 = (x[3] << 1) + t0;
+  const uint64_t t4 = (t1 << 2) + t3;
+  const uint64_t t5 = (t0 << 2) + t2;
+  x[0] = t3 + t5;
   x[1] = t5;
-  x[2] = gl::add(t2, t4);
+  x[2] = t2 + t4;
   x[3] = t4;
 }
 
-__device__ __forceinline__ void m_ext(uint64_t (&s)[PT]) {
-  m4_tile(s);
-  m4_tile(s + 4);
-  m4_tile(s + 8);
+// The external matrix plus constants: the two 32-bit halves of the words go
+// through the additions apart (below 2^39) and each word is reduced once.
+__device__ __forceinline__ void m_ext(uint64_t (&s)[PT], const uint64_t (*k)[2]) {
+  uint64_t h[2][PT];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const uint64_t sum = gl::add(gl::add(s[j], s[4 + j]), s[8 + j]);
-    s[j] = gl::add(s[j], sum);
-    s[4 + j] = gl::add(s[4 + j], sum);
-    s[8 + j] = gl::add(s[8 + j], sum);
+  for (int w = 0; w < 2; ++w) {
+#pragma unroll
+    for (int i = 0; i < PT; ++i) h[w][i] = w ? gl::hi32(s[i]) : gl::lo32(s[i]);
+#pragma unroll
+    for (int g = 0; g < PT; g += 4) m4_tile(h[w] + g);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const uint64_t sum = h[w][j] + h[w][4 + j] + h[w][8 + j];
+#pragma unroll
+      for (int g = 0; g < PT; g += 4) h[w][g + j] += sum + k[g + j][w];
+    }
   }
+  gl::unroll<3>([&](auto g) {
+    constexpr int G = 4 * decltype(g)::value;
+    join_halves<4>(s + G, h[0] + G, h[1] + G);
+  });
 }
 
-// y_i = sum + 2^mu_i x_i: the shifted word and the sum added in 96 bits,
-// one reduction.
-__device__ __forceinline__ void m_int(uint64_t (&s)[PT]) {
-  uint64_t sum = s[0];
+// y_i = sum + 2^mu_i x_i, the halves apart, plus k0 on element 0 (and all of
+// `last`, if given).
+__device__ __forceinline__ void m_int(uint64_t (&s)[PT], const uint64_t *k0, const uint64_t (*last)[2]) {
+  const uint32_t one = opaque(1u);
+  uint64_t h[2][PT];
 #pragma unroll
-  for (int i = 1; i < PT; ++i) sum = gl::add(sum, s[i]);
+  for (int w = 0; w < 2; ++w) {
+    uint64_t sum = w ? gl::hi32(s[0]) : gl::lo32(s[0]);
 #pragma unroll
-  for (int i = 0; i < PT; ++i) {
-    const unsigned e = P2_MU[i];
-    uint64_t lo = e ? s[i] << e : s[i];
-    uint32_t hi = e ? (uint32_t)(s[i] >> (64 - e)) : 0u;
-    lo += sum;
-    hi += lo < sum ? 1u : 0u;
-    s[i] = gl::reduce_limbs((uint32_t)lo, (uint32_t)(lo >> 32), hi, 0u);
+    for (int i = 1; i < PT; ++i) sum += (uint64_t)(w ? gl::hi32(s[i]) : gl::lo32(s[i])) * one;
+#pragma unroll
+    for (int i = 0; i < PT; ++i)
+      h[w][i] = sum + (uint64_t)(w ? gl::hi32(s[i]) : gl::lo32(s[i])) * opaque(1u << P2_MU[i]);
+    if (last) {
+#pragma unroll
+      for (int i = 0; i < PT; ++i) h[w][i] += last[i][w];
+    } else {
+      h[w][0] += k0[w];
+    }
   }
+  gl::unroll<3>([&](auto g) {
+    constexpr int G = 4 * decltype(g)::value;
+    join_halves<4>(s + G, h[0] + G, h[1] + G);
+  });
 }
 
-__device__ __forceinline__ void permute2(uint64_t (&s)[PT]) {
-  const PosTable &t = pos_table;  // its few constants hoist without spills
-  m_ext(s);
+__device__ __forceinline__ void permute2(uint64_t (&s)[PT], bool) {
+  const PosFast &t = table();
+  m_ext(s, t.p2_ext[0]);
 #pragma unroll 1
   for (int r = 0; r < HALF_FULL; ++r) {
-    full_round(s, t.p2_full[r]);
-    m_ext(s);
+    sbox_all(s);
+    m_ext(s, t.p2_ext[1 + r]);
   }
 #pragma unroll 1
-  for (int k = 0; k < PARTIAL; ++k) {
-    s[0] = sbox(gl::add(s[0], t.p2_partial[k]));
-    m_int(s);
+  for (int k = 0; k < PARTIAL - 1; ++k) {
+    sbox_row<1>(s);
+    m_int(s, t.p2_int[k], nullptr);
   }
+  sbox_row<1>(s);
+  m_int(s, nullptr, t.p2_last);
 #pragma unroll 1
   for (int r = 0; r < HALF_FULL; ++r) {
-    full_round(s, t.p2_full[HALF_FULL + r]);
-    m_ext(s);
+    sbox_all(s);
+    m_ext(s, t.p2_ext[1 + HALF_FULL + r]);
   }
 }
 
 // Hash selector of the kernels: 0 Poseidon, 1 Poseidon2.
-template <int H> __device__ __forceinline__ void permute_h(uint64_t (&s)[PT]) {
-  if constexpr (H == 0) permute(s);
-  else permute2(s);
+template <int H> __device__ __forceinline__ void permute_h(uint64_t (&s)[PT], bool capacity_out) {
+  if constexpr (H == 0) permute(s, capacity_out);
+  else permute2(s, capacity_out);
 }
 
 // native/poseidon_utils.cuh:8-42: leaf g absorbs the values (row r, column c)
 // at values[g rows + r + c rows count] in the order c rows + r, 8 at a time
 // into state[0..8] (the last chunk zero-padded), permuting after each chunk.
 template <int H>
-__global__ __launch_bounds__(256) void poseidon_leaves_kernel(const uint64_t *__restrict__ values,
+__global__ __launch_bounds__(256, 4) void poseidon_leaves_kernel(const uint64_t *__restrict__ values,
                                                               uint64_t *__restrict__ results, uint32_t rows,
                                                               uint32_t cols, uint32_t count, bool load_intermediate,
                                                               bool store_intermediate) {
@@ -244,7 +440,7 @@ __global__ __launch_bounds__(256) void poseidon_leaves_kernel(const uint64_t *__
   for (int i = 0; i < PT; ++i) s[i] = 0;
   if (load_intermediate) {
 #pragma unroll
-    for (int i = 0; i < CAP; ++i) s[RATE + i] = gl::canon(results[g + (uint64_t)i * count]);
+    for (int i = 0; i < CAP; ++i) s[RATE + i] = results[g + (uint64_t)i * count];
   }
   const uint64_t col_stride = (uint64_t)rows * count;
   const uint64_t *base = values + (uint64_t)g * rows;
@@ -253,16 +449,18 @@ __global__ __launch_bounds__(256) void poseidon_leaves_kernel(const uint64_t *__
   for (uint64_t off = 0; off < total; off += RATE) {
 #pragma unroll
     for (int i = 0; i < RATE; ++i) {
-      s[i] = c < cols ? gl::canon(base[r + c * col_stride]) : 0ull;
+      s[i] = c < cols ? base[r + c * col_stride] : 0ull;
       if (++r == rows) {
         r = 0;
         ++c;
       }
     }
-    permute_h<H>(s);
+    // the next chunk overwrites the rate, so only the capacity is read on
+    permute_h<H>(s, store_intermediate || off + RATE < total);
   }
 #pragma unroll
-  for (int i = 0; i < CAP; ++i) results[g + (uint64_t)i * count] = store_intermediate ? s[RATE + i] : s[i];
+  for (int i = 0; i < CAP; ++i)
+    results[g + (uint64_t)i * count] = gl::canon(store_intermediate ? s[RATE + i] : s[i]);
 }
 
 // native/poseidon_utils.cuh:44-61: node g hashes children 2g, 2g + 1 of the
@@ -277,13 +475,13 @@ __global__ __launch_bounds__(256) void poseidon_nodes_kernel(const uint64_t *__r
 #pragma unroll
   for (int i = 0; i < CAP; ++i) {
     const uint64_t *pair = values + 2 * ((uint64_t)g + (uint64_t)i * count);
-    s[i] = gl::canon(pair[0]);
-    s[CAP + i] = gl::canon(pair[1]);
+    s[i] = pair[0];
+    s[CAP + i] = pair[1];
     s[RATE + i] = 0;
   }
-  permute_h<H>(s);
+  permute_h<H>(s, false);
 #pragma unroll
-  for (int i = 0; i < CAP; ++i) results[g + (uint64_t)i * count] = s[i];
+  for (int i = 0; i < CAP; ++i) results[g + (uint64_t)i * count] = gl::canon(s[i]);
 }
 
 // ---- cooperative node hashing: one state over 16 lanes ------------------------
@@ -594,6 +792,71 @@ bool derive(const uint64_t *rc_in, PosTable &t) {
   return true;
 }
 
+// c in limbs of 24, 24 and 16 bits.
+void set_limbs(uint32_t *out, uint64_t c) {
+  out[0] = (uint32_t)(c & 0xFFFFFF);
+  out[1] = (uint32_t)((c >> 24) & 0xFFFFFF);
+  out[2] = (uint32_t)(c >> 48);
+}
+void set_const(DotConst &out, uint64_t c) {
+  const uint64_t v = gl::sub(c, 1ull << DOT_BIAS_LOG);
+  out.k[0] = (uint32_t)v;
+  out.k[1] = (uint32_t)(v >> 32);
+}
+void set_halves(uint64_t (*out)[2], const uint64_t *c, int n = PT) {
+  for (int i = 0; i < n; ++i) {
+    out[i][0] = (uint32_t)c[i];
+    out[i][1] = c[i] >> 32;
+  }
+}
+
+// The one-lane forms' table from the fused one.
+void derive_fast(const PosTable &t, PosFast &f) {
+  for (int i = 0; i < PT; ++i) f.first[i] = t.rc_full[0][i];
+  for (int r = 0; r < 3; ++r) {
+    set_halves(f.after[r], t.rc_full[1 + r]);
+    set_halves(f.after[3 + r], t.rc_full[HALF_FULL + r]);
+  }
+  // dense (v + rcf): the fused constant layer becomes each row's constant
+  for (int r = 0; r < PT; ++r) {
+    uint64_t k = 0;
+    for (int c = 0; c < PT; ++c) {
+      set_limbs(f.dense[r].c[c], t.dense[r][c]);
+      k = gl::add(k, gl::mul(t.dense[r][c], t.rcf[c]));
+    }
+    set_const(f.dense[r].k, k);
+  }
+  // z_j below is the S-box output without its constant sbox_c
+  for (int b = 0; b < BLOCKS; ++b) {
+    PosBlock &blk = f.block[b];
+    const int k0 = b * BLOCK;
+    for (int r = 0; r < BLOCK; ++r) {
+      uint64_t k = t.sbox_c[k0 + r];
+      for (int i = 0; i < PT - 1; ++i) set_limbs(blk.round[r].s[i], t.vs[k0 + r][i]);
+      for (int j = 0; j < r; ++j) {
+        uint64_t c = 0;
+        for (int i = 0; i < PT - 1; ++i) c = gl::add(c, gl::mul(t.vs[k0 + r][i], t.w_hats[k0 + j][i]));
+        set_limbs(blk.round[r].z[j], c);
+        k = gl::add(k, gl::mul(c, t.sbox_c[k0 + j]));
+      }
+      set_const(blk.round[r].k, k);
+    }
+    for (int i = 0; i < PT - 1; ++i) {
+      uint64_t k = 0;
+      for (int j = 0; j < BLOCK; ++j) {
+        set_limbs(blk.update[i].z[j], t.w_hats[k0 + j][i]);
+        k = gl::add(k, gl::mul(t.w_hats[k0 + j][i], t.sbox_c[k0 + j]));
+      }
+      set_const(blk.update[i].k, k);
+    }
+  }
+  for (int r = 0; r < HALF_FULL; ++r) set_halves(f.p2_ext[r], t.p2_full[r]);
+  set_halves(f.p2_ext[HALF_FULL], t.p2_partial, 1);
+  for (int k = 0; k + 1 < PARTIAL; ++k) set_halves(&f.p2_int[k], t.p2_partial + k + 1, 1);
+  set_halves(f.p2_last, t.p2_full[HALF_FULL]);
+  for (int r = 1; r < HALF_FULL; ++r) set_halves(f.p2_ext[HALF_FULL + r], t.p2_full[HALF_FULL + r]);
+}
+
 constexpr int MAX_DEVICES = 64;
 // Every hashing entry point holds this lock shared from its readiness check
 // through its launches; replacing the table holds it exclusively.  So no
@@ -737,6 +1000,8 @@ extern "C" int bc_poseidon_set_round_constants(const uint64_t *round_constants) 
   if (dev < 0 || dev >= MAX_DEVICES) return BC_ERROR_INVALID_VALUE;
   PosTable t{};
   if (!derive(round_constants, t)) return BC_ERROR_INVALID_VALUE;
+  PosFast f{};
+  derive_fast(t, f);
   std::unique_lock<std::shared_mutex> lk(pos_mu);
   // hashing kernels already queued on any stream of this device read the
   // table: let them finish before it changes (no new ones can be queued
@@ -744,6 +1009,8 @@ extern "C" int bc_poseidon_set_round_constants(const uint64_t *round_constants) 
   err = hipDeviceSynchronize();
   if (err != hipSuccess) return err;
   err = hipMemcpyToSymbol(HIP_SYMBOL(pos_table), &t, sizeof t, 0, hipMemcpyHostToDevice);
+  if (err != hipSuccess) return err;
+  err = hipMemcpyToSymbol(HIP_SYMBOL(pos_fast), &f, sizeof f, 0, hipMemcpyHostToDevice);
   if (err != hipSuccess) return err;
   err = hipDeviceSynchronize();
   if (err != hipSuccess) return err;
