@@ -33,7 +33,7 @@
 // in 128 registers, four waves per SIMD.  Bound: VALU issue (86% busy, at a
 // clock the load holds to 2.05 GHz): about 15.9k VALU instructions per
 // Poseidon permutation, 38% of them S-box products and 28% multiply-adds of
-// the partial rounds' dot products, and 13.0k per Poseidon2 permutation,
+// the partial rounds' dot products, and 11.9k per Poseidon2 permutation,
 // against 64 bytes absorbed.  With every word reduced to [0, p) in every step,
 // products one at a time and sparse partial rounds it was 24.8k and 16.4k;
 // 128 columns x 2^20 rows: 10.8 -> 8.9 ms a Poseidon tree, 2^18 leaves of
@@ -484,174 +484,310 @@ __global__ __launch_bounds__(256) void poseidon_nodes_kernel(const uint64_t *__r
   for (int i = 0; i < CAP; ++i) results[g + (uint64_t)i * count] = gl::canon(s[i]);
 }
 
-// ---- cooperative node hashing: one state over 16 lanes ------------------------
-// A small layer is one dependent permutation chain per lane, about 28k
-// instructions: ~91 us however few nodes the layer has.  Here lane j of a
-// 16-lane group owns state element j (lanes 12-15 compute values nobody
-// reads), so each lane runs one S-box and one matrix row per round; matrix
-// rows gather the other elements with __shfl inside the group, and the
-// constants are staged in LDS.  Used for layers of at most COOP_MAX_NODES
-// nodes (the reference likewise switches to cooperative kernels for small
-// layers at the same size, src/poseidon.rs:71,279-283).
+// ---- cooperative hashing: one state over 16 lanes ------------------------------
+// A small layer is one dependent permutation chain per lane, whatever its
+// size: 12-16k instructions at one per 8 cycles, the rate of a wave alone on
+// its SIMD.  Here lane j of a 16-lane row owns state element j (lanes 12-15
+// hold values nobody reads), so a lane runs one S-box and one matrix row per
+// round.  Sums over the row are taken on 22-bit limbs with row rotations
+// (plain 32-bit additions, 12 instructions for the 16 lanes); the MDS row and
+// the 4-tiles gather their words through the wave's LDS, a round's constants
+// come from LDS.  Used for layers and leaf sets of at most COOP_MAX_NODES
+// (the reference likewise switches to cooperative kernels for small layers at
+// the same size, src/poseidon.rs:71,279-283).
 constexpr uint32_t COOP_LANES = 16, COOP_MAX_NODES = 1u << 14;
+constexpr uint32_t COOP_NT = 512, COOP_GROUPS = COOP_NT / COOP_LANES;  // two waves per SIMD issue side by side
 
-__device__ __forceinline__ uint64_t grp(uint64_t v, uint32_t lane) { return __shfl(v, (int)lane, (int)COOP_LANES); }
+// A row's words in LDS, twice in a row so that word (j + i) mod 12 is at j + i.
+struct CoopLds {
+  PosTable t;
+  uint64_t words[COOP_GROUPS][2 * PT];
+};
 
-// sum over the 16 lanes of the group (lanes 12-15 must contribute 0)
-__device__ __forceinline__ uint64_t grp_sum(uint64_t v) {
-#pragma unroll
-  for (uint32_t m = 8; m >= 1; m >>= 1) v = gl::add(v, __shfl_xor(v, (int)m, (int)COOP_LANES));
-  return v;
+// The wave's LDS accesses run in program order; this keeps the compiler from
+// moving them across.
+__device__ __forceinline__ void coop_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-__device__ __forceinline__ uint64_t coop_mds_row(uint64_t x, uint32_t j) {
-  uint64_t lo = 0;
-  uint32_t hi = 0;
-#pragma unroll
-  for (int i = 0; i < PT; ++i) {
-    const uint64_t v = grp(x, (j + (uint32_t)i) % PT);
-    const unsigned e = MDS_EXPS[i];
-    const uint64_t t = e ? v << e : v;
-    lo += t;
-    hi += (e ? (uint32_t)(v >> (64 - e)) : 0u) + (lo < t ? 1u : 0u);
+template <int CTRL> __device__ __forceinline__ uint32_t dpp(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xF, 0xF, true);
+}
+constexpr int ROW_ROR = 0x120, ROW_NEWBCAST = 0x150;  // rotate by n inside a row of 16; lane n to the whole row
+
+// Element 0's value to every lane of the row.
+__device__ __forceinline__ uint64_t row_first(uint64_t v) {
+  return gl::pair64(dpp<ROW_NEWBCAST>(gl::lo32(v)), dpp<ROW_NEWBCAST>(gl::hi32(v)));
+}
+
+// v in limbs of 22, 22 and 20 bits; keep is the 22-bit mask, 0 in lanes whose
+// value must not count.
+struct Limbs {
+  uint32_t a, b, c;
+  __device__ __forceinline__ Limbs(uint64_t v, uint32_t keep)
+      : a(gl::lo32(v) & keep), b(gl::align32(gl::hi32(v), gl::lo32(v), 22) & keep), c((gl::hi32(v) >> 12) & keep) {}
+  template <int N> __device__ __forceinline__ void add_ror() {
+    a += dpp<ROW_ROR + N>(a);
+    b += dpp<ROW_ROR + N>(b);
+    c += dpp<ROW_ROR + N>(c);
   }
-  return gl::reduce_limbs((uint32_t)lo, (uint32_t)(lo >> 32), hi, 0u);
+  // lo + hi 2^32 += a + b 2^22 + c 2^44 (limbs below 2^32)
+  __device__ __forceinline__ void add_to(uint64_t &lo, uint64_t &hi) const {
+    lo += (uint64_t)b * opaque(1u << 22) + a;
+    hi += (uint64_t)c * opaque(1u << 12);
+  }
+};
+
+// x^7, the cube and the fourth power side by side; xv = x v beside the square.
+__device__ __forceinline__ uint64_t coop_sbox(uint64_t x, uint64_t v, uint64_t &xv) {
+  uint64_t a[2] = {x, x}, b[2] = {x, v}, s[2], c[2], r;
+  gl::mul_row<2, gl::ANY>(s, a, b);
+  xv = s[1];
+  a[0] = a[1] = s[0];
+  b[0] = x;
+  b[1] = s[0];
+  gl::mul_row<2, gl::ANY>(c, a, b);
+  gl::mul_row<1, gl::ANY>(&r, &c[0], &c[1]);
+  return r;
+}
+__device__ __forceinline__ uint64_t coop_sbox(uint64_t x) {
+  uint64_t s, a[2], b[2], c[2], r;
+  gl::mul_row<1, gl::ANY>(&s, &x, &x);
+  a[0] = a[1] = s;
+  b[0] = x;
+  b[1] = s;
+  gl::mul_row<2, gl::ANY>(c, a, b);
+  gl::mul_row<1, gl::ANY>(&r, &c[0], &c[1]);
+  return r;
 }
 
-__device__ __forceinline__ void coop_permute(uint64_t &x, uint32_t j, const PosTable &t) {
-  const uint32_t jj = j < PT ? j : PT - 1;  // table row of this lane (lanes 12-15 reuse row 11)
-  const uint32_t jm = jj ? jj - 1 : 0;      // index into the 11-entry sparse vectors
-#pragma unroll 1
-  for (int r = 0; r < HALF_FULL - 1; ++r) x = coop_mds_row(sbox(gl::add(x, t.rc_full[r][jj])), j);
-  {
-    const uint64_t v = gl::add(sbox(gl::add(x, t.rc_full[HALF_FULL - 1][jj])), t.rcf[jj]);
-    gl::Acc acc;
+// lo + hi 2^32 (both below 2^62), any u64.
+__device__ __forceinline__ uint64_t coop_join(uint64_t lo, uint64_t hi) {
+  uint64_t r;
+  join_halves<1>(&r, &lo, &hi);
+  return r;
+}
+
+// a + b for b below p, any u64.
+__device__ __forceinline__ uint64_t add_const(uint64_t a, uint64_t b) {
+  const uint64_t v = a + b;
+  return v + (v < a ? gl::EPS : 0ull);
+}
+
+// One lane's view of the cooperative permutations: element j of the state
+// whose words are staged in w.
+struct Coop {
+  const PosTable &t;
+  uint64_t *w;      // the row's 2 PT words in LDS
+  uint32_t j, jj;   // lane of the row; table row (lanes 12-15 reuse row 11)
+  uint32_t keep;    // 22-bit mask, 0 in lanes 12-15
+  __device__ __forceinline__ Coop(CoopLds &l, uint32_t lane, uint32_t group)
+      : t(l.t), w(l.words[group]), j(lane), jj(lane < PT ? lane : PT - 1), keep(lane < PT ? 0x3FFFFFu : 0u) {}
+
+  __device__ __forceinline__ void stage(uint64_t x) const {
+    coop_sync();  // the row's earlier reads come first
+    if (j < PT) w[j] = w[j + PT] = x;
+    coop_sync();
+  }
+
+  __device__ __forceinline__ uint64_t mds_row(uint64_t x) const {
+    stage(x);
+    uint64_t lo = 0, hi = 0;
 #pragma unroll
-    for (int c = 0; c < PT; ++c) gl::mac(acc, grp(v, (uint32_t)c), t.dense[jj][c]);
-    x = gl::acc_reduce(acc);
+    for (int i = 0; i < PT; ++i) {
+      const uint64_t v = w[jj + i];
+      const uint32_t c = opaque(1u << MDS_EXPS[i]);
+      lo += (uint64_t)gl::lo32(v) * c;
+      hi += (uint64_t)gl::hi32(v) * c;
+    }
+    return coop_join(lo, hi);
   }
-#pragma unroll 1
-  for (int k = 0; k < PARTIAL; ++k) {
-    const uint64_t s0 = grp(gl::add(sbox(x), t.sbox_c[k]), 0);
-    const uint64_t term = j == 0 ? s0 : (j < PT ? gl::mul(x, t.vs[k][jm]) : 0ull);
-    const uint64_t y0 = grp_sum(term);
-    x = j == 0 ? y0 : gl::add(gl::mul(s0, t.w_hats[k][jm]), x);
-  }
-  x = coop_mds_row(sbox(x), j);
-#pragma unroll 1
-  for (int r = 0; r < 3; ++r) x = coop_mds_row(sbox(gl::add(x, t.rc_full[HALF_FULL + r][jj])), j);
-}
 
-// sum_c m_c v_c for small m_c (M4 entries, at most 7): 67-bit products
-// summed in 96 bits, one reduction
-__device__ __forceinline__ uint64_t small_dot4(const uint64_t *v, const uint32_t *m) {
-  uint64_t lo = 0;
-  uint32_t hi = 0;
+  __device__ __forceinline__ void permute(uint64_t &x) const {
+    const uint32_t jm = jj ? jj - 1 : 0;  // index into the 11-entry sparse vectors
+#pragma unroll 1
+    for (int r = 0; r < HALF_FULL - 1; ++r) x = mds_row(coop_sbox(add_const(x, t.rc_full[r][jj])));
+    {
+      stage(add_const(coop_sbox(add_const(x, t.rc_full[HALF_FULL - 1][jj])), t.rcf[jj]));
+      gl::Acc acc;
 #pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    const uint64_t p = v[c] * m[c];
-    const uint32_t ph = (uint32_t)__umul64hi(v[c], (uint64_t)m[c]);
-    lo += p;
-    hi += ph + (lo < p ? 1u : 0u);
+      for (int c = 0; c < PT; ++c) gl::mac(acc, w[c], t.dense[jj][c]);
+      x = gl::acc_reduce(acc);
+    }
+#pragma unroll 1
+    for (int k = 0; k < PARTIAL; ++k) {
+      // element 0 becomes z + sum_i vs_i x_i, element i becomes x_i + w_i z
+      uint64_t term;
+      const uint64_t s = coop_sbox(x, t.vs[k][jm], term);
+      const uint64_t z = row_first(add_const(s, t.sbox_c[k]));
+      Limbs l(term, j ? keep : 0u);
+      l.add_ror<8>();
+      l.add_ror<4>();
+      l.add_ror<2>();
+      l.add_ror<1>();
+      uint64_t wz;
+      const uint64_t wk = t.w_hats[k][jm];
+      gl::mul_row<1, gl::ANY>(&wz, &z, &wk);
+      // the words' halves, then z or x + w z on top
+      const uint64_t add = j ? wz : z;
+      uint64_t lo = gl::lo32(add), hi = gl::hi32(add);
+      if (j) {
+        lo += gl::lo32(x);
+        hi += gl::hi32(x);
+      } else {
+        l.add_to(lo, hi);
+      }
+      x = coop_join(lo, hi);
+    }
+    x = mds_row(coop_sbox(x));
+#pragma unroll 1
+    for (int r = 0; r < 3; ++r) x = mds_row(coop_sbox(add_const(x, t.rc_full[HALF_FULL + r][jj])));
   }
-  return gl::reduce_limbs((uint32_t)lo, (uint32_t)(lo >> 32), hi, 0u);
-}
 
-__device__ __forceinline__ uint64_t coop_m_ext(uint64_t x, uint32_t j, const uint32_t *m4row) {
-  const uint32_t tile = j & ~3u, q = j & 3u;
-  uint64_t v[4];
+  // (J + I) (x) M4 on the three tiles: each word plus the sum over the tiles,
+  // then the 4 x 4 row, on limbs.
+  __device__ __forceinline__ uint64_t m_ext_row(uint64_t x, const uint32_t *m4row) const {
+    Limbs l(x, keep), s = l;
+    s.add_ror<8>();
+    s.add_ror<4>();
+    l.a += s.a;
+    l.b += s.b;
+    l.c += s.c;
+    auto row = [&](uint32_t v) {  // limbs below 2^25, the row sums to at most 16
+      return m4row[0] * dpp<0x00>(v) + m4row[1] * dpp<0x55>(v) + m4row[2] * dpp<0xAA>(v) + m4row[3] * dpp<0xFF>(v);
+    };
+    l.a = row(l.a);
+    l.b = row(l.b);
+    l.c = row(l.c);
+    uint64_t lo = 0, hi = 0;
+    l.add_to(lo, hi);
+    return coop_join(lo, hi);
+  }
+
+  __device__ __forceinline__ void permute2(uint64_t &x) const {
+    constexpr uint32_t M4[4][4] = {{5, 7, 1, 3}, {4, 6, 1, 1}, {1, 3, 5, 7}, {1, 1, 4, 6}};
+    uint32_t m4row[4];
 #pragma unroll
-  for (int c = 0; c < 4; ++c) v[c] = grp(x, tile + (uint32_t)c);
-  const uint64_t y = small_dot4(v, m4row);
-  const uint64_t tot = gl::add(gl::add(grp(y, q), grp(y, 4 + q)), grp(y, 8 + q));
-  return gl::add(y, tot);
-}
-
-__device__ __forceinline__ uint64_t coop_m_int(uint64_t x, uint32_t j) {
-  const uint64_t sum = grp_sum(j < PT ? x : 0ull);
-  const unsigned e = P2_MU[j < PT ? j : 0];
-  uint64_t lo = e ? x << e : x;
-  uint32_t hi = e ? (uint32_t)(x >> (64 - e)) : 0u;
-  lo += sum;
-  hi += lo < sum ? 1u : 0u;
-  return gl::reduce_limbs((uint32_t)lo, (uint32_t)(lo >> 32), hi, 0u);
-}
-
-__device__ __forceinline__ void coop_permute2(uint64_t &x, uint32_t j, const PosTable &t) {
-  constexpr uint32_t M4[4][4] = {{5, 7, 1, 3}, {4, 6, 1, 1}, {1, 3, 5, 7}, {1, 1, 4, 6}};
-  uint32_t m4row[4];
+    for (int c = 0; c < 4; ++c) {
+      const uint32_t q = j & 3u;
+      m4row[c] = q == 0 ? M4[0][c] : (q == 1 ? M4[1][c] : (q == 2 ? M4[2][c] : M4[3][c]));
+    }
+    uint32_t mu = 0;
 #pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    const uint32_t q = j & 3u;
-    m4row[c] = q == 0 ? M4[0][c] : (q == 1 ? M4[1][c] : (q == 2 ? M4[2][c] : M4[3][c]));
+    for (int i = 0; i < PT; ++i) mu = jj == (uint32_t)i ? 1u << P2_MU[i] : mu;
+    x = m_ext_row(x, m4row);
+#pragma unroll 1
+    for (int r = 0; r < HALF_FULL; ++r) x = m_ext_row(coop_sbox(add_const(x, t.p2_full[r][jj])), m4row);
+#pragma unroll 1
+    for (int k = 0; k < PARTIAL; ++k) {
+      const uint64_t s = coop_sbox(add_const(x, t.p2_partial[k]));
+      x = j ? x : s;
+      Limbs l(x, keep);
+      l.add_ror<8>();
+      l.add_ror<4>();
+      l.add_ror<2>();
+      l.add_ror<1>();
+      uint64_t lo = (uint64_t)gl::lo32(x) * mu, hi = (uint64_t)gl::hi32(x) * mu;
+      l.add_to(lo, hi);
+      x = coop_join(lo, hi);
+    }
+#pragma unroll 1
+    for (int r = 0; r < HALF_FULL; ++r) x = m_ext_row(coop_sbox(add_const(x, t.p2_full[HALF_FULL + r][jj])), m4row);
   }
-  const uint32_t jj = j < PT ? j : PT - 1;
-  x = coop_m_ext(x, j, m4row);
-#pragma unroll 1
-  for (int r = 0; r < HALF_FULL; ++r) x = coop_m_ext(sbox(gl::add(x, t.p2_full[r][jj])), j, m4row);
-#pragma unroll 1
-  for (int k = 0; k < PARTIAL; ++k) {
-    const uint64_t s = sbox(gl::add(x, t.p2_partial[k]));
-    x = coop_m_int(j == 0 ? s : x, j);
+
+  template <int H> __device__ __forceinline__ void permute_h(uint64_t &x) const {
+    if constexpr (H == 0) permute(x);
+    else permute2(x);
   }
-#pragma unroll 1
-  for (int r = 0; r < HALF_FULL; ++r) x = coop_m_ext(sbox(gl::add(x, t.p2_full[HALF_FULL + r][jj])), j, m4row);
+};
+
+__device__ __forceinline__ void coop_stage_table(CoopLds &l) {
+  const uint64_t *src = (const uint64_t *)&pos_table;
+  uint64_t *dst = (uint64_t *)&l.t;
+  for (uint32_t i = threadIdx.x; i < sizeof(PosTable) / sizeof(uint64_t); i += blockDim.x) dst[i] = src[i];
 }
 
+// `layers` consecutive node layers, the first of `count` nodes: a workgroup
+// hashes COOP_GROUPS nodes of the first layer and keeps their digests in LDS
+// for the next, so one launch climbs up to log2(COOP_GROUPS) + 1 layers
+// (count is a multiple of COOP_GROUPS or below it and a power of two when
+// layers > 1).  Layer l's digests go to its place behind the layers before it.
+constexpr uint32_t COOP_MAX_LAYERS = 6;
+static_assert(COOP_GROUPS == 1u << (COOP_MAX_LAYERS - 1), "");
 template <int H>
-__global__ __launch_bounds__(256) void poseidon_nodes_coop_kernel(const uint64_t *__restrict__ values,
-                                                                  uint64_t *__restrict__ results, uint32_t count) {
-  __shared__ PosTable lt;
-  {
-    const uint64_t *src = (const uint64_t *)&pos_table;
-    uint64_t *dst = (uint64_t *)&lt;
-    for (uint32_t i = threadIdx.x; i < sizeof(PosTable) / sizeof(uint64_t); i += blockDim.x) dst[i] = src[i];
-  }
-  __syncthreads();
-  const uint32_t g = blockIdx.x * (blockDim.x / COOP_LANES) + threadIdx.x / COOP_LANES;
-  const uint32_t j = threadIdx.x % COOP_LANES;
-  if (g >= count) return;  // whole groups leave together
+__global__ __launch_bounds__(COOP_NT) void poseidon_nodes_coop_kernel(const uint64_t *__restrict__ values,
+                                                                      uint64_t *__restrict__ results, uint32_t count,
+                                                                      uint32_t layers) {
+  __shared__ CoopLds lds;
+  __shared__ uint64_t digest[COOP_GROUPS][CAP];
+  coop_stage_table(lds);
+  const uint32_t group = threadIdx.x / COOP_LANES, j = threadIdx.x % COOP_LANES;
+  uint64_t g = (uint64_t)blockIdx.x * COOP_GROUPS + group;
   // element j: left[j] (j < 4), right[j - 4] (4 <= j < 8), capacity 0
   uint64_t x = 0;
-  if (j < 2 * CAP) x = gl::canon(values[2 * ((uint64_t)g + (uint64_t)(j & 3u) * count) + (j >> 2)]);
-  if constexpr (H == 0) coop_permute(x, j, lt);
-  else coop_permute2(x, j, lt);
-  if (j < CAP) results[g + (uint64_t)j * count] = x;
+  if (j < 2 * CAP && g < count) x = values[2 * (g + (uint64_t)(j & 3u) * count) + (j >> 2)];
+  __syncthreads();
+  const Coop c(lds, j, group);
+  uint32_t active = COOP_GROUPS;
+  for (uint32_t l = 0; l < layers; ++l) {
+    const bool on = group < active && g < count;
+    if (on) {
+      c.permute_h<H>(x);
+      if (j < CAP) {
+        const uint64_t d = gl::canon(x);
+        results[g + (uint64_t)j * count] = d;
+        digest[group][j] = d;
+      }
+    }
+    if (l + 1 == layers) return;
+    __syncthreads();
+    results += (uint64_t)CAP * count;
+    count /= 2;
+    active /= 2;
+    g = (uint64_t)blockIdx.x * active + group;
+    x = 0;
+    if (j < 2 * CAP && group < active) x = digest[2 * group + (j >> 2)][j & 3u];
+    __syncthreads();
+  }
 }
 
 // Cooperative leaves (src/poseidon.rs:194-216): the absorption of
-// poseidon_leaves_kernel with one state over a 16-lane group; for each chunk,
-// lane j < 8 loads position off + j (= c rows + r) into state element j.
+// poseidon_leaves_kernel with one state over a 16-lane row; for each chunk,
+// lane j < 8 takes position off + j (= c rows + r) into state element j, read
+// one chunk ahead.
 template <int H>
-__global__ __launch_bounds__(256) void poseidon_leaves_coop_kernel(const uint64_t *__restrict__ values,
-                                                                   uint64_t *__restrict__ results,
-                                                                   uint32_t log_rows, uint32_t cols, uint32_t count,
-                                                                   bool load_intermediate, bool store_intermediate) {
-  __shared__ PosTable lt;
-  {
-    const uint64_t *src = (const uint64_t *)&pos_table;
-    uint64_t *dst = (uint64_t *)&lt;
-    for (uint32_t i = threadIdx.x; i < sizeof(PosTable) / sizeof(uint64_t); i += blockDim.x) dst[i] = src[i];
-  }
-  __syncthreads();
-  const uint32_t g = blockIdx.x * (blockDim.x / COOP_LANES) + threadIdx.x / COOP_LANES;
-  const uint32_t j = threadIdx.x % COOP_LANES;
-  if (g >= count) return;  // whole groups leave together
+__global__ __launch_bounds__(COOP_NT) void poseidon_leaves_coop_kernel(const uint64_t *__restrict__ values,
+                                                                       uint64_t *__restrict__ results,
+                                                                       uint32_t log_rows, uint32_t cols, uint32_t count,
+                                                                       bool load_intermediate,
+                                                                       bool store_intermediate) {
+  __shared__ CoopLds lds;
+  coop_stage_table(lds);
+  const uint32_t group = threadIdx.x / COOP_LANES, j = threadIdx.x % COOP_LANES;
+  const uint64_t g = (uint64_t)blockIdx.x * COOP_GROUPS + group;
   const uint64_t rows = 1ull << log_rows;
-  uint64_t x = 0;
-  if (load_intermediate && j >= RATE && j < PT) x = gl::canon(results[g + (uint64_t)(j - RATE) * count]);
   const uint64_t col_stride = rows * count;
-  const uint64_t *base = values + (uint64_t)g * rows;
+  const uint64_t *base = values + g * rows;
   const uint64_t total = rows * cols;
+  const bool on = g < count;
+  auto chunk = [&](uint64_t off) -> uint64_t {
+    const uint64_t k = off + j;
+    return on && j < RATE && k < total ? base[(k & (rows - 1)) + (k >> log_rows) * col_stride] : 0ull;
+  };
+  uint64_t x = 0, next = chunk(0);
+  if (on && load_intermediate && j >= RATE && j < PT) x = results[g + (uint64_t)(j - RATE) * count];
+  __syncthreads();
+  if (!on) return;  // whole rows leave together, and no barrier follows
+  const Coop c(lds, j, group);
   for (uint64_t off = 0; off < total; off += RATE) {
-    if (j < RATE) {
-      const uint64_t k = off + j;
-      x = k < total ? gl::canon(base[(k & (rows - 1)) + (k >> log_rows) * col_stride]) : 0ull;
-    }
-    if constexpr (H == 0) coop_permute(x, j, lt);
-    else coop_permute2(x, j, lt);
+    if (j < RATE) x = next;
+    next = chunk(off + RATE);
+    c.permute_h<H>(x);
   }
   // the digest is state[0..4], the stored capacity state[8..12]
+  x = gl::canon(x);
   if (store_intermediate) {
     if (j >= RATE && j < PT) results[g + (uint64_t)(j - RATE) * count] = x;
   } else if (j < CAP) {
@@ -876,13 +1012,14 @@ int require_table() {
 
 using TableUse = std::shared_lock<std::shared_mutex>;
 
+// COOP: always the cooperative kernel; otherwise the cooperative kernel for
+// at most COOP_MAX_NODES leaves and one thread per leaf above.
 template <int H, bool COOP>
 int launch_leaves(const uint64_t *values, uint64_t *results, uint32_t log_rows, uint32_t cols, uint32_t count,
                   bool load, bool store, hipStream_t s) {
   if (count == 0) return BC_SUCCESS;
-  if constexpr (COOP) {
-    constexpr uint32_t per_block = 256 / COOP_LANES;
-    poseidon_leaves_coop_kernel<H><<<dim3((count + per_block - 1) / per_block), dim3(256), 0, s>>>(
+  if (COOP || count <= COOP_MAX_NODES) {
+    poseidon_leaves_coop_kernel<H><<<dim3((count + COOP_GROUPS - 1) / COOP_GROUPS), dim3(COOP_NT), 0, s>>>(
         values, results, log_rows, cols, count, load, store);
   } else {
     poseidon_leaves_kernel<H><<<dim3((count + 255) / 256), dim3(256), 0, s>>>(values, results, 1u << log_rows, cols,
@@ -891,20 +1028,31 @@ int launch_leaves(const uint64_t *values, uint64_t *results, uint32_t log_rows, 
   return hipGetLastError();
 }
 
-// COOP: always the cooperative kernel (the reference's
-// launch_cooperative_nodes_kernel); otherwise the cooperative kernel for
-// layers of at most COOP_MAX_NODES nodes and one thread per node above.
+// Node layers [values -> results], the first of `count` nodes (layers > 1: a
+// power of two).  COOP: always the cooperative kernel (the reference's
+// launch_cooperative_nodes_kernel); otherwise the cooperative kernel, several
+// layers to a launch, for layers of at most COOP_MAX_NODES nodes, and one
+// thread per node above.
 template <int H, bool COOP = false>
-int launch_nodes(const uint64_t *values, uint64_t *results, uint32_t count, hipStream_t s) {
-  if (count == 0) return BC_SUCCESS;
-  if (COOP || count <= COOP_MAX_NODES) {
-    constexpr uint32_t per_block = 256 / COOP_LANES;
-    poseidon_nodes_coop_kernel<H><<<dim3((count + per_block - 1) / per_block), dim3(256), 0, s>>>(values, results,
-                                                                                                 count);
-  } else {
-    poseidon_nodes_kernel<H><<<dim3((count + 255) / 256), dim3(256), 0, s>>>(values, results, count);
+int launch_nodes(const uint64_t *values, uint64_t *results, uint32_t count, uint32_t layers, hipStream_t s) {
+  while (layers && count) {
+    uint32_t n = 1;
+    if (COOP || count <= COOP_MAX_NODES) {
+      n = layers < COOP_MAX_LAYERS ? layers : COOP_MAX_LAYERS;
+      poseidon_nodes_coop_kernel<H>
+          <<<dim3((count + COOP_GROUPS - 1) / COOP_GROUPS), dim3(COOP_NT), 0, s>>>(values, results, count, n);
+    } else {
+      poseidon_nodes_kernel<H><<<dim3((count + 255) / 256), dim3(256), 0, s>>>(values, results, count);
+    }
+    const hipError_t err = hipGetLastError();
+    if (err != hipSuccess) return err;
+    for (layers -= n; n; --n) {
+      values = results;
+      results += (uint64_t)CAP * count;
+      count /= 2;
+    }
   }
-  return hipGetLastError();
+  return BC_SUCCESS;
 }
 
 // The entry points of both hashes share these (src/poseidon.rs is generic
@@ -939,7 +1087,7 @@ int nodes_impl(const uint64_t *values, uint64_t values_len, uint64_t *results, u
   if (!values || !results || count > 0xFFFFFFFFull) return BC_ERROR_INVALID_VALUE;
   const int rc = require_table();
   if (rc != BC_SUCCESS) return rc;
-  return launch_nodes<H, COOP>(values, results, (uint32_t)count, (hipStream_t)stream);
+  return launch_nodes<H, COOP>(values, results, (uint32_t)count, 1, (hipStream_t)stream);
 }
 
 template <int H>
@@ -949,24 +1097,14 @@ int tree_nodes_impl(const uint64_t *values, uint64_t values_len, uint64_t *resul
   // of what remains of `results`
   if (layers_count == 0) return BC_SUCCESS;
   if (values_len % RATE != 0 || values_len != results_len) return BC_ERROR_INVALID_VALUE;
-  const uint64_t leaves = values_len / RATE;
-  if (leaves == 0 || (leaves & (leaves - 1)) != 0) return BC_ERROR_INVALID_VALUE;
+  const uint64_t nodes = values_len / RATE;  // of the first layer
+  if (nodes == 0 || (nodes & (nodes - 1)) != 0) return BC_ERROR_INVALID_VALUE;
   if (layers_count > 64 || (layers_count > 1 && (values_len >> (layers_count - 1)) < RATE))
     return BC_ERROR_INVALID_VALUE;
   const int rc = require_table();
   if (rc != BC_SUCCESS) return rc;
-  const uint64_t *in = values;
-  uint64_t len = values_len;
-  uint64_t *out = results;
-  for (uint32_t l = 0; l < layers_count; ++l) {
-    const uint64_t half = len / 2;
-    const int e = nodes_impl<H>(in, len, out, half, stream);
-    if (e != BC_SUCCESS) return e;
-    in = out;
-    out += half;
-    len = half;
-  }
-  return BC_SUCCESS;
+  if (!values || !results || nodes > 0xFFFFFFFFull) return BC_ERROR_INVALID_VALUE;
+  return launch_nodes<H>(values, results, (uint32_t)nodes, layers_count, (hipStream_t)stream);
 }
 
 template <int H>
