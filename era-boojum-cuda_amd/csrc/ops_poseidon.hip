@@ -492,10 +492,13 @@ __global__ __launch_bounds__(256) void poseidon_nodes_kernel(const uint64_t *__r
 // round.  Sums over the row are taken on 22-bit limbs with row rotations
 // (plain 32-bit additions, 12 instructions for the 16 lanes); the MDS row and
 // the 4-tiles gather their words through the wave's LDS, a round's constants
-// come from LDS.  Used for layers and leaf sets of at most COOP_MAX_NODES
-// (the reference likewise switches to cooperative kernels for small layers at
-// the same size, src/poseidon.rs:71,279-283).
-constexpr uint32_t COOP_LANES = 16, COOP_MAX_NODES = 1u << 14;
+// come from LDS.  Used for layers and leaf sets of at most coop_max<H>() (the
+// reference likewise switches to cooperative kernels for small layers,
+// src/poseidon.rs:71,279-283).  Four permutations a leaf, 16 lanes against
+// one: Poseidon 129 / 256 us at 2^14, 209 / 259 at 2^15, 373 / 268 at 2^16;
+// Poseidon2 96 / 121 us at 2^14, 152 / 121 at 2^15.
+constexpr uint32_t COOP_LANES = 16;
+template <int H> constexpr uint32_t coop_max() { return H == 0 ? 1u << 15 : 1u << 14; }
 constexpr uint32_t COOP_NT = 512, COOP_GROUPS = COOP_NT / COOP_LANES;  // two waves per SIMD issue side by side
 
 // A row's words in LDS, twice in a row so that word (j + i) mod 12 is at j + i.
@@ -1013,12 +1016,12 @@ int require_table() {
 using TableUse = std::shared_lock<std::shared_mutex>;
 
 // COOP: always the cooperative kernel; otherwise the cooperative kernel for
-// at most COOP_MAX_NODES leaves and one thread per leaf above.
+// at most coop_max<H>() leaves and one thread per leaf above.
 template <int H, bool COOP>
 int launch_leaves(const uint64_t *values, uint64_t *results, uint32_t log_rows, uint32_t cols, uint32_t count,
                   bool load, bool store, hipStream_t s) {
   if (count == 0) return BC_SUCCESS;
-  if (COOP || count <= COOP_MAX_NODES) {
+  if (COOP || count <= coop_max<H>()) {
     poseidon_leaves_coop_kernel<H><<<dim3((count + COOP_GROUPS - 1) / COOP_GROUPS), dim3(COOP_NT), 0, s>>>(
         values, results, log_rows, cols, count, load, store);
   } else {
@@ -1031,13 +1034,13 @@ int launch_leaves(const uint64_t *values, uint64_t *results, uint32_t log_rows, 
 // Node layers [values -> results], the first of `count` nodes (layers > 1: a
 // power of two).  COOP: always the cooperative kernel (the reference's
 // launch_cooperative_nodes_kernel); otherwise the cooperative kernel, several
-// layers to a launch, for layers of at most COOP_MAX_NODES nodes, and one
+// layers to a launch, for layers of at most coop_max<H>() nodes, and one
 // thread per node above.
 template <int H, bool COOP = false>
 int launch_nodes(const uint64_t *values, uint64_t *results, uint32_t count, uint32_t layers, hipStream_t s) {
   while (layers && count) {
     uint32_t n = 1;
-    if (COOP || count <= COOP_MAX_NODES) {
+    if (COOP || count <= coop_max<H>()) {
       n = layers < COOP_MAX_LAYERS ? layers : COOP_MAX_LAYERS;
       poseidon_nodes_coop_kernel<H>
           <<<dim3((count + COOP_GROUPS - 1) / COOP_GROUPS), dim3(COOP_NT), 0, s>>>(values, results, count, n);

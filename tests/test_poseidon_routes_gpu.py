@@ -1,6 +1,7 @@
 """GPU parity of the two hashing routes on either side of their switch: leaf
-sets and node layers of at most 2^14 take 16 lanes a state (several node
-layers to a launch), larger ones one lane.  Bit-exact against the oracle."""
+sets and node layers of at most 2^14 (Poseidon2) or 2^15 (Poseidon) take 16
+lanes a state (several node layers to a launch), larger ones one lane.
+Bit-exact against the oracle."""
 import numpy as np
 import pytest
 
@@ -21,7 +22,7 @@ def values(count, seed):
 
 
 @pytest.mark.parametrize("p", HASHES)
-@pytest.mark.parametrize("count", [1, 31, 33, 1 << 14, (1 << 14) + 1])
+@pytest.mark.parametrize("count", [1, 31, 33, 1 << 14, (1 << 14) + 1, (1 << 15) + 1])
 @pytest.mark.parametrize("log_rows,cols", [(0, 1), (0, 13), (1, 8), (2, 3), (3, 5)])
 def test_leaves_either_side_of_the_switch(consts, p, count, log_rows, cols):  # noqa: F811
     import torch
@@ -34,7 +35,7 @@ def test_leaves_either_side_of_the_switch(consts, p, count, log_rows, cols):  # 
 
 
 @pytest.mark.parametrize("p", HASHES)
-@pytest.mark.parametrize("count", [(1 << 14) - 1, (1 << 14) + 3])
+@pytest.mark.parametrize("count", [(1 << 14) - 1, (1 << 14) + 3, (1 << 15) + 3])
 def test_checkpoints_across_the_switch(consts, p, count):  # noqa: F811
     """Capacity stored by one route's kernel and loaded by the other's."""
     import torch
