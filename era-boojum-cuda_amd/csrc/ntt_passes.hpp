@@ -31,6 +31,8 @@
 #include "gl_lazy.hpp"
 #include "ntt_device.hpp"
 
+#include <stddef.h>
+
 namespace bc {
 namespace pass {
 
@@ -138,16 +140,25 @@ struct Buf {
   }
 };
 
+// A pointer read from memory, known to point to global memory (a generic
+// pointer's accesses also wait on LDS).
+template <class T> __device__ __forceinline__ T *global_ptr(T *p) {
+  return (T *)(__attribute__((address_space(1))) T *)(uint64_t)p;
+}
+
 // Column addressing: one matrix (base + c * stride) for the standalone
-// launches, or a per-column pointer table (CT) for ragged job groups.
+// launches, or a per-column pointer table (CT) for ragged job groups; the
+// table does not change during a launch, and for a uniform c its entry is a
+// scalar load.
 template <bool CT> __device__ __forceinline__ const uint64_t *in_col(const FastArgs &a, uint64_t c) {
-  if constexpr (CT) return a.cols[c].in;
+  if constexpr (CT) return global_ptr((const uint64_t *)((const __attribute__((address_space(4))) uint64_t *)(uint64_t)a.cols)[2 * c]);
   else return a.in + c * a.stride_in;
 }
 template <bool CT> __device__ __forceinline__ uint64_t *out_col(const FastArgs &a, uint64_t c) {
-  if constexpr (CT) return a.cols[c].out;
+  if constexpr (CT) return global_ptr((uint64_t *)((const __attribute__((address_space(4))) uint64_t *)(uint64_t)a.cols)[2 * c + 1]);
   else return a.out + c * a.stride_out;
 }
+static_assert(sizeof(ColPtrs) == 16 && offsetof(ColPtrs, in) == 0 && offsetof(ColPtrs, out) == 8, "");
 
 // Addressing of a contiguous-pass tile: 4096 consecutive points of one column
 // (position pos0 of column col), or (MC: single-pass transforms shorter than
@@ -287,7 +298,7 @@ __device__ __forceinline__ void contig_run(const FastArgs &a, PassLds &sh, uint3
   // these read the (cache-resident) level table each time, which keeps 30
   // VGPRs free.
   const uint64_t *tw0 = lvl_table<LH, INV>(a.tab) + (t & ((1u << (LH - 4)) - 1u));
-  constexpr bool TW_REGS = WL && !DIT;
+  constexpr bool TW_REGS = WL && !DIT && !CT;
   uint64_t twr[16];
   if constexpr (TW_REGS) {
 #pragma unroll
@@ -605,14 +616,21 @@ __device__ __forceinline__ void strided_run(const FastArgs &a, PassLds &sh, uint
 
   p_begin = uniform64(p_begin);
   p_end = uniform64(p_end);
+  constexpr bool PREFETCH = !CT;
   uint64_t pf[16];
-  if (p_begin < p_end) load(p_begin, pf);
+  if constexpr (PREFETCH) {
+    if (p_begin < p_end) load(p_begin, pf);
+  }
   __syncthreads();  // tw0 and coset factors staged
   for (uint64_t p = p_begin; p < p_end; ++p) {
     uint64_t x[16];
+    if constexpr (PREFETCH) {
 #pragma unroll
-    for (int i = 0; i < 16; ++i) x[i] = pf[i];
-    if (p + 1 < p_end) load(p + 1, pf);  // prefetch: in flight during this pair's math
+      for (int i = 0; i < 16; ++i) x[i] = pf[i];
+      if (p + 1 < p_end) load(p + 1, pf);  // in flight during this pair's math
+    } else {
+      load(p, x);
+    }
     if constexpr (!DIT) {
       if constexpr (MODE == MODE_LDE_IN) gl::mul_each<1, 15, gl::ANY, true>(x, [&](int i) { return sh.cf[i]; });
       gl::dft_lazy<4, INV, false, gl::ANY>(x);

@@ -42,18 +42,39 @@ __shared__ PassLds ragged_lds;
 // One out-of-line function per variant: each gets its own register
 // allocation instead of the maximum over every variant inlined into the
 // persistent loop.
+// A call passes the segment's address in VGPRs, as a generic pointer.  Taken
+// back into SGPRs as a pointer to memory that does not change during the
+// launch, its fields are scalar loads and stay in SGPRs, as kernel arguments
+// would (loaded as they come, every value of the pass arguments took VGPRs and
+// every buffer access a loop over the lanes' descriptors).
+__device__ __forceinline__ FastArgs uniform_args(const RaggedSeg *sg) {
+  using Word = const __attribute__((address_space(4))) uint64_t;
+  static_assert(sizeof(FastArgs) % sizeof(uint64_t) == 0, "");
+  constexpr size_t N = sizeof(FastArgs) / sizeof(uint64_t);
+  Word *src = (Word *)uniform64((uint64_t)&sg->a);
+  uint64_t w[N];
+#pragma unroll
+  for (size_t i = 0; i < N; ++i) w[i] = src[i];
+  FastArgs a;
+  __builtin_memcpy(&a, w, sizeof a);
+  for (const uint64_t **p : {&a.tab.lvl_tw, &a.tab.w_fine, &a.tab.w_coarse, &a.tab.g_fine, &a.tab.g_coarse,
+                             &a.tab.gi_fine, &a.tab.gi_coarse})
+    *p = global_ptr(*p);
+  return a;
+}
+
 template <int LH, bool MC, uint32_t DM>
 __device__ __noinline__ void contig_unit(const RaggedSeg *sg, uint32_t b, uint32_t e) {
   constexpr bool INV = DM >= 2;
   constexpr int MODE = DM == 1 ? MODE_LDE_IN : (DM == 3 ? MODE_NINV : MODE_NONE);
-  contig_run<LH, INV, INV, MODE, MC, true>(sg->a, ragged_lds, b, e, 1);
+  contig_run<LH, INV, INV, MODE, MC, true>(uniform_args(sg), ragged_lds, b, e, 1);
 }
 
 template <int LH, uint32_t DM>
 __device__ __noinline__ void strided_unit(const RaggedSeg *sg, uint32_t rho, uint64_t b, uint64_t e) {
   constexpr bool INV = DM >= 2;
   constexpr int MODE = DM == 1 ? MODE_LDE_IN : (DM == 3 ? MODE_NINV : MODE_NONE);
-  strided_run<LH, INV, INV, MODE, true>(sg->a, ragged_lds, rho, b, e);
+  strided_run<LH, INV, INV, MODE, true>(uniform_args(sg), ragged_lds, rho, b, e);
 }
 
 template <int LH, bool MC>
