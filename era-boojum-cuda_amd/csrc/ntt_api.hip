@@ -60,6 +60,15 @@ int run_general(bc_context *ctx, const uint64_t *inputs, uint64_t *outputs, uint
   return launch_pass(a, inverse, bitrev_inputs, s);
 }
 
+// Fixes a strided pass's launch shape for `positions` r-ranges; false if it
+// cannot be launched.
+bool strided_shape(PassDesc &pd, uint64_t positions, uint32_t tuned_bpw, uint32_t *groups) {
+  if (positions > 0x7FFFFFFFull) return false;
+  pd.positions = positions;
+  *groups = strided_groups(pd.pairs, positions, tuned_bpw, &pd.a.blocks_per_wg);
+  return true;
+}
+
 }  // namespace
 
 Tables current_tables(bool &ok) {
@@ -189,9 +198,7 @@ extern "C" int bc_batch_ntt_internal(const uint64_t *inputs, uint64_t *outputs, 
   uint32_t groups[8] = {};
   for (int k = 0; k < np; ++k) {
     PassDesc &pd = passes[k];
-    if (pd.contig) continue;
-    if (pd.positions > 0x7FFFFFFFull) return BC_ERROR_INVALID_VALUE;
-    groups[k] = strided_groups(pd.pairs, pd.positions, tp.strided_bpw, &pd.a.blocks_per_wg);
+    if (!pd.contig && !strided_shape(pd, pd.positions, tp.strided_bpw, &groups[k])) return BC_ERROR_INVALID_VALUE;
   }
   for (int k = 0; k < np; ++k) {
     const PassDesc &pd = passes[k];
@@ -243,6 +250,50 @@ extern "C" int bc_batch_ntt_in_place(uint64_t *inputs_matrix, size_t inputs_len,
 
 namespace bc {
 namespace {
+
+// All 2^log_blowup forward coset transforms of an LDE, pass by pass: the
+// first pass of every coset in one launch, which reads the coefficients from
+// memory once; each later pass in one launch over all blocks, a column's
+// blocks being 2^log_blowup consecutive transforms, so that a column is just
+// 2^log_blowup times as long.  Returns NOT_BATCHED (nothing queued)
+// for shapes that go coset by coset.
+constexpr int NOT_BATCHED = -1000;
+int lde_cosets(bc_context *ctx, const uint64_t *coeffs, uint64_t *outputs, uint32_t log_n, uint32_t num_cols,
+               uint32_t stride_coeffs, uint32_t stride_out, uint32_t log_blowup, bool bitrev_coeffs, hipStream_t s) {
+  if (log_n < TILE_LOG || log_blowup == 0 || num_cols == 0) return NOT_BATCHED;
+  PassDesc passes[8];
+  const int np = describe_fast_passes(ctx->tab, coeffs, outputs, log_n, num_cols, stride_coeffs, stride_out,
+                                      bitrev_coeffs, false, log_blowup, 0, passes);
+  if (np <= 0) return NOT_BATCHED;
+  const TuneParams tp = tuned(log_n, num_cols);
+  uint32_t groups[8] = {};
+  for (int k = 0; k < np; ++k) {
+    PassDesc &pd = passes[k];
+    uint64_t positions = pd.positions;
+    if (k == 0) {
+      if (pd.mode != MODE_LDE_IN) return NOT_BATCHED;
+      pd.a.coset_log = log_blowup;
+      pd.a.coset_brev = !bitrev_coeffs;
+      positions <<= log_blowup;
+    } else {
+      if (pd.mode != MODE_NONE || ((uint64_t)pd.a.tiles << log_blowup) > 0xFFFFFFFFull) return NOT_BATCHED;
+      pd.a.log_n += log_blowup;
+      pd.a.tiles <<= log_blowup;
+      pd.pairs <<= log_blowup;
+    }
+    if (!pd.contig && !strided_shape(pd, positions, tp.strided_bpw, &groups[k])) return NOT_BATCHED;
+  }
+  for (int k = 0; k < np; ++k) {
+    const PassDesc &pd = passes[k];
+    const hipError_t err =
+        pd.contig ? launch_contig(pd.a, (int)pd.log_h, false, bitrev_coeffs, pd.mode, tp.contig_grid, s)
+                  : launch_strided(pd.a, (int)pd.log_h, false, bitrev_coeffs, pd.mode, (uint32_t)pd.positions,
+                                   groups[k], s);
+    if (err != hipSuccess) return err;
+  }
+  return BC_SUCCESS;
+}
+
 uint32_t brev_small(uint32_t x, uint32_t bits) {
   uint32_t r = 0;
   for (uint32_t i = 0; i < bits; ++i) r |= ((x >> i) & 1u) << (bits - 1 - i);
@@ -266,6 +317,13 @@ extern "C" int bc_batch_lde(const uint64_t *inputs, uint64_t *coeffs, uint64_t *
   if (rc != BC_SUCCESS) return rc;
   // 2. one forward coset transform per coset; natural coefficients give
   //    bit-reversed evaluations (n2b) and vice versa (b2n)
+  bc_context *ctx = current_context();
+  if (!ctx) return BC_ERROR_NOT_INITIALIZED;
+  if (n <= stride_coeffs) {
+    rc = lde_cosets(ctx, coeffs, outputs, log_n, num_cols, stride_coeffs, (uint32_t)stride_out, log_blowup,
+                    !bitrev_inputs, (hipStream_t)stream);
+    if (rc != NOT_BATCHED) return rc;
+  }
   for (uint32_t c = 0; c < (1u << log_blowup); ++c) {
     const uint32_t blk = bitrev_inputs ? brev_small(c, log_blowup) : c;
     rc = bc_batch_ntt_internal(coeffs, outputs + (uint64_t)blk * n, log_n, num_cols, stride_coeffs,

@@ -16,7 +16,14 @@ template <int LH, bool INV, bool DIT, int MODE, bool MC>
 __global__ __launch_bounds__(NT, DIT && LH != 12 ? 2 : 3) void
     ntt_contig_kernel(FastArgs a) {
   __shared__ PassLds sh;
-  contig_run<LH, INV, DIT, MODE, MC>(a, sh, blockIdx.x, a.tiles, gridDim.x);
+  uint32_t wg = blockIdx.x, wgs = gridDim.x;
+  if constexpr (MODE == MODE_LDE_IN && !MC) {
+    if (a.coset_log) {
+      wg = coset_split(a, wg, wgs);
+      wgs >>= a.coset_log;
+    }
+  }
+  contig_run<LH, INV, DIT, MODE, MC>(a, sh, wg, a.tiles, wgs);
 }
 
 // Three workgroups per CU for n2b h = 7 and 8 (2-6 spilled dwords; two per CU
@@ -28,7 +35,11 @@ __global__ __launch_bounds__(NT, LH >= 7 && !DIT ? 3 : 2) void ntt_strided_kerne
   const uint64_t total = (uint64_t)a.num_cols << (a.log_n - a.log_N);
   const uint64_t p_begin = (uint64_t)blockIdx.y * a.blocks_per_wg;
   const uint64_t p_end = p_begin + a.blocks_per_wg < total ? p_begin + a.blocks_per_wg : total;
-  strided_run<LH, INV, DIT, MODE>(a, sh, blockIdx.x, p_begin, p_end);
+  uint32_t rho = blockIdx.x;
+  if constexpr (MODE == MODE_LDE_IN) {
+    if (a.coset_log) rho = coset_split(a, rho, gridDim.x);
+  }
+  strided_run<LH, INV, DIT, MODE>(a, sh, rho, p_begin, p_end);
 }
 
 // -------------------------------------------------------------------------
@@ -114,7 +125,12 @@ hipError_t launch_contig(const FastArgs &a, int log_h, bool inverse, bool dit, i
                          hipStream_t stream) {
   if (a.tiles == 0) return hipSuccess;
   if (max_wgs == 0) max_wgs = default_contig_grid(dit);
-  const dim3 grid(a.tiles < max_wgs ? a.tiles : max_wgs);
+  uint32_t wgs = a.tiles < max_wgs ? a.tiles : max_wgs;
+  if (a.coset_log) {  // the cap is for all cosets together
+    const uint32_t cap = (max_wgs >> a.coset_log) > 8 ? max_wgs >> a.coset_log : 8;
+    wgs = (a.tiles < cap ? a.tiles : cap) << a.coset_log;
+  }
+  const dim3 grid(wgs);
   if (a.log_n < TILE_LOG) {  // single pass over whole columns, several per tile
     switch (log_h) {
     case 8: return contig_dir<8, true>(a, inverse, dit, mode, grid, stream);

@@ -83,6 +83,11 @@ struct FastArgs {
   uint32_t tiles;          // contiguous passes: number of 4096-point tiles
   uint32_t blocks_per_wg;  // strided passes: (column, block) pairs per workgroup
   const ColPtrs *cols;     // column-table addressing (ragged): column c at cols[c], in/out/strides unused
+  // LDE: the first pass of all 2^coset_log cosets (0: of one) in one launch of
+  // 2^coset_log times the workgroups.  Coset c is written at out +
+  // block(c) << log_n, block(c) = c, or its bit reversal (coset_brev).
+  uint32_t coset_log;
+  uint32_t coset_brev;
 };
 
 // Scaling folded into a pass (see plan in ntt_api.hip).
