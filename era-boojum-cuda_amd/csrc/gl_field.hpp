@@ -94,23 +94,37 @@ __device__ __forceinline__ uint64_t mad_carry(uint32_t a, uint32_t b, uint64_t c
   return r;
 }
 
-// mad_carry with b in an SGPR (b the same in every lane).
-__device__ __forceinline__ uint64_t mad_carry_s(uint32_t a, uint32_t b, uint64_t c, uint64_t &carry) {
-  uint64_t r;
-  asm("v_mad_u64_u32 %0, %1, %2, %3, %4" : "=v"(r), "=s"(carry) : "v"(a), "s"(b), "v"(c));
-  return r;
+// Y = x - h - cin (cin a lane mask), and n = l less Y's borrow, with n's own
+// borrow in b2.  cin is read without wait states: in a product it comes from
+// the multiply-add t2, and h and l from a widening move and a multiply-add
+// that both follow it.
+__device__ __forceinline__ uint64_t sub_fold(uint32_t x0, uint32_t x1, uint32_t h, uint32_t l, uint64_t cin,
+                                             uint32_t &n, uint64_t &b2) {
+  uint32_t lo, hi;
+  asm("v_subb_co_u32_e64 %[lo], %[b], %[x0], %[h], %[cin]\n\t"
+      "s_nop 1\n\t"
+      "v_subb_co_u32_e64 %[hi], %[b], %[x1], 0, %[b]\n\t"
+      "s_nop 1\n\t"
+      "v_subb_co_u32_e64 %[n], %[b], %[l], 0, %[b]"
+      : [lo] "=&v"(lo), [hi] "=&v"(hi), [n] "=&v"(n), [b] "=&s"(b2)
+      : [x0] "v"(x0), [x1] "v"(x1), [h] "v"(h), [l] "v"(l), [cin] "s"(cin));
+  return ((uint64_t)hi << 32) | lo;
 }
 
-// z - h - cin (cin a lane mask) with the final borrow in `borrow`.
-__device__ __forceinline__ uint64_t sub32_borrow(uint64_t z, uint32_t h, uint64_t cin, uint64_t &borrow) {
-  uint32_t lo, hi;
-  uint64_t b0;
-  asm("s_nop 1\n\t"
-      "v_subb_co_u32_e64 %[lo], %[b0], %[zlo], %[h], %[cin]\n\t"
+// Canonical value of z + c 2^64 + w (lane masks c and w, w only where c), given
+// z + EPS + w < p wherever c is set.
+__device__ __forceinline__ uint64_t fold_carry(uint64_t z, uint64_t c, uint64_t w) {
+  uint32_t lo, hi, t;
+  uint64_t k;
+  asm("v_cmp_le_u64_e64 %[k], %[P], %[z]\n\t"
+      "s_or_b64 %[k], %[k], %[c]\n\t"
+      "v_cndmask_b32_e64 %[t], 0, -1, %[k]\n\t"
+      "v_addc_co_u32_e64 %[lo], %[k], %[z0], %[t], %[w]\n\t"
       "s_nop 1\n\t"
-      "v_subb_co_u32_e64 %[hi], %[bo], %[zhi], 0, %[b0]"
-      : [lo] "=&v"(lo), [hi] "=&v"(hi), [b0] "=&s"(b0), [bo] "=&s"(borrow)
-      : [zlo] "v"((uint32_t)z), [zhi] "v"((uint32_t)(z >> 32)), [h] "v"(h), [cin] "s"(cin));
+      "v_addc_co_u32_e64 %[hi], %[k], %[z1], 0, %[k]"
+      : [lo] "=&v"(lo), [hi] "=&v"(hi), [t] "=&v"(t), [k] "=&s"(k)
+      : [z] "v"(z), [z0] "v"((uint32_t)z), [z1] "v"((uint32_t)(z >> 32)), [c] "s"(c), [w] "s"(w), [P] "s"(P)
+      : "scc");
   return ((uint64_t)hi << 32) | lo;
 }
 
@@ -168,59 +182,39 @@ __device__ __forceinline__ uint64_t fold_plus(uint64_t x, uint64_t plus) {
 //   t0 = a0 b0,  t1 = a0 b1 + hi(t0)            (< 2^64)
 //   t2 = a1 b0 + t1 = T2 + c 2^64               (c: carry out, 65-bit sum)
 //   t3 = a1 b1 + hi(T2)                         (< 2^64)
-// so a b = X + lo(t3) 2^64 + (hi(t3) + c) 2^96 with X = lo(t0) + lo(T2) 2^32,
-// and with 2^64 = EPS, 2^96 = -1:
-//   a b = X + lo(t3) EPS - hi(t3) - c = Z + c2 2^64 - hi(t3) - c,
-// where Z + c2 2^64 = X + lo(t3) EPS is the fifth multiply-add.  Then
-// W = Z - hi(t3) - c with final borrow bw, and a b = W + (c2 - bw) 2^64:
-// c2 alone leaves W <= 2^64 - 2^33 (W + EPS < p); bw alone leaves
-// W >= 2^64 - 2^32 (W - EPS canonical); both or neither leave W for the
-// canonical check.  On gfx950 the carries stay in lane masks.
+// so a b = X + l 2^64 + (h + c) 2^96 with X = lo(t0) + lo(T2) 2^32, l = lo(t3),
+// h = hi(t3), and with 2^64 = EPS, 2^96 = -1: a b = X + l EPS - h - c.
+// Y = X - h - c may borrow 2^64; EPS for that borrow is one less in the factor
+// of the last multiply-add, Z = Y + (l - borrow) EPS.  Where l = 0 and there
+// is a borrow the factor wraps to 2^32 - 1 (borrow b2), 2^32 EPS = -1 too
+// much, so b2 is added back.  Z's carry out adds EPS: it leaves Z <= 2^64 -
+// 2^33, so Z + EPS + b2 < p, and b2 implies it.  On gfx950 the carries stay in
+// lane masks.  (gl_lazy.hpp has the same steps for several products side by
+// side, without the wait states.)
 GL_FN uint64_t mul(uint64_t a, uint64_t b) {
   const uint32_t a0 = (uint32_t)a, a1 = (uint32_t)(a >> 32);
   const uint32_t b0 = (uint32_t)b, b1 = (uint32_t)(b >> 32);
   const uint64_t t0 = (uint64_t)a0 * b0;
   const uint64_t t1 = (uint64_t)a0 * b1 + (t0 >> 32);
 #if defined(__HIP_DEVICE_COMPILE__)
-  uint64_t c, c2, bw;
+  uint64_t c, c2, b2;
+  uint32_t n;
   const uint64_t t2 = dev::mad_carry(a1, b0, t1, c);
   const uint64_t t3 = (uint64_t)a1 * b1 + (t2 >> 32);
-  const uint64_t z = dev::mad_carry((uint32_t)t3, 0xFFFFFFFFu, (t2 << 32) | (uint32_t)t0, c2);
-  const uint64_t w = dev::sub32_borrow(z, (uint32_t)(t3 >> 32), c, bw);
-  return dev::fold_masks(w, c2, bw);
+  const uint64_t y = dev::sub_fold((uint32_t)t0, (uint32_t)t2, (uint32_t)(t3 >> 32), (uint32_t)t3, c, n, b2);
+  const uint64_t z = dev::mad_carry(n, 0xFFFFFFFFu, y, c2);
+  return dev::fold_carry(z, c2, b2);
 #else
   const uint64_t p2 = (uint64_t)a1 * b0;
   const uint64_t t2 = p2 + t1;
   const bool c = t2 < p2;
   const uint64_t t3 = (uint64_t)a1 * b1 + (t2 >> 32);
-  const uint64_t x = (t2 << 32) | (uint32_t)t0;
-  const uint64_t z = (uint64_t)(uint32_t)t3 * EPS + x;
-  const bool c2 = z < x;
-  unsigned b0w, bw;
-  const uint32_t lo = __builtin_subc((uint32_t)z, (uint32_t)(t3 >> 32), (unsigned)c, &b0w);
-  const uint32_t hi = __builtin_subc((uint32_t)(z >> 32), 0u, b0w, &bw);
-  return fold(((uint64_t)hi << 32) | lo, c2 && !bw, bw && !c2);
-#endif
-}
-
-// mul for a b that is the same in every lane of the wave (the caller's
-// promise: lanes of another b get lane 0's).  On gfx950 b is taken into SGPRs,
-// so a loop-invariant b hoisted out of a loop costs no VGPRs.
-GL_FN uint64_t mul_uniform(uint64_t a, uint64_t b) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  const uint32_t a0 = (uint32_t)a, a1 = (uint32_t)(a >> 32);
-  const uint32_t b0 = __builtin_amdgcn_readfirstlane((uint32_t)b);
-  const uint32_t b1 = __builtin_amdgcn_readfirstlane((uint32_t)(b >> 32));
-  const uint64_t t0 = (uint64_t)a0 * b0;
-  const uint64_t t1 = (uint64_t)a0 * b1 + (t0 >> 32);
-  uint64_t c, c2, bw;
-  const uint64_t t2 = dev::mad_carry_s(a1, b0, t1, c);
-  const uint64_t t3 = (uint64_t)a1 * b1 + (t2 >> 32);
-  const uint64_t z = dev::mad_carry((uint32_t)t3, 0xFFFFFFFFu, (t2 << 32) | (uint32_t)t0, c2);
-  const uint64_t w = dev::sub32_borrow(z, (uint32_t)(t3 >> 32), c, bw);
-  return dev::fold_masks(w, c2, bw);
-#else
-  return mul(a, b);
+  const uint64_t x = (t2 << 32) | (uint32_t)t0, h = (t3 >> 32) + c;
+  const uint64_t y = x - h;
+  const uint32_t n = (uint32_t)t3 - (x < h);
+  const bool b2 = (uint32_t)t3 == 0 && x < h;
+  const uint64_t z = (uint64_t)n * EPS + y;
+  return z + (z < y || z >= P ? EPS : 0ull) + b2;
 #endif
 }
 

@@ -14,7 +14,11 @@
 // turn, so for N >= 3 a mask is read at least two instructions after it was
 // written and no wait states are spent; rows of 1 or 2 spend them in s_nops.
 // As much of a row as can be is one asm block: the compiler counts a block as
-// one instruction and would add wait states between two of them.
+// one instruction and would add wait states between two of them, and it does
+// not know the masks a block writes, so a block that starts by reading one
+// spends the states itself when N < 3 (sub_fold and sub_borrow need not: the
+// mask they read comes from the multiply-add t2, and between the two lie, for
+// every N, the move that widens t2's high word and the multiply-add t3).
 //
 // Lazy values.  Inside a DFT a value is V = x + e 2^64 with x any u64 and e a
 // small signed integer: a sum or difference is three carry instructions
@@ -182,7 +186,7 @@ template <int N> struct Rows;
                                const Mask *w) {                                                                        \
       Mask k[N];                                                                                                       \
       uint32_t t[N];                                                                                                   \
-      asm(GL_CAT##N(GL_S_ONES) GL_CAT##N(GL_S_FLO) GL_WAIT##N GL_CAT##N(GL_S_FHI)                                      \
+      asm(GL_WAIT##N GL_CAT##N(GL_S_ONES) GL_CAT##N(GL_S_FLO) GL_WAIT##N GL_CAT##N(GL_S_FHI)                           \
           : GL_LIST##N(GL_O_r0), GL_LIST##N(GL_O_r1), GL_LIST##N(GL_O_t), GL_LIST##N(GL_O_k)                           \
           : GL_LIST##N(GL_I_x0), GL_LIST##N(GL_I_x1), GL_LIST##N(GL_I_m), GL_LIST##N(GL_I_w));                         \
     }                                                                                                                  \
@@ -395,6 +399,27 @@ GL_FN void mul_row(uint64_t *o, const uint64_t *a, const uint64_t *b, int32_t *e
     else W::fold_any(r0, r1, z0, z1, c2, b2);
     join(o, r0, r1);
   }
+}
+
+// s[i] = lo[i] + hi[i] 2^32 for lo, hi < 2^62 (any u64): hi = h0 + h1 2^32
+// gives lo + h1 EPS + h0 2^32, one multiply-add, one addition into the high
+// word and its carry.
+template <int N> GL_FN void join_halves(uint64_t *s, const uint64_t *lo, const uint64_t *hi) {
+  uint32_t z1[N], h0[N], r[N], up[N];
+  uint64_t z[N];
+  row::Mask drop[N];
+  unroll<N>([&](auto k) {
+    constexpr int i = decltype(k)::value;
+    z[i] = (hi[i] >> 32) * EPS + lo[i];
+    z1[i] = hi32(z[i]);
+    h0[i] = lo32(hi[i]);
+  });
+  row::Rows<N>::add_bit(r, up, z1, h0);
+  unroll<N>([&](auto k) {
+    constexpr int i = decltype(k)::value;
+    z[i] = pair64(lo32(z[i]), r[i]);
+  });
+  row::Rows<N>::mad_eps(s, drop, up, z);
 }
 
 // x[i] *= w(i) for i in [FIRST, FIRST + COUNT), in rows of four and one

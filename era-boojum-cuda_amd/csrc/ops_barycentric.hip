@@ -24,6 +24,7 @@
 // in the field, so the order does not change the result).
 #include "../../include/boojum_ntt.h"
 #include "gl_ext.hpp"
+#include "gl_lazy.hpp"
 #include "ntt_device.hpp"
 
 #include <mutex>
@@ -39,35 +40,72 @@ namespace {
 constexpr uint32_t LC_NT = 256;  // threads per workgroup
 constexpr uint32_t LC_B = 4;     // coefficients per thread
 
-// Product in the base field (c1 unused) or in the extension.
-template <bool EXT> __device__ __forceinline__ gl::E2 pmul(gl::E2 a, gl::E2 b) {
-  if constexpr (EXT) return gl::e2_mul(a, b);
-  else return {gl::mul(a.c0, b.c0), 0};
+// N products side by side, in the base field (c1 unused) or in the extension:
+// any u64 components in and out.  The extension's four component products of
+// a pair are one row; a0 b0 + 7 a1 b1 and a0 b1 + a1 b0 are summed by 32-bit
+// halves and reduced once.
+template <bool EXT, int N>
+__device__ __forceinline__ void pmul(gl::E2 *r, const gl::E2 *a, const gl::E2 *b) {
+  if constexpr (!EXT) {
+    uint64_t x[N], y[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      x[i] = a[i].c0;
+      y[i] = b[i].c0;
+    }
+    gl::mul_row<N, gl::ANY>(x, x, y);
+#pragma unroll
+    for (int i = 0; i < N; ++i) r[i] = {x[i], 0};
+  } else {
+    gl::unroll<N>([&](auto k) {
+      constexpr int i = decltype(k)::value;
+      uint64_t x[4] = {a[i].c0, a[i].c1, a[i].c0, a[i].c1}, y[4] = {b[i].c0, b[i].c1, b[i].c1, b[i].c0};
+      gl::mul_row<4, gl::ANY>(x, x, y);
+      uint64_t lo[2], hi[2], o[2];
+      lo[0] = (uint64_t)gl::lo32(x[1]) * gl::E2_NON_RESIDUE + gl::lo32(x[0]);
+      hi[0] = (uint64_t)gl::hi32(x[1]) * gl::E2_NON_RESIDUE + gl::hi32(x[0]);
+      lo[1] = (uint64_t)gl::lo32(x[2]) + gl::lo32(x[3]);
+      hi[1] = (uint64_t)gl::hi32(x[2]) + gl::hi32(x[3]);
+      gl::join_halves<2>(o, lo, hi);
+      r[i] = {o[0], o[1]};
+    });
+  }
+}
+template <bool EXT> __device__ __forceinline__ gl::E2 pmul1(gl::E2 a, gl::E2 b) {
+  gl::E2 r;
+  pmul<EXT, 1>(&r, &a, &b);
+  return r;
 }
 
 // Thread t of workgroup b owns outputs i = 1024 b + 256 j + t (j < 4; stores
 // coalesced for each j) with denominators d = x omega_N^-idx - coset (idx = i,
 // or brev(i) when the output is bit-reversed); padding outputs (i >= N) use
 // d = 1.  All 1024 denominators of the workgroup share ONE field inversion
-// through a product tree in LDS: each thread multiplies its four (keeping
-// prefix products); the 256 thread products are paired up over 8 levels
-// (the left operand of every pairing stays in its thread's registers); thread
-// 0 inverts the total and multiplies in the common factor; going back down,
-// a node's inverse I gives its children I * right and I * left.  Each thread
-// ends with common / (its own product) and peels off its four coefficients
-// with its prefix products.  The common factor is
+// through a product tree: each thread multiplies its four (keeping prefix
+// products); wave 0 takes the 256 thread products, four to a lane, and
+// multiplies them up a binary tree of 63 nodes kept in LDS, inverts the root,
+// multiplies in the common factor and goes back down: a child's inverse is
+// its parent's times its sibling's product.  Each thread ends with common /
+// (its own product) and peels off its four coefficients with its prefix
+// products.  The common factor is
 //   coset (x^N - coset^N) / (N coset^N) = (x^N - coset^N) f,
 // with coset^N and f = coset / (N coset^N) from the host (they depend on
-// coset and N only); wave 0 squares x log N times while the power-table reads
-// are in flight, and workgroup 0 stores the common factor for the caller, as
-// the reference's first kernel does.
+// coset and N only); wave 1 squares x log N times while wave 0 climbs the tree
+// and inverts, and workgroup 0 stores the common factor for the caller, as the
+// reference's first kernel does.
+//
+// Bound: the serial chain (8 tree products, an inversion of 72 products, 8
+// products down), at one instruction per 8 cycles of a wave.  With a workgroup
+// barrier per level, two products a node on the way down, the squarings ahead
+// of the tree and products one at a time an extension call took 26 us at 2^10
+// and 42 us at 2^20.
 template <bool EXT>
 __global__ __launch_bounds__(LC_NT) void bary_coeffs_kernel(Tables tab, const uint64_t *x, uint64_t *common_out,
                                                             uint64_t coset, uint64_t coset_n, uint64_t f,
                                                             uint64_t *coeffs, uint32_t log_count, bool bit_reverse) {
-  constexpr uint32_t LEVELS = 8;  // log2(LC_NT)
-  __shared__ uint64_t node[2][LC_NT];  // subtree products (c0, c1)
-  __shared__ uint64_t down[2][LC_NT];  // inverses handed to right children
+  __shared__ gl::E2 leaf[LC_NT];  // thread products, then their inverses times the common factor
+  __shared__ gl::E2 tree[128];    // node i's children are 2 i and 2 i + 1; lane l of wave 0 is node 64 + l
+  __shared__ gl::E2 common;
   const uint32_t t = threadIdx.x;
   const uint64_t count = 1ull << log_count;
   const gl::E2 xv{gl::canon(x[0]), EXT ? gl::canon(x[1]) : 0ull};
@@ -81,81 +119,102 @@ __global__ __launch_bounds__(LC_NT) void bary_coeffs_kernel(Tables tab, const ui
                                      : (uint32_t)i;
     w[j] = i < count ? pow_w(tab, 0u - (log_count ? idx << (32 - log_count) : 0u)) : 0ull;  // omega_N^-idx
   }
-  // Wave 0 forms the common factor while the table reads are in flight (the
-  // squaring chain is serial; the other waves skip it).
-  gl::E2 cf{0, 0};
-  if (t < 64) {
-    gl::E2 xn = xv;
-    for (uint32_t i = 0; i < log_count; ++i) xn = pmul<EXT>(xn, xn);
-    cf = {gl::mul(gl::sub(xn.c0, coset_n), f), EXT ? gl::mul(xn.c1, f) : 0ull};
-    if (blockIdx.x == 0 && t == 0) {
-      common_out[0] = cf.c0;
-      if constexpr (EXT) common_out[1] = cf.c1;
-    }
-  }
   gl::E2 d[LC_B], pre[LC_B];
-  gl::E2 v{1, 0};
+  {
+    uint64_t p0[LC_B], p1[LC_B], xs0[LC_B], xs1[LC_B];
 #pragma unroll
-  for (uint32_t j = 0; j < LC_B; ++j) {
-    const uint64_t i = base + (uint64_t)j * LC_NT;
-    gl::E2 dj{1, 0};
-    if (i < count) {
-      dj.c0 = gl::sub(gl::mul(xv.c0, w[j]), coset);
-      if constexpr (EXT) dj.c1 = gl::mul(xv.c1, w[j]);
+    for (uint32_t j = 0; j < LC_B; ++j) {
+      xs0[j] = xv.c0;
+      xs1[j] = xv.c1;
     }
-    d[j] = dj;
-    pre[j] = v;
-    v = pmul<EXT>(v, dj);
+    gl::mul_row<LC_B, gl::CANON>(p0, w, xs0);
+    if constexpr (EXT) gl::mul_row<LC_B, gl::CANON>(p1, w, xs1);
+#pragma unroll
+    for (uint32_t j = 0; j < LC_B; ++j) {
+      const bool in = base + (uint64_t)j * LC_NT < count;
+      d[j] = {in ? gl::sub(p0[j], coset) : 1ull, EXT && in ? p1[j] : 0ull};
+    }
   }
-
-  // Up: at level l, thread t (a multiple of 2^(l+1)) joins [t, t + 2^l) and
-  // [t + 2^l, t + 2^(l+1)).
-  gl::E2 left[LEVELS];
-  node[0][t] = v.c0;
-  node[1][t] = v.c1;
+  pre[0] = {1, 0};
+  pre[1] = d[0];
+#pragma unroll
+  for (uint32_t j = 2; j < LC_B; ++j) pre[j] = pmul1<EXT>(pre[j - 1], d[j - 1]);
+  leaf[t] = pmul1<EXT>(pre[LC_B - 1], d[LC_B - 1]);
   __syncthreads();
-#pragma unroll
-  for (uint32_t l = 0; l < LEVELS; ++l) {
-    const uint32_t s = 1u << l;
-    if ((t & (2 * s - 1)) == 0) {
-      left[l] = v;
-      v = pmul<EXT>(v, gl::E2{node[0][t + s], node[1][t + s]});
-      node[0][t] = v.c0;
-      node[1][t] = v.c1;
-    }
-    __syncthreads();
-  }
-  // Root: I = common / total.
-  gl::E2 inv_node{0, 0};
-  if (t == 0) {
-    gl::E2 ti;
-    if constexpr (EXT) ti = gl::e2_inv(v);
-    else ti = {gl::inv(v.c0), 0};
-    inv_node = pmul<EXT>(ti, cf);
-  }
-  // Down: the parent's inverse times the sibling's product.
-#pragma unroll
-  for (uint32_t l = LEVELS; l-- > 0;) {
-    const uint32_t s = 1u << l;
-    if ((t & (2 * s - 1)) == 0) {
-      const gl::E2 r = pmul<EXT>(inv_node, left[l]);
-      down[0][t + s] = r.c0;
-      down[1][t + s] = r.c1;
-      inv_node = pmul<EXT>(inv_node, gl::E2{node[0][t + s], node[1][t + s]});
-    }
-    __syncthreads();
-    if ((t & (2 * s - 1)) == s) inv_node = gl::E2{down[0][t], down[1][t]};
-  }
 
-  // inv_node = common / (d_0 d_1 d_2 d_3) of this thread.
+  auto wave_sync = [] {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
+  gl::E2 q[4], pairs[2], root_inv{0, 0};
+  if (t < 64) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) q[k] = leaf[4 * t + k];
+    const gl::E2 l[2] = {q[0], q[2]}, r[2] = {q[1], q[3]};
+    pmul<EXT, 2>(pairs, l, r);
+    gl::E2 v = pmul1<EXT>(pairs[0], pairs[1]);
+    tree[64 + t] = v;
+    for (uint32_t n = 32; n; n >>= 1) {
+      wave_sync();
+      if (t < n) {
+        v = pmul1<EXT>(tree[2 * (n + t)], tree[2 * (n + t) + 1]);
+        tree[n + t] = v;
+      }
+    }
+    if (t == 0) {
+      v = {gl::canon(v.c0), gl::canon(v.c1)};
+      if constexpr (EXT) root_inv = gl::e2_inv(v);
+      else root_inv = {gl::inv(v.c0), 0};
+    }
+  } else if (t < 128) {
+    gl::E2 xn = xv;
+    for (uint32_t i = 0; i < log_count; ++i) xn = pmul1<EXT>(xn, xn);
+    if (t == 64) {
+      common = {gl::mul(gl::sub(gl::canon(xn.c0), coset_n), f), EXT ? gl::mul(xn.c1, f) : 0ull};
+      if (blockIdx.x == 0) {
+        common_out[0] = common.c0;
+        if constexpr (EXT) common_out[1] = common.c1;
+      }
+    }
+  }
+  __syncthreads();
+  if (t < 64) {
+    if (t == 0) tree[1] = pmul1<EXT>(root_inv, common);
+    for (uint32_t n = 2; n <= 64; n <<= 1) {
+      wave_sync();
+      // child n + t takes its parent's inverse times its sibling's product;
+      // every child has read its sibling before the products are replaced
+      gl::E2 v{0, 0};
+      if (t < n) v = pmul1<EXT>(tree[(n + t) >> 1], tree[(n + t) ^ 1]);
+      wave_sync();
+      if (t < n) tree[n + t] = v;
+    }
+    const gl::E2 self = tree[64 + t];
+    const gl::E2 halves_in[2] = {self, self}, other[2] = {pairs[1], pairs[0]};
+    gl::E2 halves[2];
+    pmul<EXT, 2>(halves, halves_in, other);
+    const gl::E2 in[4] = {halves[0], halves[0], halves[1], halves[1]}, sib[4] = {q[1], q[0], q[3], q[2]};
+    gl::E2 out[4];
+    pmul<EXT, 4>(out, in, sib);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) leaf[4 * t + k] = out[k];
+  }
+  __syncthreads();
+
+  // common / (d_0 d_1 d_2 d_3) of this thread
+  gl::E2 rest = leaf[t];
 #pragma unroll
   for (uint32_t j = LC_B; j-- > 0;) {
     const uint64_t i = base + (uint64_t)j * LC_NT;
-    const gl::E2 l = pmul<EXT>(inv_node, pre[j]);
-    inv_node = pmul<EXT>(inv_node, d[j]);
+    const gl::E2 a[2] = {rest, rest}, b[2] = {pre[j], d[j]};
+    gl::E2 o[2];
+    if (j) pmul<EXT, 2>(o, a, b);
+    else o[0] = rest;
+    rest = o[1];
     if (i < count) {
-      coeffs[i] = l.c0;
-      if constexpr (EXT) coeffs[count + i] = l.c1;
+      coeffs[i] = gl::canon(o[0].c0);
+      if constexpr (EXT) coeffs[count + i] = gl::canon(o[0].c1);
     }
   }
 }

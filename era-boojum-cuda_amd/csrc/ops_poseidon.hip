@@ -160,27 +160,6 @@ __device__ __forceinline__ uint32_t opaque(uint32_t v) {
   return v;
 }
 
-// s[i] = lo[i] + hi[i] 2^32 for lo, hi < 2^62 (any u64): hi = h0 + h1 2^32
-// gives lo + h1 EPS + h0 2^32, one multiply-add, one addition into the high
-// word and its carry.
-template <int N> __device__ __forceinline__ void join_halves(uint64_t *s, const uint64_t *lo, const uint64_t *hi) {
-  uint32_t z1[N], h0[N], r[N], up[N];
-  uint64_t z[N];
-  gl::row::Mask drop[N];
-  gl::unroll<N>([&](auto k) {
-    constexpr int i = decltype(k)::value;
-    z[i] = (hi[i] >> 32) * gl::EPS + lo[i];
-    z1[i] = gl::hi32(z[i]);
-    h0[i] = gl::lo32(hi[i]);
-  });
-  gl::row::Rows<N>::add_bit(r, up, z1, h0);
-  gl::unroll<N>([&](auto k) {
-    constexpr int i = decltype(k)::value;
-    z[i] = gl::pair64(gl::lo32(z[i]), r[i]);
-  });
-  gl::row::Rows<N>::mad_eps(s, drop, up, z);
-}
-
 // MDS rows R0..R0+N-1: y_r = sum_i 2^e_i x_((r + i) mod 12) + k_r with the two
 // 32-bit halves of the words summed apart (12 terms below 2^48, one
 // multiply-add each): 24 multiply-adds and 4 instructions a row.
@@ -203,7 +182,7 @@ __device__ __forceinline__ void mds_rows(uint64_t *y, const uint64_t (&s)[PT], c
         hi[r] += (uint64_t)gl::hi32(v) * c[i];
       }
     }
-    join_halves<4>(y + G, lo, hi);
+    gl::join_halves<4>(y + G, lo, hi);
   });
 }
 
@@ -251,7 +230,7 @@ struct Dot {
 __device__ __forceinline__ uint64_t dot_value(const Dot &d, uint32_t c24, uint32_t c16) {
   uint64_t lo, hi, r;
   d.halves(lo, hi, c24, c16);
-  join_halves<1>(&r, &lo, &hi);
+  gl::join_halves<1>(&r, &lo, &hi);
   return r;
 }
 
@@ -367,7 +346,7 @@ __device__ __forceinline__ void m_ext(uint64_t (&s)[PT], const uint64_t (*k)[2])
   }
   gl::unroll<3>([&](auto g) {
     constexpr int G = 4 * decltype(g)::value;
-    join_halves<4>(s + G, h[0] + G, h[1] + G);
+    gl::join_halves<4>(s + G, h[0] + G, h[1] + G);
   });
 }
 
@@ -393,7 +372,7 @@ __device__ __forceinline__ void m_int(uint64_t (&s)[PT], const uint64_t *k0, con
   }
   gl::unroll<3>([&](auto g) {
     constexpr int G = 4 * decltype(g)::value;
-    join_halves<4>(s + G, h[0] + G, h[1] + G);
+    gl::join_halves<4>(s + G, h[0] + G, h[1] + G);
   });
 }
 
@@ -569,7 +548,7 @@ __device__ __forceinline__ uint64_t coop_sbox(uint64_t x) {
 // lo + hi 2^32 (both below 2^62), any u64.
 __device__ __forceinline__ uint64_t coop_join(uint64_t lo, uint64_t hi) {
   uint64_t r;
-  join_halves<1>(&r, &lo, &hi);
+  gl::join_halves<1>(&r, &lo, &hi);
   return r;
 }
 
