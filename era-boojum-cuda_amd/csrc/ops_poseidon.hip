@@ -28,16 +28,16 @@
 // through M^-1: element 0 lands after the previous round's S-box, elements
 // 1..11 pass that S-box untouched.
 //
-// One thread hashes one leaf or node: the permutation is a serial chain of
-// field products with no data shared between hashes, and 12 state words fit
-// in 128 registers, four waves per SIMD.  Bound: VALU issue (86% busy, at a
-// clock the load holds to 2.05 GHz): about 15.9k VALU instructions per
-// Poseidon permutation, 38% of them S-box products and 28% multiply-adds of
-// the partial rounds' dot products, and 11.9k per Poseidon2 permutation,
-// against 64 bytes absorbed.  With every word reduced to [0, p) in every step,
-// products one at a time and sparse partial rounds it was 24.8k and 16.4k;
-// 128 columns x 2^20 rows: 10.8 -> 8.9 ms a Poseidon tree, 2^18 leaves of
-// 2 x 93 values: 3.30 -> 2.32 ms a Poseidon2 tree.
+// One lane hashes one leaf or node: the permutation is a serial chain of field
+// products with no data shared between hashes, and 12 state words fit in 128
+// registers, four waves per SIMD.  A wave's 64 states take Poseidon's matrix
+// products to the matrix cores together (MatMul).  Bound: vector issue slots:
+// about 10.3k vector instructions per Poseidon permutation, 60% of them S-box
+// products, and 11.9k (cheaper ones) per Poseidon2 permutation, against 64
+// bytes absorbed.  With every word reduced to [0, p) in every step, products
+// one at a time and sparse partial rounds it was 24.8k and 16.4k; 128 columns
+// x 2^20 rows: 10.7 -> 5.5 ms a Poseidon tree, 2^18 leaves of 2 x 93 values:
+// 3.30 -> 1.97 ms a Poseidon2 tree.
 #include "../../include/boojum_ntt.h"
 #include "gl_lazy.hpp"
 
@@ -73,42 +73,37 @@ __device__ PosTable pos_table;
 
 // Constants of the one-lane-per-state permutations (permute, permute2).
 //
-// A constant factor b of a dot product is kept as three limbs, b = c0 +
-// c1 2^24 + c2 2^48 (c0, c1 < 2^24, c2 < 2^16), so that products with a
-// 32-bit half of a state word can be summed in 64 bits without carries.
+// Matrix products of Poseidon run on the matrix cores (MatMul below): a matrix's
+// operand bytes are in pos_mat, the constant terms of its rows here, as two
+// 64-bit halves that also hold the bias MAT_BIAS.
+//
+// A factor b of a dot product formed on the vector unit is kept as three
+// limbs, b = c0 + c1 2^24 + c2 2^48 (c0, c1 < 2^24, c2 < 2^16), so that
+// products with a 32-bit half of a state word can be summed in 64 bits without
+// carries.
 constexpr int LIMBS = 3;
 constexpr int BLOCK = 11, BLOCKS = PARTIAL / BLOCK;  // partial rounds are run in blocks of 11
 // 2^DOT_BIAS_LOG is added to the low accumulator of every dot product (see
-// Dot::value) and taken out of its constant.
+// Dot::value) and taken out of a constant.
 constexpr int DOT_BIAS_LOG = 54;
+constexpr int MAT_BIAS_LOG = 46;
 
-struct DotConst {
-  uint32_t k[2];  // constant term, low and high half, less the bias
-};
 // Partial rounds in blocks.  With z_j the S-box output of round j of a block
 // and s_1..s_11 the other words at the block's start, the words at round r
 // are s_i + sum_{j<r} w_j,i z_j, so element 0 after round r is
 //   z_r + vs_r . s + sum_{j<r} (vs_r . w_j) z_j + constant,
-// and the words 1..11 are only formed at the block's end, with one reduction
-// per word instead of one per word and round.
+// and the words 1..11 are only formed at the block's end.  The vs_r . s of all
+// rounds are one 11 x 11 matrix product at the block's start, the words at its
+// end another; only the sums over z are serial.
 struct PosBlock {
-  struct {
-    DotConst k;
-    uint32_t s[PT - 1][LIMBS];
-    uint32_t z[BLOCK][LIMBS];  // j < r used
-  } round[BLOCK];
-  struct {
-    DotConst k;
-    uint32_t z[BLOCK][LIMBS];
-  } update[PT - 1];
+  uint64_t start[PT][2];             // constants of the rounds' element 0 (the last row unused)
+  uint32_t z[BLOCK][BLOCK][LIMBS];   // [r][j], j < r used
+  uint64_t end[PT][2];               // constants of words 1..11 (the last row unused)
 };
 struct PosFast {
-  uint64_t first[PT];        // constants of round 0
-  uint64_t after[7][PT][2];  // added behind each MDS, halves in 64 bits: rounds 1-3, then 27-29 and none
-  struct {
-    DotConst k;
-    uint32_t c[PT][LIMBS];
-  } dense[PT];
+  uint64_t first[PT];       // constants of round 0
+  uint64_t mds[7][PT][2];   // behind each MDS: rounds 1-3, then 27-29 and none
+  uint64_t dense[PT][2];
   PosBlock block[BLOCKS];
   // Poseidon2: behind the first external matrix and behind each full round's
   // (the constants of the round that follows; element 0 alone before a
@@ -119,6 +114,20 @@ struct PosFast {
   uint64_t p2_last[PT][2];
 };
 
+// The matrices on the matrix cores.  A constant c multiplies a word by its
+// bytes x_b: c x = sum_b (c 2^8b mod p) x_b, and each c 2^8b mod p is written
+// as eight signed bytes d_l (balanced digits, of the residue or the residue
+// less p), so that row limb l of an output is an integer sum over words and
+// bytes of d_l x_b.  The operand is signed, so x_b - 128 goes in, and 128
+// times the digits' sum into the row's constant.  12 words of 8 bytes are
+// three steps of 32, four outputs of 8 limbs a tile of 32 rows.
+enum { MAT_MDS = 0, MAT_DENSE = 1, MAT_BLOCK = 2, MATS = MAT_BLOCK + 2 * BLOCKS };
+constexpr int MAT_TILES = 3, MAT_STEPS = 3;
+struct PosMat {
+  int8_t a[MATS][MAT_TILES][MAT_STEPS][64][16];  // operand bytes of each lane
+};
+
+__device__ __align__(16) PosMat pos_mat;
 __device__ PosFast pos_fast;
 
 // The table, through an address the optimizer cannot see through: a kernel
@@ -133,13 +142,6 @@ __device__ __forceinline__ const PosFast &table() {
   Const *p = (Const *)&pos_fast;
   asm volatile("" : "+s"(p));
   return *(const PosFast *)p;
-}
-
-__device__ __forceinline__ uint64_t sbox(uint64_t x) {
-  const uint64_t x2 = gl::mul(x, x);
-  const uint64_t x3 = gl::mul(x2, x);
-  const uint64_t x4 = gl::mul(x2, x2);
-  return gl::mul(x3, x4);
 }
 
 // x^7 of N words, any u64 in and out.
@@ -164,46 +166,104 @@ __device__ __forceinline__ uint32_t opaque(uint32_t v) {
   return v;
 }
 
-// MDS rows R0..R0+N-1: y_r = sum_i 2^e_i x_((r + i) mod 12) + k_r with the two
-// 32-bit halves of the words summed apart (12 terms below 2^48, one
-// multiply-add each): 24 multiply-adds and 4 instructions a row.
-template <int R0, int N>
-__device__ __forceinline__ void mds_rows(uint64_t *y, const uint64_t (&s)[PT], const uint64_t (*k)[2]) {
-  uint32_t c[PT];
+// Matrix products of the states of a whole wave (every lane of the wave runs
+// this, also those without a state of their own).  Lane h's state is column
+// h % 32 of one of two 32-column tiles, and a tile's operand wants the first
+// two words of a step in lanes 0..31 and the next two in lanes 32..63, for the
+// same 32 states: v_permlane32_swap turns two words of all 64 states into
+// that for both tiles.  Of the result a lane holds, for its column, limbs 0..3
+// of the four outputs (lanes 0..31) or limbs 4..7 (lanes 32..63); two limbs are
+// put together (they are below 2^21), the same swap brings the sums of every
+// state to its own lane, and the halves are formed with the row's constant
+// (which holds a bias that keeps them positive) and reduced once.
+//
+// The permutation is bound by vector issue slots, and matrix instructions run
+// beside those of other waves: an output costs 15 slots here, 28 as an MDS row
+// on the vector unit and 82 as a dense row of 11 words.  Poseidon, tree of 2^20
+// leaves of 128 words: 6.9 -> 5.5 ms (10.3k vector instructions a permutation
+// instead of 15.9k).  Tiles are kept apart for the scheduler: interleaved they
+// took 66 registers more than the 128 that four waves a SIMD leave.
+struct MatMul {
+  using V4 = int __attribute__((ext_vector_type(4)));
+  using V16 = int __attribute__((ext_vector_type(16)));
+  static constexpr uint32_t SIGNS = 0x80808080u;
+  V4 x[MAT_STEPS][2];
+  __device__ __forceinline__ explicit MatMul(const uint64_t (&w)[PT]) {
 #pragma unroll
-  for (int i = 0; i < PT; ++i) c[i] = opaque(1u << MDS_EXPS[i]);
-  gl::unroll<N / 4>([&](auto g) {
-    constexpr int G = 4 * decltype(g)::value;
-    uint64_t lo[4], hi[4];
+    for (int st = 0; st < MAT_STEPS; ++st)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      lo[r] = k[R0 + G + r][0];
-      hi[r] = k[R0 + G + r][1];
+      for (int d = 0; d < 4; ++d) {
+        const uint64_t a = w[4 * st + d / 2], b = w[4 * st + 2 + d / 2];
+        const auto r = __builtin_amdgcn_permlane32_swap((d % 2 ? gl::hi32(a) : gl::lo32(a)) ^ SIGNS,
+                                                        (d % 2 ? gl::hi32(b) : gl::lo32(b)) ^ SIGNS, false, false);
+        x[st][0][d] = (int)r[0];
+        x[st][1][d] = (int)r[1];
+      }
+  }
+  // The words of step st again (the swap is its own inverse).
+  __device__ __forceinline__ void words(uint64_t *w, int st) const {
+    uint32_t h[2][4];
 #pragma unroll
-      for (int i = 0; i < PT; ++i) {
-        const uint64_t v = s[(R0 + G + r + i) % PT];
-        lo[r] += (uint64_t)gl::lo32(v) * c[i];
-        hi[r] += (uint64_t)gl::hi32(v) * c[i];
+    for (int d = 0; d < 4; ++d) {
+      const auto r = __builtin_amdgcn_permlane32_swap((uint32_t)x[st][0][d], (uint32_t)x[st][1][d], false, false);
+      h[0][d] = r[0] ^ SIGNS;
+      h[1][d] = r[1] ^ SIGNS;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) w[i] = gl::pair64(h[i / 2][2 * (i % 2)], h[i / 2][2 * (i % 2) + 1]);
+  }
+  // y[q] = output 4 tile + q, + add[q]
+  template <bool ADD = false>
+  __device__ __forceinline__ void tile(uint64_t *y, int mat, int tile, const uint64_t (*k)[2],
+                                       const uint64_t *add = nullptr) const {
+    const V4 *a = (const V4 *)&pos_mat.a[mat][tile][0][threadIdx.x % 64][0];
+    V16 acc[2] = {};
+#pragma unroll
+    for (int st = 0; st < MAT_STEPS; ++st) {
+      const V4 op = a[st * 64];
+      acc[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(op, x[st][0], acc[0], 0, 0, 0);
+      acc[1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(op, x[st][1], acc[1], 0, 0, 0);
+    }
+    // vector registers, so that the row constant may be the scalar operand
+    int32_t one = 1, c16 = 1 << 16;
+    asm("" : "+v"(one), "+v"(c16));
+    uint64_t h[2][4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      // two limbs at a time, before the swap: |l| < 2^21
+      int32_t l[2][2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const auto r = __builtin_amdgcn_permlane32_swap(
+            (uint32_t)acc[0][4 * q + 2 * i] + ((uint32_t)acc[0][4 * q + 2 * i + 1] << 8),
+            (uint32_t)acc[1][4 * q + 2 * i] + ((uint32_t)acc[1][4 * q + 2 * i + 1] << 8), false, false);
+        l[0][i] = (int32_t)r[0];
+        l[1][i] = (int32_t)r[1];
+      }
+#pragma unroll
+      for (int w = 0; w < 2; ++w) {
+        int64_t v = (int64_t)l[w][1] * c16 + (int64_t)k[4 * tile + q][w];
+        v += (int64_t)l[w][0] * one;
+        if constexpr (ADD) v += (uint64_t)(w ? gl::hi32(add[q]) : gl::lo32(add[q])) * (uint32_t)one;
+        h[w][q] = (uint64_t)v;
       }
     }
-    gl::join_halves<4>(y + G, lo, hi);
-  });
-}
-
-__device__ __forceinline__ void mds(uint64_t (&s)[PT], const uint64_t (*k)[2]) {
-  uint64_t y[PT];
-  mds_rows<0, PT>(y, s, k);
+    gl::join_halves<4>(y, h[0], h[1]);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  __device__ __forceinline__ void all(uint64_t *y, int mat, const uint64_t (*k)[2]) const {
 #pragma unroll
-  for (int i = 0; i < PT; ++i) s[i] = y[i];
-}
+    for (int t = 0; t < MAT_TILES; ++t) tile(y + 4 * t, mat, t, k);
+  }
+};
 
 // A dot product of state words with table constants: six 64-bit sums, one
 // multiply-add per word half and limb.  At most 22 terms, so the sums stay
 // below 2^61 (limbs of 24 bits) and 2^53 (16 bits).
 struct Dot {
   uint64_t p0, p1 = 0, p2 = 0, q0, q1 = 0, q2 = 0;
-  __device__ __forceinline__ explicit Dot(const DotConst &k)
-      : p0(gl::pair64(k.k[0], 1u << (DOT_BIAS_LOG - 32))), q0(k.k[1]) {}
+  __device__ __forceinline__ explicit Dot(uint64_t start)  // the sum's first term, less the bias
+      : p0(gl::pair64(gl::lo32(start), 1u << (DOT_BIAS_LOG - 32))), q0(gl::hi32(start)) {}
   __device__ __forceinline__ void mac(uint64_t a, const uint32_t *c) {
     const uint64_t a0 = gl::lo32(a), a1 = gl::hi32(a);
     p0 += a0 * c[0];
@@ -252,60 +312,54 @@ __device__ __forceinline__ void permute(uint64_t (&s)[PT], bool capacity_out) {
 #pragma unroll 1
   for (int r = 0; r < HALF_FULL - 1; ++r) {
     sbox_all(s);
-    mds(s, t.after[r]);
+    MatMul(s).all(s, MAT_MDS, t.mds[r]);
   }
   sbox_all(s);
+  MatMul(s).all(s, MAT_DENSE, t.dense);
   const uint32_t c24 = opaque(1u << 24), c16 = opaque(1u << 16), one = opaque(1u);
-  {
-    uint64_t v[PT];
-#pragma unroll
-    for (int i = 0; i < PT; ++i) v[i] = s[i];
-#pragma unroll
-    for (int r = 0; r < PT; ++r) {
-      Dot d(t.dense[r].k);
-#pragma unroll
-      for (int c = 0; c < PT; ++c) d.mac(v[c], t.dense[r].c[c]);
-      s[r] = dot_value(d, c24, c16);
-    }
-  }
 #pragma unroll 1
   for (int b = 0; b < BLOCKS; ++b) {
     const PosBlock &blk = t.block[b];
-    uint64_t z[BLOCK];
+    uint64_t first[4], z[PT], w[PT];
+#pragma unroll
+    for (int i = 1; i < PT; ++i) w[i - 1] = s[i];
+    w[PT - 1] = 0;
+    const MatMul start(w);
 #pragma unroll
     for (int r = 0; r < BLOCK; ++r) {
+      if (r % 4 == 0) start.tile(first, MAT_BLOCK + 2 * b, r / 4, blk.start);
       z[r] = s[0];
       sbox_row<1>(z + r);
-      Dot d(blk.round[r].k);
+      Dot d(first[r % 4]);
 #pragma unroll
-      for (int i = 1; i < PT; ++i) d.mac(s[i], blk.round[r].s[i - 1]);
-#pragma unroll
-      for (int j = 0; j < r; ++j) d.mac(z[j], blk.round[r].z[j]);
+      for (int j = 0; j < r; ++j) d.mac(z[j], blk.z[r][j]);
       d.add(z[r], one);
       s[0] = dot_value(d, c24, c16);
     }
+    z[PT - 1] = 0;
+    const MatMul end(z);
 #pragma unroll
-    for (int i = 1; i < PT; ++i) {
-      Dot d(blk.update[i - 1].k);
-#pragma unroll
-      for (int j = 0; j < BLOCK; ++j) d.mac(z[j], blk.update[i - 1].z[j]);
-      d.add(s[i], one);
-      s[i] = dot_value(d, c24, c16);
+    for (int tl = 0; tl < MAT_TILES; ++tl) {
+      start.words(w + 4 * tl, tl);
+      end.tile<true>(w + 4 * tl, MAT_BLOCK + 2 * b + 1, tl, blk.end, w + 4 * tl);
     }
+#pragma unroll
+    for (int i = 1; i < PT; ++i) s[i] = w[i - 1];
   }
 #pragma unroll 1
   for (int r = 0; r < 3; ++r) {
     sbox_all(s);
-    mds(s, t.after[3 + r]);
+    MatMul(s).all(s, MAT_MDS, t.mds[3 + r]);
   }
   sbox_all(s);
   uint64_t y[CAP];
+  const MatMul m(s);
   if (capacity_out) {
-    mds_rows<RATE, CAP>(y, s, t.after[6]);
+    m.tile(y, MAT_MDS, RATE / CAP, t.mds[6]);
 #pragma unroll
     for (int i = 0; i < CAP; ++i) s[RATE + i] = y[i];
   } else {
-    mds_rows<0, CAP>(y, s, t.after[6]);
+    m.tile(y, MAT_MDS, 0, t.mds[6]);
 #pragma unroll
     for (int i = 0; i < CAP; ++i) s[i] = y[i];
   }
@@ -416,8 +470,10 @@ __global__ __launch_bounds__(256, 4) void poseidon_leaves_kernel(const uint64_t 
                                                               uint64_t *__restrict__ results, uint32_t rows,
                                                               uint32_t cols, uint32_t count, bool load_intermediate,
                                                               bool store_intermediate) {
-  const uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
-  if (g >= count) return;
+  // a wave's lanes all take part in its matrix products, so lanes past the end
+  // hash the last leaf again and store nothing
+  const uint32_t lane_leaf = blockIdx.x * blockDim.x + threadIdx.x;
+  const uint32_t g = lane_leaf < count ? lane_leaf : count - 1;
   uint64_t s[PT];
 #pragma unroll
   for (int i = 0; i < PT; ++i) s[i] = 0;
@@ -441,6 +497,7 @@ __global__ __launch_bounds__(256, 4) void poseidon_leaves_kernel(const uint64_t 
     // the next chunk overwrites the rate, so only the capacity is read on
     permute_h<H>(s, store_intermediate || off + RATE < total);
   }
+  if (lane_leaf >= count) return;
 #pragma unroll
   for (int i = 0; i < CAP; ++i)
     results[g + (uint64_t)i * count] = gl::canon(store_intermediate ? s[RATE + i] : s[i]);
@@ -450,10 +507,10 @@ __global__ __launch_bounds__(256, 4) void poseidon_leaves_kernel(const uint64_t 
 // layer below (4 columns of 2 count digests): state[i] = left[i],
 // state[4 + i] = right[i], capacity zero.
 template <int H>
-__global__ __launch_bounds__(256) void poseidon_nodes_kernel(const uint64_t *__restrict__ values,
+__global__ __launch_bounds__(256, 4) void poseidon_nodes_kernel(const uint64_t *__restrict__ values,
                                                              uint64_t *__restrict__ results, uint32_t count) {
-  const uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
-  if (g >= count) return;
+  const uint32_t lane_node = blockIdx.x * blockDim.x + threadIdx.x;
+  const uint32_t g = lane_node < count ? lane_node : count - 1;
   uint64_t s[PT];
 #pragma unroll
   for (int i = 0; i < CAP; ++i) {
@@ -463,6 +520,7 @@ __global__ __launch_bounds__(256) void poseidon_nodes_kernel(const uint64_t *__r
     s[RATE + i] = 0;
   }
   permute_h<H>(s, false);
+  if (lane_node >= count) return;
 #pragma unroll
   for (int i = 0; i < CAP; ++i) results[g + (uint64_t)i * count] = gl::canon(s[i]);
 }
@@ -920,11 +978,6 @@ void set_limbs(uint32_t *out, uint64_t c) {
   out[1] = (uint32_t)((c >> 24) & 0xFFFFFF);
   out[2] = (uint32_t)(c >> 48);
 }
-void set_const(DotConst &out, uint64_t c) {
-  const uint64_t v = gl::sub(c, 1ull << DOT_BIAS_LOG);
-  out.k[0] = (uint32_t)v;
-  out.k[1] = (uint32_t)(v >> 32);
-}
 void set_halves(uint64_t (*out)[2], const uint64_t *c, int n = PT) {
   for (int i = 0; i < n; ++i) {
     out[i][0] = (uint32_t)c[i];
@@ -932,45 +985,84 @@ void set_halves(uint64_t (*out)[2], const uint64_t *c, int n = PT) {
   }
 }
 
-// The one-lane forms' table from the fused one.
-void derive_fast(const PosTable &t, PosFast &f) {
+// Eight signed bytes d_l with sum d_l 2^8l = c mod p.  The balanced digits of
+// a residue up to 0x7F7F...7F end without a carry; of a larger one they carry
+// out 2^64, and the residue less p (whose digits those of c + 2^64 - p are)
+// takes its place.
+void signed_bytes(int8_t *d, uint64_t c) {
+  uint64_t v = c > 0x7F7F7F7F7F7F7F7Full ? c + gl::EPS : c;  // c - p mod 2^64
+  for (int l = 0; l < 8; ++l) {
+    d[l] = (int8_t)(uint8_t)v;
+    v = (v >> 8) + (d[l] < 0 ? 1 : 0);
+  }
+}
+
+// Operand bytes and row constants of the matrix rows[o][w] (o < 12, w < 12)
+// plus constants k[o] (see PosMat).
+void set_mat(PosMat &m, int mat, uint64_t (*kout)[2], int outputs, const uint64_t (*rows)[PT], const uint64_t *k) {
+  for (int o = 0; o < outputs; ++o) {
+    uint64_t kv = k[o];
+    for (int w = 0; w < PT; ++w) {
+      uint64_t c = rows[o][w];
+      kv = gl::add(kv, gl::mul(c, 0x8080808080808080ull));
+      for (int b = 0; b < 8; ++b) {
+        int8_t d[8];
+        signed_bytes(d, c);
+        // the word's byte is byte `at` of lanes 32 half + row in its step
+        const int st = w / 4, half = (w % 4) / 2, at = 8 * (w % 2) + b;
+        for (int l = 0; l < 8; ++l) m.a[mat][o / 4][st][32 * half + 8 * (o % 4) + l][at] = d[l];
+        c = gl::mul(c, 256);
+      }
+    }
+    const uint64_t bias = 1ull << MAT_BIAS_LOG;
+    kv = gl::sub(kv, gl::mul(bias, 1 + (1ull << 32)));
+    kout[o][0] = bias + (uint32_t)kv;
+    kout[o][1] = bias + (kv >> 32);
+  }
+}
+
+// The one-lane forms' tables from the fused one.
+void derive_fast(const PosTable &t, PosFast &f, PosMat &m) {
+  uint64_t rows[PT][PT], k[PT];
   for (int i = 0; i < PT; ++i) f.first[i] = t.rc_full[0][i];
-  for (int r = 0; r < 3; ++r) {
-    set_halves(f.after[r], t.rc_full[1 + r]);
-    set_halves(f.after[3 + r], t.rc_full[HALF_FULL + r]);
+  for (int r = 0; r < PT; ++r)
+    for (int c = 0; c < PT; ++c) rows[r][c] = mds_entry(r, c);
+  for (int i = 0; i < 7; ++i) {
+    for (int r = 0; r < PT; ++r) k[r] = i < 3 ? t.rc_full[1 + i][r] : (i < 6 ? t.rc_full[HALF_FULL + i - 3][r] : 0);
+    set_mat(m, MAT_MDS, f.mds[i], PT, rows, k);
   }
   // dense (v + rcf): the fused constant layer becomes each row's constant
   for (int r = 0; r < PT; ++r) {
-    uint64_t k = 0;
-    for (int c = 0; c < PT; ++c) {
-      set_limbs(f.dense[r].c[c], t.dense[r][c]);
-      k = gl::add(k, gl::mul(t.dense[r][c], t.rcf[c]));
-    }
-    set_const(f.dense[r].k, k);
+    k[r] = 0;
+    for (int c = 0; c < PT; ++c) k[r] = gl::add(k[r], gl::mul(t.dense[r][c], t.rcf[c]));
   }
+  set_mat(m, MAT_DENSE, f.dense, PT, t.dense, k);
   // z_j below is the S-box output without its constant sbox_c
   for (int b = 0; b < BLOCKS; ++b) {
     PosBlock &blk = f.block[b];
     const int k0 = b * BLOCK;
+    memset(rows, 0, sizeof rows);
     for (int r = 0; r < BLOCK; ++r) {
-      uint64_t k = t.sbox_c[k0 + r];
-      for (int i = 0; i < PT - 1; ++i) set_limbs(blk.round[r].s[i], t.vs[k0 + r][i]);
+      // the bias of the round's sum over z comes out of its first term
+      k[r] = gl::sub(t.sbox_c[k0 + r], 1ull << DOT_BIAS_LOG);
+      for (int i = 0; i < PT - 1; ++i) rows[r][i] = t.vs[k0 + r][i];
       for (int j = 0; j < r; ++j) {
         uint64_t c = 0;
         for (int i = 0; i < PT - 1; ++i) c = gl::add(c, gl::mul(t.vs[k0 + r][i], t.w_hats[k0 + j][i]));
-        set_limbs(blk.round[r].z[j], c);
-        k = gl::add(k, gl::mul(c, t.sbox_c[k0 + j]));
+        set_limbs(blk.z[r][j], c);
+        k[r] = gl::add(k[r], gl::mul(c, t.sbox_c[k0 + j]));
       }
-      set_const(blk.round[r].k, k);
     }
+    set_mat(m, MAT_BLOCK + 2 * b, blk.start, BLOCK, rows, k);
+    memset(rows, 0, sizeof rows);
     for (int i = 0; i < PT - 1; ++i) {
-      uint64_t k = 0;
+      k[i] = 0;
       for (int j = 0; j < BLOCK; ++j) {
-        set_limbs(blk.update[i].z[j], t.w_hats[k0 + j][i]);
-        k = gl::add(k, gl::mul(t.w_hats[k0 + j][i], t.sbox_c[k0 + j]));
+        rows[i][j] = t.w_hats[k0 + j][i];
+        k[i] = gl::add(k[i], gl::mul(t.w_hats[k0 + j][i], t.sbox_c[k0 + j]));
       }
-      set_const(blk.update[i].k, k);
     }
+    set_mat(m, MAT_BLOCK + 2 * b + 1, blk.end, PT - 1, rows, k);
   }
   for (int r = 0; r < HALF_FULL; ++r) set_halves(f.p2_ext[r], t.p2_full[r]);
   set_halves(f.p2_ext[HALF_FULL], t.p2_partial, 1);
@@ -1125,7 +1217,8 @@ extern "C" int bc_poseidon_set_round_constants(const uint64_t *round_constants) 
   PosTable t{};
   if (!derive(round_constants, t)) return BC_ERROR_INVALID_VALUE;
   PosFast f{};
-  derive_fast(t, f);
+  std::vector<PosMat> m(1);
+  derive_fast(t, f, m[0]);
   std::unique_lock<std::shared_mutex> lk(pos_mu);
   // hashing kernels already queued on any stream of this device read the
   // table: let them finish before it changes (no new ones can be queued
@@ -1135,6 +1228,8 @@ extern "C" int bc_poseidon_set_round_constants(const uint64_t *round_constants) 
   err = hipMemcpyToSymbol(HIP_SYMBOL(pos_table), &t, sizeof t, 0, hipMemcpyHostToDevice);
   if (err != hipSuccess) return err;
   err = hipMemcpyToSymbol(HIP_SYMBOL(pos_fast), &f, sizeof f, 0, hipMemcpyHostToDevice);
+  if (err != hipSuccess) return err;
+  err = hipMemcpyToSymbol(HIP_SYMBOL(pos_mat), &m[0], sizeof m[0], 0, hipMemcpyHostToDevice);
   if (err != hipSuccess) return err;
   err = hipDeviceSynchronize();
   if (err != hipSuccess) return err;
