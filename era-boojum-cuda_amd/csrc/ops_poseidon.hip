@@ -527,19 +527,19 @@ __global__ __launch_bounds__(256, 4) void poseidon_nodes_kernel(const uint64_t *
 
 // ---- cooperative hashing: one state over 16 lanes ------------------------------
 // A small layer is one dependent permutation chain per lane, whatever its
-// size: 12-16k instructions at one per 8 cycles, the rate of a wave alone on
+// size: 10-12k instructions at one per 8 cycles, the rate of a wave alone on
 // its SIMD.  Here lane j of a 16-lane row owns state element j (lanes 12-15
 // hold values nobody reads), so a lane runs one S-box and one matrix row per
 // round.  Sums over the row are taken on 22-bit limbs with row rotations
 // (plain 32-bit additions, 12 instructions for the 16 lanes); the MDS row and
 // the 4-tiles gather their words through the wave's LDS, a round's constants
-// come from LDS.  Used for layers and leaf sets of at most coop_max<H>() (the
+// come from LDS.  Used for layers and leaf sets of at most COOP_MAX (the
 // reference likewise switches to cooperative kernels for small layers,
 // src/poseidon.rs:71,279-283).  Four permutations a leaf, 16 lanes against
-// one: Poseidon 129 / 256 us at 2^14, 209 / 259 at 2^15, 373 / 268 at 2^16;
-// Poseidon2 96 / 121 us at 2^14, 152 / 121 at 2^15.
+// one: Poseidon 71 / 119 us at 2^13, 117 / 118 at 2^14, 207 / 120 at 2^15;
+// Poseidon2 50 / 102 us at 2^13, 84 / 102 at 2^14, 151 / 103 at 2^15.
 constexpr uint32_t COOP_LANES = 16;
-template <int H> constexpr uint32_t coop_max() { return H == 0 ? 1u << 15 : 1u << 14; }
+constexpr uint32_t COOP_MAX = 1u << 14;
 constexpr uint32_t COOP_NT = 512, COOP_GROUPS = COOP_NT / COOP_LANES;  // two waves per SIMD issue side by side
 
 // A row's words in LDS, twice in a row so that word (j + i) mod 12 is at j + i.
@@ -1091,12 +1091,12 @@ int require_table() {
 using TableUse = std::shared_lock<std::shared_mutex>;
 
 // COOP: always the cooperative kernel; otherwise the cooperative kernel for
-// at most coop_max<H>() leaves and one thread per leaf above.
+// at most COOP_MAX leaves and one thread per leaf above.
 template <int H, bool COOP>
 int launch_leaves(const uint64_t *values, uint64_t *results, uint32_t log_rows, uint32_t cols, uint32_t count,
                   bool load, bool store, hipStream_t s) {
   if (count == 0) return BC_SUCCESS;
-  if (COOP || count <= coop_max<H>()) {
+  if (COOP || count <= COOP_MAX) {
     poseidon_leaves_coop_kernel<H><<<dim3((count + COOP_GROUPS - 1) / COOP_GROUPS), dim3(COOP_NT), 0, s>>>(
         values, results, log_rows, cols, count, load, store);
   } else {
@@ -1109,13 +1109,13 @@ int launch_leaves(const uint64_t *values, uint64_t *results, uint32_t log_rows, 
 // Node layers [values -> results], the first of `count` nodes (layers > 1: a
 // power of two).  COOP: always the cooperative kernel (the reference's
 // launch_cooperative_nodes_kernel); otherwise the cooperative kernel, several
-// layers to a launch, for layers of at most coop_max<H>() nodes, and one
+// layers to a launch, for layers of at most COOP_MAX nodes, and one
 // thread per node above.
 template <int H, bool COOP = false>
 int launch_nodes(const uint64_t *values, uint64_t *results, uint32_t count, uint32_t layers, hipStream_t s) {
   while (layers && count) {
     uint32_t n = 1;
-    if (COOP || count <= coop_max<H>()) {
+    if (COOP || count <= COOP_MAX) {
       n = layers < COOP_MAX_LAYERS ? layers : COOP_MAX_LAYERS;
       poseidon_nodes_coop_kernel<H>
           <<<dim3((count + COOP_GROUPS - 1) / COOP_GROUPS), dim3(COOP_NT), 0, s>>>(values, results, count, n);

@@ -1,5 +1,5 @@
 """GPU parity of the two hashing routes on either side of their switch: leaf
-sets and node layers of at most 2^14 (Poseidon2) or 2^15 (Poseidon) take 16
+sets and node layers of at most 2^14 take 16
 lanes a state (several node layers to a launch), larger ones one lane.
 Bit-exact against the oracle."""
 import numpy as np
