@@ -385,22 +385,35 @@ __device__ __forceinline__ void m4_tile(uint64_t *x) {
   x[3] = t4;
 }
 
-// The external matrix plus constants: the two 32-bit halves of the words go
-// through the additions apart (below 2^39) and each word is reduced once.
+// acc + a * c, kept from being put together with others of the same factor.
+__device__ __forceinline__ uint64_t mad_keep(uint32_t a, uint32_t c, uint64_t acc) {
+  uint64_t r = acc + (uint64_t)a * c;
+  asm("" : "+v"(r));
+  return r;
+}
+
+// The external matrix plus constants: M4 on each tile plus the sum of the
+// tiles.  The two 32-bit halves of the words go through the additions apart
+// (below 2^39) and each word is reduced once; halves are added to 64-bit sums
+// as products with 1, since as addends they would need a zeroed upper register
+// each.
 __device__ __forceinline__ void m_ext(uint64_t (&s)[PT], const uint64_t (*k)[2]) {
+  const uint32_t one = opaque(1u);
   uint64_t h[2][PT];
 #pragma unroll
   for (int w = 0; w < 2; ++w) {
 #pragma unroll
-    for (int i = 0; i < PT; ++i) h[w][i] = w ? gl::hi32(s[i]) : gl::lo32(s[i]);
+    for (int j = 0; j < 4; ++j) {
+      uint64_t sum = w ? gl::hi32(s[j]) : gl::lo32(s[j]);
+#pragma unroll
+      for (int g = 4; g < PT; g += 4) sum = mad_keep(w ? gl::hi32(s[g + j]) : gl::lo32(s[g + j]), one, sum);
+#pragma unroll
+      for (int g = 0; g < PT; g += 4) h[w][g + j] = mad_keep(w ? gl::hi32(s[g + j]) : gl::lo32(s[g + j]), one, sum);
+    }
 #pragma unroll
     for (int g = 0; g < PT; g += 4) m4_tile(h[w] + g);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const uint64_t sum = h[w][j] + h[w][4 + j] + h[w][8 + j];
-#pragma unroll
-      for (int g = 0; g < PT; g += 4) h[w][g + j] += sum + k[g + j][w];
-    }
+    for (int i = 0; i < PT; ++i) h[w][i] += k[i][w];
   }
   gl::unroll<3>([&](auto g) {
     constexpr int G = 4 * decltype(g)::value;
@@ -408,24 +421,63 @@ __device__ __forceinline__ void m_ext(uint64_t (&s)[PT], const uint64_t (*k)[2])
   });
 }
 
-// y_i = sum + 2^mu_i x_i, the halves apart, plus k0 on element 0 (and all of
-// `last`, if given).
-__device__ __forceinline__ void m_int(uint64_t (&s)[PT], const uint64_t *k0, const uint64_t (*last)[2]) {
-  const uint32_t one = opaque(1u);
-  uint64_t h[2][PT];
+// 1, 2^mu_i and 2^2mu_i in SGPRs, each of a value of its own to the optimizer
+// (products with the same factor would be put together behind a sum).
+struct P2Factors {
+  uint32_t one[PT], d[PT], dd[PT];
+  __device__ __forceinline__ P2Factors() {
+#pragma unroll
+    for (int i = 0; i < PT; ++i) {
+      one[i] = 1u;
+      d[i] = 1u << P2_MU[i];
+      dd[i] = 1u << (2 * P2_MU[i]);
+      asm volatile("" : "+s"(one[i]), "+s"(d[i]), "+s"(dd[i]));
+    }
+  }
+};
+
+// Two partial rounds but for the first one's S-box.  M_I x = sum(x) + D x with
+// D = diag(2^mu), so with S = sum(x), z the S-box of element 0 after the first
+// matrix, and T the sum of the other elements after it,
+//   u_0 = S + D_0 x_0 (+ k0),  T = 11 S + sum_{i>0} D_i x_i,
+//   y_0 = T + z + D_0 z (+ k1),  y_i = T + z + D_i S + D_i^2 x_i:
+// only element 0 is reduced between the two.  The halves go apart, below
+// 2^61.
+__device__ __forceinline__ void two_partial_rounds(uint64_t (&s)[PT], const P2Factors &f, const uint64_t *k0,
+                                                   const uint64_t *k1, const uint64_t (*last)[2]) {
+  uint64_t S[2], h[2][PT], u[2], z;
 #pragma unroll
   for (int w = 0; w < 2; ++w) {
-    uint64_t sum = w ? gl::hi32(s[0]) : gl::lo32(s[0]);
+    S[w] = w ? gl::hi32(s[0]) : gl::lo32(s[0]);
 #pragma unroll
-    for (int i = 1; i < PT; ++i) sum += (uint64_t)(w ? gl::hi32(s[i]) : gl::lo32(s[i])) * one;
+    for (int i = 1; i < PT; ++i) S[w] += (uint64_t)(w ? gl::hi32(s[i]) : gl::lo32(s[i])) * f.one[i];
+    u[w] = S[w] + k0[w] + (uint64_t)(w ? gl::hi32(s[0]) : gl::lo32(s[0])) * f.d[0];
+  }
+  gl::join_halves<1>(&z, u, u + 1);
+  sbox_row<1>(&z);
 #pragma unroll
-    for (int i = 0; i < PT; ++i)
-      h[w][i] = sum + (uint64_t)(w ? gl::hi32(s[i]) : gl::lo32(s[i])) * opaque(1u << P2_MU[i]);
+  for (int w = 0; w < 2; ++w) {
+    uint64_t t = (S[w] << 3) + S[w];
+    t = (S[w] << 1) + t;
+#pragma unroll
+    for (int i = 1; i < PT; ++i) t += (uint64_t)(w ? gl::hi32(s[i]) : gl::lo32(s[i])) * f.d[i];
+    const uint32_t zw = w ? gl::hi32(z) : gl::lo32(z);
+    t += (uint64_t)zw * f.one[0];
+    h[w][0] = t + (uint64_t)zw * f.d[0];
+    if (!last) h[w][0] += k1[w];
+    // S by 2^4, 2^8, 2^12: a product with D_i is a shift by up to 3 in the addition
+    uint64_t sh[4] = {S[w]};
+#pragma unroll
+    for (int g = 1; g < 4; ++g) {
+      sh[g] = sh[g - 1] << 4;
+      asm("" : "+v"(sh[g]));
+    }
+#pragma unroll
+    for (int i = 1; i < PT; ++i)
+      h[w][i] = (sh[P2_MU[i] / 4] << (P2_MU[i] % 4)) + t + (uint64_t)(w ? gl::hi32(s[i]) : gl::lo32(s[i])) * f.dd[i];
     if (last) {
 #pragma unroll
       for (int i = 0; i < PT; ++i) h[w][i] += last[i][w];
-    } else {
-      h[w][0] += k0[w];
     }
   }
   gl::unroll<3>([&](auto g) {
@@ -442,13 +494,14 @@ __device__ __forceinline__ void permute2(uint64_t (&s)[PT], bool) {
     sbox_all(s);
     m_ext(s, t.p2_ext[1 + r]);
   }
+  const P2Factors f;
 #pragma unroll 1
-  for (int k = 0; k < PARTIAL - 1; ++k) {
+  for (int k = 0; k < PARTIAL - 2; k += 2) {
     sbox_row<1>(s);
-    m_int(s, t.p2_int[k], nullptr);
+    two_partial_rounds(s, f, t.p2_int[k], t.p2_int[k + 1], nullptr);
   }
   sbox_row<1>(s);
-  m_int(s, nullptr, t.p2_last);
+  two_partial_rounds(s, f, t.p2_int[PARTIAL - 2], nullptr, t.p2_last);
 #pragma unroll 1
   for (int r = 0; r < HALF_FULL; ++r) {
     sbox_all(s);
@@ -456,7 +509,6 @@ __device__ __forceinline__ void permute2(uint64_t (&s)[PT], bool) {
   }
 }
 
-// Hash selector of the kernels: 0 Poseidon, 1 Poseidon2.
 template <int H> __device__ __forceinline__ void permute_h(uint64_t (&s)[PT], bool capacity_out) {
   if constexpr (H == 0) permute(s, capacity_out);
   else permute2(s, capacity_out);
