@@ -5,7 +5,7 @@ ABI.  Tensors are HIP torch tensors of int64/uint64.  Extension values
 matrix column of N elements as a double vector (N c0 values, then N c1)."""
 import ctypes
 
-from ._lib import BC_ERROR_INVALID_VALUE, HipError, lib
+from ._lib import BC_ERROR_INVALID_VALUE, HipError, current_stream_handle, lib
 
 # src/barycentric.rs:265-267
 EVAL_BASE_AT_BASE = 0
@@ -26,8 +26,7 @@ def _check(rc, what):
 
 
 def _stream(stream):
-    import torch
-    return (stream or torch.cuda.current_stream()).cuda_stream
+    return stream.cuda_stream if stream else current_stream_handle()
 
 
 def precompute_lagrange_coeffs(at_ext, x, common_factor_storage, coset, lagrange_coeffs, bit_reverse, stream=None):

@@ -9,7 +9,7 @@ panic; launch failures raise HipError (the reference's `CudaResult::Err`).
 """
 import ctypes
 
-from ._lib import BC_ERROR_INVALID_VALUE, BC_ERROR_NOT_INITIALIZED, HipError, lib
+from ._lib import BC_ERROR_INVALID_VALUE, BC_ERROR_NOT_INITIALIZED, HipError, current_stream_handle, lib
 
 
 def _slice(t):
@@ -24,10 +24,7 @@ def _slice(t):
 
 
 def _stream(t, stream):
-    import torch
-    if stream is None:
-        stream = torch.cuda.current_stream(t.device)
-    return stream.cuda_stream
+    return current_stream_handle(t.get_device()) if stream is None else stream.cuda_stream
 
 
 def _check(rc, what):

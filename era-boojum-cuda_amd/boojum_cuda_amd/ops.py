@@ -3,7 +3,7 @@ reference's `ops_complex` functions of the same names
 (src/ops_complex.rs:29-86, 207-330) over the C ABI.  Tensors are HIP torch
 tensors of int64/uint64; a slice's length is the element count, as a
 DeviceSlice's is in the reference."""
-from ._lib import BC_ERROR_INVALID_VALUE, HipError, lib
+from ._lib import BC_ERROR_INVALID_VALUE, HipError, current_stream_handle, lib
 
 
 def _check(rc, what):
@@ -15,8 +15,7 @@ def _check(rc, what):
 
 
 def _stream(stream):
-    import torch
-    return (stream or torch.cuda.current_stream()).cuda_stream
+    return stream.cuda_stream if stream else current_stream_handle()
 
 
 def bit_reverse(src, dst, rows, cols, src_stride=None, dst_stride=None, stream=None):

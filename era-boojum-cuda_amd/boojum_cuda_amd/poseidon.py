@@ -13,7 +13,7 @@ import ctypes
 
 import numpy as np
 
-from ._lib import BC_ERROR_INVALID_VALUE, BC_ERROR_NOT_INITIALIZED, HipError, lib
+from ._lib import BC_ERROR_INVALID_VALUE, BC_ERROR_NOT_INITIALIZED, HipError, current_stream_handle, lib
 
 RATE = 8
 CAPACITY = 4
@@ -36,8 +36,7 @@ def _check(rc, what):
 
 
 def _stream(stream):
-    import torch
-    return (stream or torch.cuda.current_stream()).cuda_stream
+    return stream.cuda_stream if stream else current_stream_handle()
 
 
 def _u64(a):

@@ -6,7 +6,7 @@ import ctypes
 from dataclasses import dataclass
 from typing import Optional
 
-from ._lib import BC_ERROR_INVALID_VALUE, HipError, lib
+from ._lib import BC_ERROR_INVALID_VALUE, HipError, current_stream_handle, lib
 
 OP_NTT, OP_INTT, OP_LDE = 0, 1, 2
 
@@ -70,8 +70,7 @@ class RaggedPlan:
         self._h = h
 
     def run(self, stream=None):
-        import torch
-        s = (stream or torch.cuda.current_stream()).cuda_stream
+        s = stream.cuda_stream if stream else current_stream_handle()
         _check(lib().bc_ragged_run(self._h, s), "ragged_run")
 
     def wait_status(self):
@@ -92,16 +91,14 @@ class RaggedPlan:
 
 def run_plain(jobs, stream=None):
     """The same jobs as separate launch sequences (the per-job path)."""
-    import torch
-    s = (stream or torch.cuda.current_stream()).cuda_stream
+    s = stream.cuda_stream if stream else current_stream_handle()
     _check(lib().bc_ragged_run_plain(_array(jobs), len(jobs), s), "ragged_run_plain")
 
 
 def run_no_alloc(jobs, stream=None):
     """Plans and runs the jobs with the plan in the library's static device
     array (no device allocation; results as RaggedPlan(jobs).run())."""
-    import torch
-    s = (stream or torch.cuda.current_stream()).cuda_stream
+    s = stream.cuda_stream if stream else current_stream_handle()
     _check(lib().bc_ragged_run_no_alloc(_array(jobs), len(jobs), s), "ragged_run_no_alloc")
 
 

@@ -4,7 +4,7 @@ run in continuous batches (see include/boojum_ntt.h).  Also the seeded input
 generator (bc_fill_seeded).  No reference counterpart."""
 import ctypes
 
-from ._lib import BC_ERROR_INVALID_VALUE, HipError, lib
+from ._lib import BC_ERROR_INVALID_VALUE, HipError, current_stream_handle, lib
 from .ragged import OP_INTT, OP_LDE, OP_NTT  # noqa: F401  (re-exported op codes)
 
 
@@ -56,8 +56,7 @@ def _check(rc, what):
 
 def fill_seeded(out, log_n, num_cols, stride, seed, first_col=0, stream=None):
     """Seeded raw u64 inputs on the device (the oracle's fill_raw stream)."""
-    import torch
-    s = (stream or torch.cuda.current_stream()).cuda_stream
+    s = stream.cuda_stream if stream else current_stream_handle()
     _check(lib().bc_fill_seeded(out.data_ptr(), log_n, num_cols, stride, seed, first_col, s), "fill_seeded")
 
 
