@@ -39,27 +39,6 @@ bc_context *current_context() {
 }
 
 
-// log_n < 8: one pass of the generic LDS kernel.
-int run_general(bc_context *ctx, const uint64_t *inputs, uint64_t *outputs, uint32_t log_n, uint32_t num_ntts,
-                uint32_t stride_in, uint32_t stride_out, bool bitrev_inputs, bool inverse, uint32_t log_ext,
-                uint32_t coset_exp, uint64_t n_inv, hipStream_t s) {
-  PassArgs a{};
-  a.tab = ctx->tab;
-  a.num_cols = num_ntts;
-  a.log_n = log_n;
-  a.log_ext = log_ext;
-  a.coset_exp = coset_exp;
-  a.n_inv = n_inv;
-  a.first = a.last = 1;
-  a.in = inputs;
-  a.stride_in = stride_in;
-  a.out = outputs;
-  a.stride_out = stride_out;
-  a.log_N = log_n;
-  a.log_H = log_n;
-  return launch_pass(a, inverse, bitrev_inputs, s);
-}
-
 // Fixes a strided pass's launch shape for `positions` r-ranges; false if it
 // cannot be launched.
 bool strided_shape(PassDesc &pd, uint64_t positions, uint32_t tuned_bpw, uint32_t *groups) {
@@ -179,9 +158,18 @@ extern "C" int bc_batch_ntt_internal(const uint64_t *inputs, uint64_t *outputs, 
 
   hipStream_t s = (hipStream_t)stream;
   if (log_n < 8) {
-    const uint32_t coset_exp = log_ext ? (uint32_t)((uint64_t)coset_index << (32 - log_n - log_ext)) : 0u;
-    return run_general(ctx, inputs, outputs, log_n, num_ntts, stride_in, stride_out, bitrev_inputs, inverse, log_ext,
-                       coset_exp, gl::inv(n % gl::P), s);
+    FastArgs a{};
+    a.tab = ctx->tab;
+    a.num_cols = num_ntts;
+    a.log_n = log_n;
+    a.log_ext = log_ext;
+    a.coset_exp = log_ext ? (uint32_t)((uint64_t)coset_index << (32 - log_n - log_ext)) : 0u;
+    a.n_inv = gl::inv(n % gl::P);
+    a.in = inputs;
+    a.stride_in = stride_in;
+    a.out = outputs;
+    a.stride_out = stride_out;
+    return launch_short(a, inverse, bitrev_inputs, s);
   }
 
   const TuneParams tp = tuned(log_n, num_ntts);

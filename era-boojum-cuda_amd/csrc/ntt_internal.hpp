@@ -40,24 +40,6 @@ constexpr uint32_t LVL_TW_MAX_LOG = 12;
 __host__ __device__ constexpr uint32_t lvl_tw_offset(uint32_t m) { return 15u * ((1u << (m - 4)) - 2u); }
 constexpr uint32_t LVL_TW_BLOCK = 15u * ((1u << (LVL_TW_MAX_LOG - 3)) - 2u);  // entries per direction
 
-// One HBM pass of a batched transform (see ntt_kernels.hip for the math).
-struct PassArgs {
-  const uint64_t *in;
-  uint64_t *out;
-  uint64_t stride_in;   // elements between consecutive input columns
-  uint64_t stride_out;  // elements between consecutive output columns
-  uint64_t n_inv;       // n^-1 mod p (last pass of an inverse transform)
-  Tables tab;
-  uint32_t num_cols;
-  uint32_t log_n;      // column length
-  uint32_t log_N;      // block length this pass works inside
-  uint32_t log_H;      // sub-transform length this pass computes
-  uint32_t first;      // pass reads the caller's input (coset pre-scaling)
-  uint32_t last;       // pass writes the final output (inverse post-scaling)
-  uint32_t log_ext;    // LDE: log2 blowup, 0 = plain transform
-  uint32_t coset_exp;  // coset_index << (32 - log_n - log_ext)
-};
-
 // Per-column base pointers of one pass (ragged job groups: the columns of
 // several jobs, each with its own buffers, processed as one batch).
 struct ColPtrs {
@@ -145,7 +127,6 @@ void tune_autoload();
 
 constexpr uint32_t TILE_LOG = 12;
 constexpr uint32_t TILE = 1u << TILE_LOG;
-constexpr uint32_t TILE_THREADS = 256;
 
 // Latency path (ntt_small.hip): 1..SMALL_MAX_COLS columns of 2^SMALL_LOG_N
 // points with no coset, as two launches of one-wave workgroups.
@@ -156,10 +137,8 @@ bool small_path_applies(uint32_t log_n, uint32_t num_cols, uint32_t log_ext, con
 hipError_t launch_small(const Tables &tab, const uint64_t *inputs, uint64_t *outputs, uint32_t num_cols,
                         uint64_t stride_in, uint64_t stride_out, bool bitrev_inputs, bool inverse, hipStream_t s);
 
-// Host: the split of log_n into per-pass sub-transform sizes, n2b order
-// (first entry = the pass that works on the top index bits).
-int plan_passes(uint32_t log_n, uint32_t *log_h, int max_passes);
-
-hipError_t launch_pass(const PassArgs &a, bool inverse, bool b2n, hipStream_t stream);
+// log_n 1..7 (ntt_small.hip): a.coset_exp, a.log_ext and a.n_inv as for the
+// fast passes.
+hipError_t launch_short(const FastArgs &a, bool inverse, bool bitrev_inputs, hipStream_t s);
 
 }  // namespace bc

@@ -1,9 +1,28 @@
 // Register-resident NTT pass bodies for gfx950 (device code shared by the
 // standalone pass kernels and the ragged persistent kernel).
 //
-// The math of a pass is the one described in ntt_kernels.hip: inside blocks of
-// N points, for every r < R = N / H, an H-point sub-DFT over j (positions
-// j * R + r), with the twist omega_N^(r * brev(j)).  Two tile shapes cover
+// Semantics (reference: src/ntt.rs:527-583 and native/ntt.cu:105-122):
+//   forward:  X_k = sum_i x_i s^i w^(ik)
+//   inverse:  y_i = n^-1 s^-i sum_k x_k w^(-ik)
+// with w = omega_n, s = g * omega_{n 2^ext}^coset when log_ext > 0 (else 1).
+// n2b: natural input, bit-reversed output; b2n: bit-reversed input, natural
+// output.
+//
+// Decomposition.  A transform of 2^L points is split into HBM passes
+// L = h_0 + h_1 + ... (plan_passes).  In n2b order pass p works inside blocks
+// of N = 2^(L - h_0 - ... - h_{p-1}) points.  Writing an index inside a block
+// as i = j * R + r (R = N / H, H = 2^h_p), the pass runs, for every r, an
+// H-point natural->bit-reversed DFT over j (root omega_H), then multiplies the
+// value at position j by the twist omega_N^(r * brev(j)).  The next pass then
+// works on blocks of R contiguous points.  This is the four-step recursion of
+// the DFT; the last pass has R = 1 and no twist.
+//
+// b2n is the transpose of n2b: the same diagonal twists and the same
+// symmetric sub-DFTs applied in the reverse order, so passes run last-first,
+// each pass applies its twist before its sub-DFT, and sub-DFTs use the
+// bit-reversed-input (decimation in time) form.
+//
+// Two tile shapes cover
 // every pass of a transform with log_n >= 8:
 //
 //   contig<h>  (8 <= h <= 12): R = 1, the last pass in n2b order.  A tile is

@@ -1,6 +1,7 @@
-// Latency path for a few columns of 2^16 points (the single-column case of the
-// reference's benches): two launches of one-wave workgroups, each wave holding
-// one 256-point sub-DFT at 4 values per lane.
+// Transforms of one wave, 4 values per lane: columns of 2..128 points
+// (ntt_short_kernel, below), and the latency path for a few columns of 2^16
+// points (the single-column case of the reference's benches) as two launches
+// of one-wave workgroups, each wave holding one 256-point sub-DFT.
 //
 // The pass kernels of ntt_fast.hip give each thread 16 values of a 4096-point
 // tile, so one 2^16 column is 16 workgroups per pass and the call takes one
@@ -215,7 +216,139 @@ template <bool INV, bool DIT> hipError_t launch_pair(const FastArgs &top, const 
   return hipGetLastError();
 }
 
+// Columns of 2^LN points, LN = 1..7: the lower LN bits of a wave's 256-point
+// transform, 2^(8-LN) columns to a wave.  Position p of the wave's 256 values
+// is point p mod 2^LN of its column p / 2^LN; at stage s register i of lane l
+// holds the position with register bits at B = 6 - 2s, and the stages above
+// the columns' length (and the exchanges behind them) fall away.  With odd LN
+// the first stage is radix 2 over its lower bit.
+//
+// A small call is bound by one wave's serial work behind the launch: 256
+// columns of 2^4 / 2^7 points took 8.7-14 / 12-17 us as 4096-point tiles of
+// 256 threads with 16 values each, 6.5-7 us here, about a call's time on the
+// host.  Large ones are bound by memory in pieces of columns: 2^26 values in
+// columns of 2^4 / 2^7 305-514 / 399-614 -> 262-344 / 327-490 us.
+constexpr uint32_t SHORT_WAVES = 4;  // waves a workgroup of many-column calls has
+template <int LN, bool INV, bool DIT>
+__global__ __launch_bounds__(SHORT_WAVES * SW) void ntt_short_kernel(FastArgs a) {
+  constexpr int S0 = 4 - (LN + 1) / 2;
+  __shared__ WaveLds sh_all[SHORT_WAVES];
+  const uint32_t l = threadIdx.x % SW;
+  WaveLds &sh = sh_all[threadIdx.x / SW];
+  const uint64_t col0 = ((uint64_t)blockIdx.x * (blockDim.x / SW) + threadIdx.x / SW) << (8 - LN);
+  auto pos = [&](int s, int i) -> uint32_t {
+    const int b = 6 - 2 * s;
+    return ((l >> b) << (b + 2)) | ((uint32_t)i << b) | (l & ((1u << b) - 1u));
+  };
+  // twist of register i behind (DIT: before) stage s
+  uint64_t tw[3][3];
+  static_for<3 - S0>([&](auto k) {
+    constexpr int S = S0 + decltype(k)::value, B = 6 - 2 * S;
+    constexpr bool ODD = S == S0 && LN % 2;
+    const uint32_t rp = l & ((1u << B) - 1u);
+    if constexpr (ODD) {
+      tw[S][0] = root(a.tab, B + 1, rp, INV);
+    } else {
+#pragma unroll
+      for (int i = 1; i < 4; ++i) tw[S][i - 1] = root(a.tab, B + 2, rp * brev2((uint32_t)i), INV);
+    }
+  });
+  auto twist = [&](auto s, uint64_t *x) {
+    constexpr int S = decltype(s)::value;
+    if constexpr (S == 3) return;
+    else if constexpr (S == S0 && LN % 2) {
+      x[1] = gl::mul(x[1], tw[S][0]);
+      x[3] = gl::mul(x[3], tw[S][0]);
+    } else {
+#pragma unroll
+      for (int i = 1; i < 4; ++i) x[i] = gl::mul(x[i], tw[S][i - 1]);
+    }
+  };
+  auto dft = [&](auto s, uint64_t *x) {
+    constexpr int A = decltype(s)::value == S0 && LN % 2 ? 1 : 2;
+#pragma unroll
+    for (int g = 0; g < 4; g += 1 << A) {
+      if constexpr (DIT) dft_dit<A, INV>(x + g);
+      else dft_dif<A, INV>(x + g);
+    }
+  };
+  auto exchange = [&](auto s, uint64_t *x) {  // between stages S and S + 1, either way
+    constexpr int S = decltype(s)::value;
+    if constexpr (S == 0) swap_lane45(x);
+    else if constexpr (S == 1) swap_lanes_lds<2>(x, sh.ex2, l);
+    else if constexpr (S == 2) swap_lanes_lds<0>(x, sh.ex3, l);
+  };
+  uint64_t x[4];
+  constexpr int FIRST = DIT ? 3 : S0, LAST = DIT ? S0 : 3;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint32_t p = pos(FIRST, i), j = p & ((1u << LN) - 1u);
+    const uint64_t c = col0 + (p >> LN);
+    x[i] = c < a.num_cols ? gl::canon(a.in[c * a.stride_in + j]) : 0ull;
+  }
+  if (!INV && a.log_ext) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint32_t j = pos(FIRST, i) & ((1u << LN) - 1u);
+      x[i] = gl::mul(x[i], coset_pow(a.tab, a.coset_exp, DIT ? brev_bits(j, LN) : j, false));
+    }
+  }
+  static_for<4 - S0>([&](auto k) {
+    constexpr int K = decltype(k)::value, S = DIT ? 3 - K : S0 + K;
+    constexpr std::integral_constant<int, S> s{};
+    if constexpr (DIT) {
+      if constexpr (K > 0) exchange(s, x);
+      twist(s, x);
+      dft(s, x);
+    } else {
+      dft(s, x);
+      twist(s, x);
+      if constexpr (S < 3) exchange(s, x);
+    }
+  });
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint32_t p = pos(LAST, i), j = p & ((1u << LN) - 1u);
+    const uint64_t c = col0 + (p >> LN);
+    if (c >= a.num_cols) continue;
+    uint64_t v = x[i];
+    if (INV) {
+      v = gl::mul(v, a.n_inv);
+      if (a.log_ext) v = gl::mul(v, coset_pow(a.tab, a.coset_exp, DIT ? j : brev_bits(j, LN), true));
+    }
+    a.out[c * a.stride_out + j] = gl::canon(v);
+  }
+}
+
+template <int LN> hipError_t launch_short_ln(const FastArgs &a, bool inverse, bool dit, hipStream_t s) {
+  // one-wave workgroups until the chip has four on every SIMD
+  const uint64_t waves = ((uint64_t)a.num_cols + (1u << (8 - LN)) - 1) >> (8 - LN);
+  const uint32_t per_wg = waves > 4096 ? SHORT_WAVES : 1;
+  const dim3 grid((uint32_t)((waves + per_wg - 1) / per_wg)), block(per_wg * SW);
+  if (inverse) {
+    if (dit) ntt_short_kernel<LN, true, true><<<grid, block, 0, s>>>(a);
+    else ntt_short_kernel<LN, true, false><<<grid, block, 0, s>>>(a);
+  } else {
+    if (dit) ntt_short_kernel<LN, false, true><<<grid, block, 0, s>>>(a);
+    else ntt_short_kernel<LN, false, false><<<grid, block, 0, s>>>(a);
+  }
+  return hipGetLastError();
+}
+
 }  // namespace
+
+hipError_t launch_short(const FastArgs &a, bool inverse, bool bitrev_inputs, hipStream_t s) {
+  switch (a.log_n) {
+  case 1: return launch_short_ln<1>(a, inverse, bitrev_inputs, s);
+  case 2: return launch_short_ln<2>(a, inverse, bitrev_inputs, s);
+  case 3: return launch_short_ln<3>(a, inverse, bitrev_inputs, s);
+  case 4: return launch_short_ln<4>(a, inverse, bitrev_inputs, s);
+  case 5: return launch_short_ln<5>(a, inverse, bitrev_inputs, s);
+  case 6: return launch_short_ln<6>(a, inverse, bitrev_inputs, s);
+  case 7: return launch_short_ln<7>(a, inverse, bitrev_inputs, s);
+  default: return hipErrorInvalidValue;
+  }
+}
 
 bool small_path_applies(uint32_t log_n, uint32_t num_cols, uint32_t log_ext, const TuneParams &tp) {
   if (log_n != SMALL_LOG_N || log_ext != 0 || num_cols < 1 || num_cols > 65535) return false;
