@@ -597,6 +597,9 @@ constexpr uint32_t COOP_NT = 512, COOP_GROUPS = COOP_NT / COOP_LANES;  // two wa
 // A row's words in LDS, twice in a row so that word (j + i) mod 12 is at j + i.
 struct CoopLds {
   PosTable t;
+  // constants behind Poseidon2's partial rounds, by halves: of element 0 in
+  // round k (k > 0), of element j behind the last at PARTIAL + j, then zeros
+  uint64_t p2_add[PARTIAL + PT + 1][2];
   uint64_t words[COOP_GROUPS][2 * PT];
 };
 
@@ -659,6 +662,118 @@ __device__ __forceinline__ uint64_t coop_sbox(uint64_t x) {
   return r;
 }
 
+// Poseidon2's partial round: the S-box of element 0 with the sum over the
+// other elements in its waits.  A mask written by a vector instruction may be
+// read two instructions later at the earliest (and a rotation reads a register
+// two instructions after its write), and a wave alone on its SIMD pays a full
+// issue slot for every s_nop that fills such a gap: 27 of 119 slots a round.
+// The sum does not depend on the S-box, so its instructions stand there.
+//
+// rest.lo + rest.hi 2^32 becomes (k_lo + k_hi 2^32) + mu x + the sum of x over
+// the lanes with keep set, the sum on limbs a, b, c of 22, 22 and 20 bits; its
+// b and c are left to be added.
+struct RestSum {
+  uint64_t lo, hi;
+  uint32_t b, c;
+};
+#define BC_ROR(v, n) "v_add_u32_dpp %[" #v "], %[" #v "], %[" #v "] row_ror:" #n " row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
+__device__ __forceinline__ uint64_t coop_sbox_rest(uint64_t x, uint32_t keep, uint32_t mu, uint64_t k_lo, uint64_t k_hi,
+                                                   RestSum &rest) {
+  const uint32_t x0 = gl::lo32(x), x1 = gl::hi32(x);
+  uint32_t a, b, c;
+  // products as mul_row: two halves' products, the middle one with its carry
+  auto top = [](uint64_t t, uint32_t u, uint32_t v) { return (uint64_t)u * v + gl::hi32(t); };
+  auto mid = [](uint32_t u0, uint32_t u1, uint32_t v0, uint32_t v1, uint64_t &p, uint64_t &carry) {
+    p = (uint64_t)u0 * v0;
+    uint64_t t = (uint64_t)u0 * v1 + gl::hi32(p);
+    asm("v_mad_u64_u32 %0, %1, %2, %3, %4" : "=v"(t), "=s"(carry) : "v"(u1), "v"(v0), "v"(t));
+    return t;
+  };
+  uint64_t p, q, t, v, m, n;
+  uint32_t e0, e1, r2, f, g0, g1;
+  // the square
+  t = mid(x0, x1, x0, x1, p, m);
+  q = top(t, x1, x1);
+  asm("s_nop 0\n"
+      "v_subb_co_u32_e64 %[e0], %[m], %[p0], %[q1], %[m]\n"
+      "v_and_b32 %[a], %[x0], %[keep]\n"
+      "v_alignbit_b32 %[b], %[x1], %[x0], 22\n"
+      "v_subb_co_u32_e64 %[e1], %[m], %[t0], 0, %[m]\n"
+      "v_lshrrev_b32 %[c], 12, %[x1]\n"
+      "v_and_b32 %[b], %[b], %[keep]\n"
+      "v_subb_co_u32_e64 %[r2], %[m], %[q0], 0, %[m]\n"
+      : [e0] "=&v"(e0), [e1] "=&v"(e1), [r2] "=&v"(r2), [a] "=&v"(a), [b] "=&v"(b), [c] "=&v"(c), [m] "+s"(m)
+      : [p0] "v"(gl::lo32(p)), [q1] "v"(gl::hi32(q)), [t0] "v"(gl::lo32(t)), [q0] "v"(gl::lo32(q)), [x0] "v"(x0),
+        [x1] "v"(x1), [keep] "v"(keep));
+  uint64_t w;  // masks nobody reads
+  asm("v_mad_u64_u32 %[v], %[n], %[r2], -1, %[e]\n"
+      "v_and_b32 %[c], %[c], %[keep]\n"
+      "v_mad_u64_u32 %[lo], %[w], %[x0], %[mu], %[k]\n"
+      "v_cndmask_b32_e64 %[f], 0, -1, %[n]\n"
+      : [v] "=&v"(v), [n] "=&s"(n), [w] "=&s"(w), [f] "=&v"(f), [c] "+v"(c), [lo] "=&v"(rest.lo)
+      : [r2] "v"(r2), [e] "v"(gl::pair64(e0, e1)), [keep] "v"(keep), [x0] "v"(x0), [mu] "v"(mu), [k] "v"(k_lo));
+  uint32_t s0, s1;
+  asm("v_addc_co_u32_e64 %[s0], %[m], %[v0], %[f], %[m]\n" BC_ROR(a, 8) BC_ROR(b, 8)
+      "v_addc_co_u32_e64 %[s1], %[m], %[v1], 0, %[m]\n"
+      : [s0] "=&v"(s0), [s1] "=&v"(s1), [m] "+s"(m), [a] "+v"(a), [b] "+v"(b)
+      : [v0] "v"(gl::lo32(v)), [v1] "v"(gl::hi32(v)), [f] "v"(f));
+  // the cube and the fourth power
+  uint64_t p2, q2, t2, v2, m2, n2;
+  uint32_t d0, d1, h2, f2;
+  t = mid(s0, s1, x0, x1, p, m);
+  t2 = mid(s0, s1, s0, s1, p2, m2);
+  q = top(t, s1, x1);
+  q2 = top(t2, s1, s1);
+  asm("v_subb_co_u32_e64 %[e0], %[m], %[p0], %[q1], %[m]\n"
+      "v_subb_co_u32_e64 %[d0], %[m2], %[p20], %[q21], %[m2]\n" BC_ROR(c, 8)
+      "v_subb_co_u32_e64 %[e1], %[m], %[t0], 0, %[m]\n"
+      "v_subb_co_u32_e64 %[d1], %[m2], %[t20], 0, %[m2]\n" BC_ROR(a, 4)
+      "v_subb_co_u32_e64 %[r2], %[m], %[q0], 0, %[m]\n"
+      "v_subb_co_u32_e64 %[h2], %[m2], %[q20], 0, %[m2]\n"
+      : [e0] "=&v"(e0), [e1] "=&v"(e1), [r2] "=&v"(r2), [d0] "=&v"(d0), [d1] "=&v"(d1), [h2] "=&v"(h2), [a] "+v"(a),
+        [c] "+v"(c), [m] "+s"(m), [m2] "+s"(m2)
+      : [p0] "v"(gl::lo32(p)), [q1] "v"(gl::hi32(q)), [t0] "v"(gl::lo32(t)), [q0] "v"(gl::lo32(q)),
+        [p20] "v"(gl::lo32(p2)), [q21] "v"(gl::hi32(q2)), [t20] "v"(gl::lo32(t2)), [q20] "v"(gl::lo32(q2)));
+  asm("v_mad_u64_u32 %[v], %[n], %[r2], -1, %[e]\n"
+      "v_mad_u64_u32 %[v2], %[n2], %[h2], -1, %[d]\n" BC_ROR(b, 4)
+      "v_cndmask_b32_e64 %[f], 0, -1, %[n]\n"
+      "v_cndmask_b32_e64 %[f2], 0, -1, %[n2]\n"
+      : [v] "=&v"(v), [n] "=&s"(n), [f] "=&v"(f), [v2] "=&v"(v2), [n2] "=&s"(n2), [f2] "=&v"(f2), [b] "+v"(b)
+      : [r2] "v"(r2), [e] "v"(gl::pair64(e0, e1)), [h2] "v"(h2), [d] "v"(gl::pair64(d0, d1)));
+  asm("v_addc_co_u32_e64 %[s0], %[m], %[v0], %[f], %[m]\n"
+      "v_addc_co_u32_e64 %[g0], %[m2], %[v20], %[f2], %[m2]\n" BC_ROR(c, 4)
+      "v_addc_co_u32_e64 %[s1], %[m], %[v1], 0, %[m]\n"
+      "v_addc_co_u32_e64 %[g1], %[m2], %[v21], 0, %[m2]\n"
+      : [s0] "=&v"(s0), [s1] "=&v"(s1), [g0] "=&v"(g0), [g1] "=&v"(g1), [m] "+s"(m), [m2] "+s"(m2), [c] "+v"(c)
+      : [v0] "v"(gl::lo32(v)), [v1] "v"(gl::hi32(v)), [f] "v"(f), [v20] "v"(gl::lo32(v2)), [v21] "v"(gl::hi32(v2)),
+        [f2] "v"(f2));
+  // their product
+  t = mid(s0, s1, g0, g1, p, m);
+  q = top(t, s1, g1);
+  asm("s_nop 0\n"
+      "v_subb_co_u32_e64 %[e0], %[m], %[p0], %[q1], %[m]\n" BC_ROR(a, 2) BC_ROR(b, 2)
+      "v_subb_co_u32_e64 %[e1], %[m], %[t0], 0, %[m]\n" BC_ROR(c, 2) BC_ROR(a, 1)
+      "v_subb_co_u32_e64 %[r2], %[m], %[q0], 0, %[m]\n"
+      : [e0] "=&v"(e0), [e1] "=&v"(e1), [r2] "=&v"(r2), [a] "+v"(a), [b] "+v"(b), [c] "+v"(c), [m] "+s"(m)
+      : [p0] "v"(gl::lo32(p)), [q1] "v"(gl::hi32(q)), [t0] "v"(gl::lo32(t)), [q0] "v"(gl::lo32(q)));
+  asm("v_mad_u64_u32 %[v], %[n], %[r2], -1, %[e]\n" BC_ROR(b, 1) BC_ROR(c, 1)
+      "v_cndmask_b32_e64 %[f], 0, -1, %[n]\n"
+      : [v] "=&v"(v), [n] "=&s"(n), [f] "=&v"(f), [b] "+v"(b), [c] "+v"(c)
+      : [r2] "v"(r2), [e] "v"(gl::pair64(e0, e1)));
+  // the last two wait for the rotations that read s0 and s1 next
+  asm("v_addc_co_u32_e64 %[s0], %[m], %[v0], %[f], %[m]\n"
+      "v_mad_u64_u32 %[lo], %[w], %[a], 1, %[lo]\n"
+      "v_mad_u64_u32 %[hi], %[w], %[x1], %[mu], %[k]\n"
+      "v_addc_co_u32_e64 %[s1], %[m], %[v1], 0, %[m]\n"
+      "s_nop 1\n"
+      : [s0] "=&v"(s0), [s1] "=&v"(s1), [m] "+s"(m), [w] "=&s"(w), [lo] "+v"(rest.lo), [hi] "=&v"(rest.hi)
+      : [v0] "v"(gl::lo32(v)), [v1] "v"(gl::hi32(v)), [f] "v"(f), [a] "v"(a), [x1] "v"(x1), [mu] "v"(mu), [k] "v"(k_hi));
+  rest.b = b;
+  rest.c = c;
+  return gl::pair64(s0, s1);
+}
+#undef BC_ROR
+
 // lo + hi 2^32 (both below 2^62), any u64.
 __device__ __forceinline__ uint64_t coop_join(uint64_t lo, uint64_t hi) {
   uint64_t r;
@@ -676,11 +791,12 @@ __device__ __forceinline__ uint64_t add_const(uint64_t a, uint64_t b) {
 // whose words are staged in w.
 struct Coop {
   const PosTable &t;
+  const uint64_t (&p2_add)[PARTIAL + PT + 1][2];
   uint64_t *w;      // the row's 2 PT words in LDS
   uint32_t j, jj;   // lane of the row; table row (lanes 12-15 reuse row 11)
   uint32_t keep;    // 22-bit mask, 0 in lanes 12-15
   __device__ __forceinline__ Coop(CoopLds &l, uint32_t lane, uint32_t group)
-      : t(l.t), w(l.words[group]), j(lane), jj(lane < PT ? lane : PT - 1), keep(lane < PT ? 0x3FFFFFu : 0u) {}
+      : t(l.t), p2_add(l.p2_add), w(l.words[group]), j(lane), jj(lane < PT ? lane : PT - 1), keep(lane < PT ? 0x3FFFFFu : 0u) {}
 
   __device__ __forceinline__ void stage(uint64_t x) const {
     coop_sync();  // the row's earlier reads come first
@@ -743,8 +859,8 @@ struct Coop {
   }
 
   // (J + I) (x) M4 on the three tiles: each word plus the sum over the tiles,
-  // then the 4 x 4 row, on limbs.
-  __device__ __forceinline__ uint64_t m_ext_row(uint64_t x, const uint32_t *m4row) const {
+  // then the 4 x 4 row, on limbs, plus the constant k.
+  __device__ __forceinline__ uint64_t m_ext_row(uint64_t x, const uint32_t *m4row, uint64_t k) const {
     Limbs l(x, keep), s = l;
     s.add_ror<8>();
     s.add_ror<4>();
@@ -757,7 +873,7 @@ struct Coop {
     l.a = row(l.a);
     l.b = row(l.b);
     l.c = row(l.c);
-    uint64_t lo = 0, hi = 0;
+    uint64_t lo = gl::lo32(k), hi = gl::hi32(k);
     l.add_to(lo, hi);
     return coop_join(lo, hi);
   }
@@ -770,27 +886,28 @@ struct Coop {
       const uint32_t q = j & 3u;
       m4row[c] = q == 0 ? M4[0][c] : (q == 1 ? M4[1][c] : (q == 2 ? M4[2][c] : M4[3][c]));
     }
-    uint32_t mu = 0;
+    uint32_t mu = 0;  // of the lane's own word in the rest sum: none for element 0
 #pragma unroll
-    for (int i = 0; i < PT; ++i) mu = jj == (uint32_t)i ? 1u << P2_MU[i] : mu;
-    x = m_ext_row(x, m4row);
+    for (int i = 1; i < PT; ++i) mu = jj == (uint32_t)i ? 1u << P2_MU[i] : mu;
+    const uint32_t keep_rest = j ? keep : 0u, z_factor = j ? 1u : 1u + (1u << P2_MU[0]);
+    // the constants of the next round ride on each matrix
+    x = m_ext_row(x, m4row, t.p2_full[0][jj]);
 #pragma unroll 1
-    for (int r = 0; r < HALF_FULL; ++r) x = m_ext_row(coop_sbox(add_const(x, t.p2_full[r][jj])), m4row);
+    for (int r = 1; r < HALF_FULL; ++r) x = m_ext_row(coop_sbox(x), m4row, t.p2_full[r][jj]);
+    x = m_ext_row(coop_sbox(x), m4row, j ? 0ull : t.p2_partial[0]);
 #pragma unroll 1
-    for (int k = 0; k < PARTIAL; ++k) {
-      const uint64_t s = coop_sbox(add_const(x, t.p2_partial[k]));
-      x = j ? x : s;
-      Limbs l(x, keep);
-      l.add_ror<8>();
-      l.add_ror<4>();
-      l.add_ror<2>();
-      l.add_ror<1>();
-      uint64_t lo = (uint64_t)gl::lo32(x) * mu, hi = (uint64_t)gl::hi32(x) * mu;
-      l.add_to(lo, hi);
-      x = coop_join(lo, hi);
+    for (int k = 1; k <= PARTIAL; ++k) {
+      // y_0 = rest + (1 + 2^mu_0) z, y_i = rest + mu_i x_i + z
+      const uint64_t *kp = p2_add[k == PARTIAL ? PARTIAL + jj : (j ? PARTIAL + PT : (uint32_t)k)];
+      RestSum rest;
+      const uint64_t z = row_first(coop_sbox_rest(x, keep_rest, mu, kp[0], kp[1], rest));
+      rest.lo += (uint64_t)rest.b * opaque(1u << 22) + (uint64_t)gl::lo32(z) * z_factor;
+      rest.hi += (uint64_t)rest.c * opaque(1u << 12) + (uint64_t)gl::hi32(z) * z_factor;
+      x = coop_join(rest.lo, rest.hi);
     }
 #pragma unroll 1
-    for (int r = 0; r < HALF_FULL; ++r) x = m_ext_row(coop_sbox(add_const(x, t.p2_full[HALF_FULL + r][jj])), m4row);
+    for (int r = 1; r < HALF_FULL; ++r) x = m_ext_row(coop_sbox(x), m4row, t.p2_full[HALF_FULL + r][jj]);
+    x = m_ext_row(coop_sbox(x), m4row, 0);
   }
 
   template <int H> __device__ __forceinline__ void permute_h(uint64_t &x) const {
@@ -803,6 +920,13 @@ __device__ __forceinline__ void coop_stage_table(CoopLds &l) {
   const uint64_t *src = (const uint64_t *)&pos_table;
   uint64_t *dst = (uint64_t *)&l.t;
   for (uint32_t i = threadIdx.x; i < sizeof(PosTable) / sizeof(uint64_t); i += blockDim.x) dst[i] = src[i];
+  if (threadIdx.x <= PARTIAL + PT) {
+    const uint32_t i = threadIdx.x;
+    const uint64_t k = i < PARTIAL ? pos_table.p2_partial[i]
+                                   : (i < PARTIAL + PT ? pos_table.p2_full[HALF_FULL][i - PARTIAL] : 0ull);
+    l.p2_add[i][0] = gl::lo32(k);
+    l.p2_add[i][1] = gl::hi32(k);
+  }
 }
 
 // `layers` consecutive node layers, the first of `count` nodes: a workgroup
