@@ -588,15 +588,24 @@ __global__ __launch_bounds__(256, 4) void poseidon_nodes_kernel(const uint64_t *
 // come from LDS.  Used for layers and leaf sets of at most COOP_MAX (the
 // reference likewise switches to cooperative kernels for small layers,
 // src/poseidon.rs:71,279-283).  Four permutations a leaf, 16 lanes against
-// one: Poseidon 71 / 119 us at 2^13, 117 / 118 at 2^14, 207 / 120 at 2^15;
-// Poseidon2 50 / 102 us at 2^13, 84 / 102 at 2^14, 151 / 103 at 2^15.
+// one: Poseidon 64 / 119 us at 2^13, 107 / 118 at 2^14, 193 / 121 at 2^15;
+// Poseidon2 49 / 91 us at 2^13, 86 / 91 at 2^14, 158 / 92 at 2^15.
 constexpr uint32_t COOP_LANES = 16;
 constexpr uint32_t COOP_MAX = 1u << 14;
 constexpr uint32_t COOP_NT = 512, COOP_GROUPS = COOP_NT / COOP_LANES;  // two waves per SIMD issue side by side
 
+// A lane's part of a Poseidon partial round: its row and column entries (0 and
+// 1 for element 0) and, by halves, what the S-box's constant c adds (c itself
+// for element 0, else w c).
+struct PartialLane {
+  uint64_t v, w, k[2];
+};
+__device__ PartialLane pos_partial_lanes[PARTIAL][PT];
+
 // A row's words in LDS, twice in a row so that word (j + i) mod 12 is at j + i.
 struct CoopLds {
   PosTable t;
+  PartialLane partial[PARTIAL][PT];
   // constants behind Poseidon2's partial rounds, by halves: of element 0 in
   // round k (k > 0), of element j behind the last at PARTIAL + j, then zeros
   uint64_t p2_add[PARTIAL + PT + 1][2];
@@ -639,18 +648,7 @@ struct Limbs {
   }
 };
 
-// x^7, the cube and the fourth power side by side; xv = x v beside the square.
-__device__ __forceinline__ uint64_t coop_sbox(uint64_t x, uint64_t v, uint64_t &xv) {
-  uint64_t a[2] = {x, x}, b[2] = {x, v}, s[2], c[2], r;
-  gl::mul_row<2, gl::ANY>(s, a, b);
-  xv = s[1];
-  a[0] = a[1] = s[0];
-  b[0] = x;
-  b[1] = s[0];
-  gl::mul_row<2, gl::ANY>(c, a, b);
-  gl::mul_row<1, gl::ANY>(&r, &c[0], &c[1]);
-  return r;
-}
+// x^7, the cube and the fourth power side by side.
 __device__ __forceinline__ uint64_t coop_sbox(uint64_t x) {
   uint64_t s, a[2], b[2], c[2], r;
   gl::mul_row<1, gl::ANY>(&s, &x, &x);
@@ -662,13 +660,29 @@ __device__ __forceinline__ uint64_t coop_sbox(uint64_t x) {
   return r;
 }
 
-// Poseidon2's partial round: the S-box of element 0 with the sum over the
-// other elements in its waits.  A mask written by a vector instruction may be
-// read two instructions later at the earliest (and a rotation reads a register
-// two instructions after its write), and a wave alone on its SIMD pays a full
-// issue slot for every s_nop that fills such a gap: 27 of 119 slots a round.
-// The sum does not depend on the S-box, so its instructions stand there.
-//
+// Partial rounds: the S-box of element 0 with the sum over the row in its
+// waits.  A mask written by a vector instruction may be read two instructions
+// later at the earliest (and a rotation reads a register two instructions
+// after its write), and a wave alone on its SIMD pays a full issue slot for
+// every s_nop that fills such a gap: 27 of 119 slots in a Poseidon2 round.
+// The sum does not depend on the S-box's end, so its instructions stand there
+// (104 slots; a Poseidon2 tree of 2^11 leaves, one permutation each, 122 -> 115
+// us; 128 with the same sum ahead of the S-box).  Poseidon: 168 -> 131 slots,
+// four permutations a leaf 63.9 -> 57.8 us at 2^10 leaves.
+#define BC_ROR(v, n) "v_add_u32_dpp %[" #v "], %[" #v "], %[" #v "] row_ror:" #n " row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
+// A product's 32-bit steps, as in mul_row: u v0 + ..., the middle sum with its
+// carry, and the top half.
+__device__ __forceinline__ uint64_t coop_mid(uint64_t u, uint64_t v, uint64_t &p, uint64_t &carry) {
+  p = (uint64_t)gl::lo32(u) * gl::lo32(v);
+  uint64_t t = (uint64_t)gl::lo32(u) * gl::hi32(v) + gl::hi32(p);
+  asm("v_mad_u64_u32 %0, %1, %2, %3, %4" : "=v"(t), "=s"(carry) : "v"(gl::hi32(u)), "v"(gl::lo32(v)), "v"(t));
+  return t;
+}
+__device__ __forceinline__ uint64_t coop_top(uint64_t t, uint64_t u, uint64_t v) {
+  return (uint64_t)gl::hi32(u) * gl::hi32(v) + gl::hi32(t);
+}
+
+// Poseidon2:
 // rest.lo + rest.hi 2^32 becomes (k_lo + k_hi 2^32) + mu x + the sum of x over
 // the lanes with keep set, the sum on limbs a, b, c of 22, 22 and 20 bits; its
 // b and c are left to be added.
@@ -676,24 +690,15 @@ struct RestSum {
   uint64_t lo, hi;
   uint32_t b, c;
 };
-#define BC_ROR(v, n) "v_add_u32_dpp %[" #v "], %[" #v "], %[" #v "] row_ror:" #n " row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
 __device__ __forceinline__ uint64_t coop_sbox_rest(uint64_t x, uint32_t keep, uint32_t mu, uint64_t k_lo, uint64_t k_hi,
                                                    RestSum &rest) {
   const uint32_t x0 = gl::lo32(x), x1 = gl::hi32(x);
   uint32_t a, b, c;
-  // products as mul_row: two halves' products, the middle one with its carry
-  auto top = [](uint64_t t, uint32_t u, uint32_t v) { return (uint64_t)u * v + gl::hi32(t); };
-  auto mid = [](uint32_t u0, uint32_t u1, uint32_t v0, uint32_t v1, uint64_t &p, uint64_t &carry) {
-    p = (uint64_t)u0 * v0;
-    uint64_t t = (uint64_t)u0 * v1 + gl::hi32(p);
-    asm("v_mad_u64_u32 %0, %1, %2, %3, %4" : "=v"(t), "=s"(carry) : "v"(u1), "v"(v0), "v"(t));
-    return t;
-  };
   uint64_t p, q, t, v, m, n;
   uint32_t e0, e1, r2, f, g0, g1;
   // the square
-  t = mid(x0, x1, x0, x1, p, m);
-  q = top(t, x1, x1);
+  t = coop_mid(x, x, p, m);
+  q = coop_top(t, x, x);
   asm("s_nop 0\n"
       "v_subb_co_u32_e64 %[e0], %[m], %[p0], %[q1], %[m]\n"
       "v_and_b32 %[a], %[x0], %[keep]\n"
@@ -720,10 +725,10 @@ __device__ __forceinline__ uint64_t coop_sbox_rest(uint64_t x, uint32_t keep, ui
   // the cube and the fourth power
   uint64_t p2, q2, t2, v2, m2, n2;
   uint32_t d0, d1, h2, f2;
-  t = mid(s0, s1, x0, x1, p, m);
-  t2 = mid(s0, s1, s0, s1, p2, m2);
-  q = top(t, s1, x1);
-  q2 = top(t2, s1, s1);
+  t = coop_mid(gl::pair64(s0, s1), x, p, m);
+  t2 = coop_mid(gl::pair64(s0, s1), gl::pair64(s0, s1), p2, m2);
+  q = coop_top(t, gl::pair64(s0, s1), x);
+  q2 = coop_top(t2, gl::pair64(s0, s1), gl::pair64(s0, s1));
   asm("v_subb_co_u32_e64 %[e0], %[m], %[p0], %[q1], %[m]\n"
       "v_subb_co_u32_e64 %[d0], %[m2], %[p20], %[q21], %[m2]\n" BC_ROR(c, 8)
       "v_subb_co_u32_e64 %[e1], %[m], %[t0], 0, %[m]\n"
@@ -748,8 +753,8 @@ __device__ __forceinline__ uint64_t coop_sbox_rest(uint64_t x, uint32_t keep, ui
       : [v0] "v"(gl::lo32(v)), [v1] "v"(gl::hi32(v)), [f] "v"(f), [v20] "v"(gl::lo32(v2)), [v21] "v"(gl::hi32(v2)),
         [f2] "v"(f2));
   // their product
-  t = mid(s0, s1, g0, g1, p, m);
-  q = top(t, s1, g1);
+  t = coop_mid(gl::pair64(s0, s1), gl::pair64(g0, g1), p, m);
+  q = coop_top(t, gl::pair64(s0, s1), gl::pair64(g0, g1));
   asm("s_nop 0\n"
       "v_subb_co_u32_e64 %[e0], %[m], %[p0], %[q1], %[m]\n" BC_ROR(a, 2) BC_ROR(b, 2)
       "v_subb_co_u32_e64 %[e1], %[m], %[t0], 0, %[m]\n" BC_ROR(c, 2) BC_ROR(a, 1)
@@ -772,7 +777,143 @@ __device__ __forceinline__ uint64_t coop_sbox_rest(uint64_t x, uint32_t keep, ui
   rest.c = c;
   return gl::pair64(s0, s1);
 }
+
+// Poseidon: the S-box of element 0, and the sum of v x over the lanes with keep
+// set as limbs a, b, c (whose last rotations are left).  acc.lo + acc.hi 2^32
+// becomes (k_lo + k_hi 2^32) + f x (f: 0 or 1).
+struct TermSum {
+  uint64_t lo, hi;
+  uint32_t a, b, c;
+};
+__device__ __forceinline__ uint64_t coop_sbox_terms(uint64_t x, uint64_t vx, uint32_t keep, uint32_t fx, uint64_t k_lo,
+                                                    uint64_t k_hi, TermSum &acc) {
+  const uint32_t x0 = gl::lo32(x), x1 = gl::hi32(x);
+  uint64_t p, q, t, v, m, n, p2, q2, t2, v2, m2, n2, w;  // w: masks nobody reads
+  uint32_t e0, e1, r2, f, s0, s1, d0, d1, h2, f2, g0, g1, a, b, c;
+  // the square and the term
+  t = coop_mid(x, x, p, m);
+  t2 = coop_mid(vx, x, p2, m2);
+  q = coop_top(t, x, x);
+  q2 = coop_top(t2, vx, x);
+  asm("v_subb_co_u32_e64 %[e0], %[m], %[p0], %[q1], %[m]\n"
+      "v_subb_co_u32_e64 %[d0], %[m2], %[p20], %[q21], %[m2]\n"
+      "v_mad_u64_u32 %[lo], %[w], %[x0], %[fx], %[kl]\n"
+      "v_subb_co_u32_e64 %[e1], %[m], %[t0], 0, %[m]\n"
+      "v_subb_co_u32_e64 %[d1], %[m2], %[t20], 0, %[m2]\n"
+      "v_mad_u64_u32 %[hi], %[w], %[x1], %[fx], %[kh]\n"
+      "v_subb_co_u32_e64 %[r2], %[m], %[q0], 0, %[m]\n"
+      "v_subb_co_u32_e64 %[h2], %[m2], %[q20], 0, %[m2]\n"
+      : [e0] "=&v"(e0), [e1] "=&v"(e1), [r2] "=&v"(r2), [d0] "=&v"(d0), [d1] "=&v"(d1), [h2] "=&v"(h2),
+        [lo] "=&v"(acc.lo), [hi] "=&v"(acc.hi), [m] "+s"(m), [m2] "+s"(m2), [w] "=&s"(w)
+      : [p0] "v"(gl::lo32(p)), [q1] "v"(gl::hi32(q)), [t0] "v"(gl::lo32(t)), [q0] "v"(gl::lo32(q)),
+        [p20] "v"(gl::lo32(p2)), [q21] "v"(gl::hi32(q2)), [t20] "v"(gl::lo32(t2)), [q20] "v"(gl::lo32(q2)),
+        [x0] "v"(x0), [x1] "v"(x1), [fx] "v"(fx), [kl] "v"(k_lo), [kh] "v"(k_hi));
+  asm("v_mad_u64_u32 %[v], %[n], %[r2], -1, %[e]\n"
+      "v_mad_u64_u32 %[v2], %[n2], %[h2], -1, %[d]\n"
+      "s_nop 0\n"
+      "v_cndmask_b32_e64 %[f], 0, -1, %[n]\n"
+      "v_cndmask_b32_e64 %[f2], 0, -1, %[n2]\n"
+      : [v] "=&v"(v), [n] "=&s"(n), [f] "=&v"(f), [v2] "=&v"(v2), [n2] "=&s"(n2), [f2] "=&v"(f2)
+      : [r2] "v"(r2), [e] "v"(gl::pair64(e0, e1)), [h2] "v"(h2), [d] "v"(gl::pair64(d0, d1)));
+  asm("v_addc_co_u32_e64 %[s0], %[m], %[v0], %[f], %[m]\n"
+      "v_addc_co_u32_e64 %[g0], %[m2], %[v20], %[f2], %[m2]\n"
+      "s_nop 0\n"
+      "v_addc_co_u32_e64 %[s1], %[m], %[v1], 0, %[m]\n"
+      "v_addc_co_u32_e64 %[g1], %[m2], %[v21], 0, %[m2]\n"
+      : [s0] "=&v"(s0), [s1] "=&v"(s1), [g0] "=&v"(g0), [g1] "=&v"(g1), [m] "+s"(m), [m2] "+s"(m2)
+      : [v0] "v"(gl::lo32(v)), [v1] "v"(gl::hi32(v)), [f] "v"(f), [v20] "v"(gl::lo32(v2)), [v21] "v"(gl::hi32(v2)),
+        [f2] "v"(f2));
+  const uint64_t sq = gl::pair64(s0, s1);
+  const uint32_t y0 = g0, y1 = g1;  // the term
+  // the cube and the fourth power
+  t = coop_mid(sq, x, p, m);
+  t2 = coop_mid(sq, sq, p2, m2);
+  q = coop_top(t, sq, x);
+  q2 = coop_top(t2, sq, sq);
+  asm("v_subb_co_u32_e64 %[e0], %[m], %[p0], %[q1], %[m]\n"
+      "v_subb_co_u32_e64 %[d0], %[m2], %[p20], %[q21], %[m2]\n"
+      "v_and_b32 %[a], %[y0], %[keep]\n"
+      "v_subb_co_u32_e64 %[e1], %[m], %[t0], 0, %[m]\n"
+      "v_subb_co_u32_e64 %[d1], %[m2], %[t20], 0, %[m2]\n"
+      "v_alignbit_b32 %[b], %[y1], %[y0], 22\n"
+      "v_subb_co_u32_e64 %[r2], %[m], %[q0], 0, %[m]\n"
+      "v_subb_co_u32_e64 %[h2], %[m2], %[q20], 0, %[m2]\n"
+      : [e0] "=&v"(e0), [e1] "=&v"(e1), [r2] "=&v"(r2), [d0] "=&v"(d0), [d1] "=&v"(d1), [h2] "=&v"(h2), [a] "=&v"(a),
+        [b] "=&v"(b), [m] "+s"(m), [m2] "+s"(m2)
+      : [p0] "v"(gl::lo32(p)), [q1] "v"(gl::hi32(q)), [t0] "v"(gl::lo32(t)), [q0] "v"(gl::lo32(q)),
+        [p20] "v"(gl::lo32(p2)), [q21] "v"(gl::hi32(q2)), [t20] "v"(gl::lo32(t2)), [q20] "v"(gl::lo32(q2)),
+        [y0] "v"(y0), [y1] "v"(y1), [keep] "v"(keep));
+  asm("v_mad_u64_u32 %[v], %[n], %[r2], -1, %[e]\n"
+      "v_mad_u64_u32 %[v2], %[n2], %[h2], -1, %[d]\n"
+      "v_lshrrev_b32 %[c], 12, %[y1]\n"
+      "v_cndmask_b32_e64 %[f], 0, -1, %[n]\n"
+      "v_cndmask_b32_e64 %[f2], 0, -1, %[n2]\n"
+      : [v] "=&v"(v), [n] "=&s"(n), [f] "=&v"(f), [v2] "=&v"(v2), [n2] "=&s"(n2), [f2] "=&v"(f2), [c] "=&v"(c)
+      : [r2] "v"(r2), [e] "v"(gl::pair64(e0, e1)), [h2] "v"(h2), [d] "v"(gl::pair64(d0, d1)), [y1] "v"(y1));
+  asm("v_addc_co_u32_e64 %[s0], %[m], %[v0], %[f], %[m]\n"
+      "v_addc_co_u32_e64 %[g0], %[m2], %[v20], %[f2], %[m2]\n"
+      "v_and_b32 %[b], %[b], %[keep]\n"
+      "v_addc_co_u32_e64 %[s1], %[m], %[v1], 0, %[m]\n"
+      "v_addc_co_u32_e64 %[g1], %[m2], %[v21], 0, %[m2]\n"
+      : [s0] "=&v"(s0), [s1] "=&v"(s1), [g0] "=&v"(g0), [g1] "=&v"(g1), [m] "+s"(m), [m2] "+s"(m2), [b] "+v"(b)
+      : [v0] "v"(gl::lo32(v)), [v1] "v"(gl::hi32(v)), [f] "v"(f), [v20] "v"(gl::lo32(v2)), [v21] "v"(gl::hi32(v2)),
+        [f2] "v"(f2), [keep] "v"(keep));
+  // their product
+  const uint64_t cube = gl::pair64(s0, s1), fourth = gl::pair64(g0, g1);
+  t = coop_mid(cube, fourth, p, m);
+  q = coop_top(t, cube, fourth);
+  asm("s_nop 0\n"
+      "v_subb_co_u32_e64 %[e0], %[m], %[p0], %[q1], %[m]\n"
+      "v_and_b32 %[c], %[c], %[keep]\n" BC_ROR(a, 8)
+      "v_subb_co_u32_e64 %[e1], %[m], %[t0], 0, %[m]\n" BC_ROR(b, 8) BC_ROR(c, 8)
+      "v_subb_co_u32_e64 %[r2], %[m], %[q0], 0, %[m]\n"
+      : [e0] "=&v"(e0), [e1] "=&v"(e1), [r2] "=&v"(r2), [a] "+v"(a), [b] "+v"(b), [c] "+v"(c), [m] "+s"(m)
+      : [p0] "v"(gl::lo32(p)), [q1] "v"(gl::hi32(q)), [t0] "v"(gl::lo32(t)), [q0] "v"(gl::lo32(q)), [keep] "v"(keep));
+  asm("v_mad_u64_u32 %[v], %[n], %[r2], -1, %[e]\n" BC_ROR(a, 4) BC_ROR(b, 4)
+      "v_cndmask_b32_e64 %[f], 0, -1, %[n]\n"
+      : [v] "=&v"(v), [n] "=&s"(n), [f] "=&v"(f), [a] "+v"(a), [b] "+v"(b)
+      : [r2] "v"(r2), [e] "v"(gl::pair64(e0, e1)));
+  // the rotations behind the last instruction also stand before the broadcast
+  // of s0 and s1, which waits as they do
+  asm("v_addc_co_u32_e64 %[s0], %[m], %[v0], %[f], %[m]\n" BC_ROR(c, 4) BC_ROR(a, 2)
+      "v_addc_co_u32_e64 %[s1], %[m], %[v1], 0, %[m]\n" BC_ROR(b, 2) BC_ROR(c, 2) BC_ROR(a, 1) BC_ROR(b, 1) BC_ROR(c, 1)
+      : [s0] "=&v"(s0), [s1] "=&v"(s1), [m] "+s"(m), [a] "+v"(a), [b] "+v"(b), [c] "+v"(c)
+      : [v0] "v"(gl::lo32(v)), [v1] "v"(gl::hi32(v)), [f] "v"(f));
+  acc.a = a;
+  acc.b = b;
+  acc.c = c;
+  return gl::pair64(s0, s1);
+}
 #undef BC_ROR
+
+// a b + lo + hi 2^32 (lo, hi < 2^52), any u64.
+__device__ __forceinline__ uint64_t coop_mul_add(uint64_t a, uint64_t b, uint64_t lo, uint64_t hi) {
+  const uint64_t p = (uint64_t)gl::lo32(a) * gl::lo32(b) + lo;
+  uint64_t t = (uint64_t)gl::lo32(a) * gl::hi32(b) + (hi + gl::hi32(p));
+  uint64_t m, n, v;
+  asm("v_mad_u64_u32 %0, %1, %2, %3, %4" : "=v"(t), "=s"(m) : "v"(gl::hi32(a)), "v"(gl::lo32(b)), "v"(t));
+  const uint64_t q = coop_top(t, a, b);
+  uint32_t e0, e1, r2, f, s0, s1;
+  asm("s_nop 0\n"
+      "v_subb_co_u32_e64 %[e0], %[m], %[p0], %[q1], %[m]\n"
+      "s_nop 1\n"
+      "v_subb_co_u32_e64 %[e1], %[m], %[t0], 0, %[m]\n"
+      "s_nop 1\n"
+      "v_subb_co_u32_e64 %[r2], %[m], %[q0], 0, %[m]\n"
+      : [e0] "=&v"(e0), [e1] "=&v"(e1), [r2] "=&v"(r2), [m] "+s"(m)
+      : [p0] "v"(gl::lo32(p)), [q1] "v"(gl::hi32(q)), [t0] "v"(gl::lo32(t)), [q0] "v"(gl::lo32(q)));
+  asm("v_mad_u64_u32 %[v], %[n], %[r2], -1, %[e]\n"
+      "s_nop 1\n"
+      "v_cndmask_b32_e64 %[f], 0, -1, %[n]\n"
+      : [v] "=&v"(v), [n] "=&s"(n), [f] "=&v"(f)
+      : [r2] "v"(r2), [e] "v"(gl::pair64(e0, e1)));
+  asm("v_addc_co_u32_e64 %[s0], %[m], %[v0], %[f], %[m]\n"
+      "s_nop 1\n"
+      "v_addc_co_u32_e64 %[s1], %[m], %[v1], 0, %[m]\n"
+      : [s0] "=&v"(s0), [s1] "=&v"(s1), [m] "+s"(m)
+      : [v0] "v"(gl::lo32(v)), [v1] "v"(gl::hi32(v)), [f] "v"(f));
+  return gl::pair64(s0, s1);
+}
 
 // lo + hi 2^32 (both below 2^62), any u64.
 __device__ __forceinline__ uint64_t coop_join(uint64_t lo, uint64_t hi) {
@@ -791,12 +932,13 @@ __device__ __forceinline__ uint64_t add_const(uint64_t a, uint64_t b) {
 // whose words are staged in w.
 struct Coop {
   const PosTable &t;
+  const PartialLane (&partial)[PARTIAL][PT];
   const uint64_t (&p2_add)[PARTIAL + PT + 1][2];
   uint64_t *w;      // the row's 2 PT words in LDS
   uint32_t j, jj;   // lane of the row; table row (lanes 12-15 reuse row 11)
   uint32_t keep;    // 22-bit mask, 0 in lanes 12-15
   __device__ __forceinline__ Coop(CoopLds &l, uint32_t lane, uint32_t group)
-      : t(l.t), p2_add(l.p2_add), w(l.words[group]), j(lane), jj(lane < PT ? lane : PT - 1), keep(lane < PT ? 0x3FFFFFu : 0u) {}
+      : t(l.t), partial(l.partial), p2_add(l.p2_add), w(l.words[group]), j(lane), jj(lane < PT ? lane : PT - 1), keep(lane < PT ? 0x3FFFFFu : 0u) {}
 
   __device__ __forceinline__ void stage(uint64_t x) const {
     coop_sync();  // the row's earlier reads come first
@@ -804,9 +946,10 @@ struct Coop {
     coop_sync();
   }
 
-  __device__ __forceinline__ uint64_t mds_row(uint64_t x) const {
+  // The MDS row plus the next round's constant k.
+  __device__ __forceinline__ uint64_t mds_row(uint64_t x, uint64_t k) const {
     stage(x);
-    uint64_t lo = 0, hi = 0;
+    uint64_t lo = gl::lo32(k), hi = gl::hi32(k);
 #pragma unroll
     for (int i = 0; i < PT; ++i) {
       const uint64_t v = w[jj + i];
@@ -818,44 +961,32 @@ struct Coop {
   }
 
   __device__ __forceinline__ void permute(uint64_t &x) const {
-    const uint32_t jm = jj ? jj - 1 : 0;  // index into the 11-entry sparse vectors
+    x = add_const(x, t.rc_full[0][jj]);
 #pragma unroll 1
-    for (int r = 0; r < HALF_FULL - 1; ++r) x = mds_row(coop_sbox(add_const(x, t.rc_full[r][jj])));
+    for (int r = 1; r < HALF_FULL; ++r) x = mds_row(coop_sbox(x), t.rc_full[r][jj]);
     {
-      stage(add_const(coop_sbox(add_const(x, t.rc_full[HALF_FULL - 1][jj])), t.rcf[jj]));
+      stage(add_const(coop_sbox(x), t.rcf[jj]));
       gl::Acc acc;
 #pragma unroll
       for (int c = 0; c < PT; ++c) gl::mac(acc, w[c], t.dense[jj][c]);
       x = gl::acc_reduce(acc);
     }
+    // element 0 becomes z + sum_i vs_i x_i, element i becomes x_i + w_i z
+    const uint32_t keep_rest = j ? keep : 0u, fx = j ? 1u : 0u;
+    const uint32_t g0 = j ? 0u : 1u, g22 = j ? 0u : 1u << 22, g12 = j ? 0u : 1u << 12;
 #pragma unroll 1
     for (int k = 0; k < PARTIAL; ++k) {
-      // element 0 becomes z + sum_i vs_i x_i, element i becomes x_i + w_i z
-      uint64_t term;
-      const uint64_t s = coop_sbox(x, t.vs[k][jm], term);
-      const uint64_t z = row_first(add_const(s, t.sbox_c[k]));
-      Limbs l(term, j ? keep : 0u);
-      l.add_ror<8>();
-      l.add_ror<4>();
-      l.add_ror<2>();
-      l.add_ror<1>();
-      uint64_t wz;
-      const uint64_t wk = t.w_hats[k][jm];
-      gl::mul_row<1, gl::ANY>(&wz, &z, &wk);
-      // the words' halves, then z or x + w z on top
-      const uint64_t add = j ? wz : z;
-      uint64_t lo = gl::lo32(add), hi = gl::hi32(add);
-      if (j) {
-        lo += gl::lo32(x);
-        hi += gl::hi32(x);
-      } else {
-        l.add_to(lo, hi);
-      }
-      x = coop_join(lo, hi);
+      const PartialLane &pl = partial[k][jj];
+      TermSum acc;
+      const uint64_t z = row_first(coop_sbox_terms(x, pl.v, keep_rest, fx, pl.k[0], pl.k[1], acc));
+      acc.lo += (uint64_t)acc.a * g0;
+      acc.lo += (uint64_t)acc.b * g22;
+      acc.hi += (uint64_t)acc.c * g12;
+      x = coop_mul_add(pl.w, z, acc.lo, acc.hi);
     }
-    x = mds_row(coop_sbox(x));
 #pragma unroll 1
-    for (int r = 0; r < 3; ++r) x = mds_row(coop_sbox(add_const(x, t.rc_full[HALF_FULL + r][jj])));
+    for (int r = 0; r < 3; ++r) x = mds_row(coop_sbox(x), t.rc_full[HALF_FULL + r][jj]);
+    x = mds_row(coop_sbox(x), 0);
   }
 
   // (J + I) (x) M4 on the three tiles: each word plus the sum over the tiles,
@@ -916,10 +1047,16 @@ struct Coop {
   }
 };
 
-__device__ __forceinline__ void coop_stage_table(CoopLds &l) {
+template <int H> __device__ __forceinline__ void coop_stage_table(CoopLds &l) {
   const uint64_t *src = (const uint64_t *)&pos_table;
   uint64_t *dst = (uint64_t *)&l.t;
   for (uint32_t i = threadIdx.x; i < sizeof(PosTable) / sizeof(uint64_t); i += blockDim.x) dst[i] = src[i];
+  if constexpr (H == 0) {
+    src = (const uint64_t *)&pos_partial_lanes;
+    dst = (uint64_t *)&l.partial;
+    for (uint32_t i = threadIdx.x; i < sizeof l.partial / sizeof(uint64_t); i += blockDim.x) dst[i] = src[i];
+    return;
+  }
   if (threadIdx.x <= PARTIAL + PT) {
     const uint32_t i = threadIdx.x;
     const uint64_t k = i < PARTIAL ? pos_table.p2_partial[i]
@@ -942,7 +1079,7 @@ __global__ __launch_bounds__(COOP_NT) void poseidon_nodes_coop_kernel(const uint
                                                                       uint32_t layers) {
   __shared__ CoopLds lds;
   __shared__ uint64_t digest[COOP_GROUPS][CAP];
-  coop_stage_table(lds);
+  coop_stage_table<H>(lds);
   const uint32_t group = threadIdx.x / COOP_LANES, j = threadIdx.x % COOP_LANES;
   uint64_t g = (uint64_t)blockIdx.x * COOP_GROUPS + group;
   // element j: left[j] (j < 4), right[j - 4] (4 <= j < 8), capacity 0
@@ -984,7 +1121,7 @@ __global__ __launch_bounds__(COOP_NT) void poseidon_leaves_coop_kernel(const uin
                                                                        bool load_intermediate,
                                                                        bool store_intermediate) {
   __shared__ CoopLds lds;
-  coop_stage_table(lds);
+  coop_stage_table<H>(lds);
   const uint32_t group = threadIdx.x / COOP_LANES, j = threadIdx.x % COOP_LANES;
   const uint64_t g = (uint64_t)blockIdx.x * COOP_GROUPS + group;
   const uint64_t rows = 1ull << log_rows;
@@ -1197,6 +1334,18 @@ void set_mat(PosMat &m, int mat, uint64_t (*kout)[2], int outputs, const uint64_
   }
 }
 
+void derive_lanes(const PosTable &t, PartialLane (*lanes)[PT]) {
+  for (int k = 0; k < PARTIAL; ++k)
+    for (int j = 0; j < PT; ++j) {
+      PartialLane &l = lanes[k][j];
+      l.v = j ? t.vs[k][j - 1] : 0;
+      l.w = j ? t.w_hats[k][j - 1] : 1;
+      const uint64_t c = gl::mul(l.w, t.sbox_c[k]);
+      l.k[0] = (uint32_t)c;
+      l.k[1] = c >> 32;
+    }
+}
+
 // The one-lane forms' tables from the fused one.
 void derive_fast(const PosTable &t, PosFast &f, PosMat &m) {
   uint64_t rows[PT][PT], k[PT];
@@ -1395,6 +1544,8 @@ extern "C" int bc_poseidon_set_round_constants(const uint64_t *round_constants) 
   PosFast f{};
   std::vector<PosMat> m(1);
   derive_fast(t, f, m[0]);
+  PartialLane lanes[PARTIAL][PT];
+  derive_lanes(t, lanes);
   std::unique_lock<std::shared_mutex> lk(pos_mu);
   // hashing kernels already queued on any stream of this device read the
   // table: let them finish before it changes (no new ones can be queued
@@ -1404,6 +1555,8 @@ extern "C" int bc_poseidon_set_round_constants(const uint64_t *round_constants) 
   err = hipMemcpyToSymbol(HIP_SYMBOL(pos_table), &t, sizeof t, 0, hipMemcpyHostToDevice);
   if (err != hipSuccess) return err;
   err = hipMemcpyToSymbol(HIP_SYMBOL(pos_fast), &f, sizeof f, 0, hipMemcpyHostToDevice);
+  if (err != hipSuccess) return err;
+  err = hipMemcpyToSymbol(HIP_SYMBOL(pos_partial_lanes), lanes, sizeof lanes, 0, hipMemcpyHostToDevice);
   if (err != hipSuccess) return err;
   err = hipMemcpyToSymbol(HIP_SYMBOL(pos_mat), &m[0], sizeof m[0], 0, hipMemcpyHostToDevice);
   if (err != hipSuccess) return err;
