@@ -142,9 +142,14 @@ uint32_t brev_bits_host(uint32_t x, uint32_t bits) {
 // Work-unit sizes (see ragged_build).  The persistent kernel runs two
 // workgroups on each of the 256 CUs.  Measured on a 200-job batch of
 // 2^10..2^21 points: 2.04, 2.00, 2.02, 2.14 ms at 2, 4, 8 and 16 units per
-// workgroup (units of 32 tiles wherever a segment had 64 of them: 2.16 ms); a
-// 400-job batch up to 2^23 runs the same from 2 to 32.
+// workgroup (units of 32 tiles wherever a segment had 64 of them: 2.16 ms).
+// The lower bounds pay for a unit's setup in smaller levels, a strided unit's
+// (twists of its r range) more than a contiguous one's: 120 jobs of 2^13..2^19
+// 644 us with none, 605 at 4 strided, 582 at 4 and 4, 571 at 8 and 4, 587 at 8
+// and 8, 592 at 16 and 8; 150 jobs of 2^10..2^18 453, 434, 414, 410, 424, 425;
+// 20 jobs of 2^10..2^14 155 throughout.
 constexpr uint64_t PERSISTENT_WORKGROUPS = 512, UNITS_PER_WORKGROUP = 5, MAX_UNIT = 32;
+constexpr uint64_t MIN_UNIT_STRIDED = 8, MIN_UNIT_CONTIG = 4;
 
 // A stage group: the same transform (log_n, direction, coset) applied to
 // columns of several jobs, planned and run as one batch through per-column
@@ -278,8 +283,9 @@ int ragged_build(const bc_ragged_job *jobs, uint32_t num_jobs, const Tables &tab
 
   // Work units.  A level ends when its last unit does, so units are sized for
   // the level: about UNITS_PER_WORKGROUP of them for each of the persistent
-  // workgroups, of at most MAX_UNIT tiles (which is what amortizes a unit's
-  // setup: twists, coset factors, the queue pop), unless tuned.
+  // workgroups, of at most MAX_UNIT tiles, and of at least MIN_UNIT (which
+  // amortizes a unit's setup: twists, coset factors, the queue pop) as long as
+  // that leaves a unit for every other workgroup, unless tuned.
   uint64_t level_tiles[RAGGED_MAX_LEVELS] = {};
   for (const PlanSeg &ps : segs) {
     if (ps.level >= RAGGED_MAX_LEVELS) return BC_ERROR_INVALID_VALUE;
@@ -288,7 +294,11 @@ int ragged_build(const bc_ragged_job *jobs, uint32_t num_jobs, const Tables &tab
   for (PlanSeg &ps : segs) {
     RaggedSeg &r = ps.s;
     uint64_t u = r.per_unit;
-    if (!u) u = std::min<uint64_t>(level_tiles[ps.level] / (PERSISTENT_WORKGROUPS * UNITS_PER_WORKGROUP), MAX_UNIT);
+    if (!u) {
+      const uint64_t tiles = level_tiles[ps.level];
+      u = std::max(std::min(tiles / (PERSISTENT_WORKGROUPS * UNITS_PER_WORKGROUP), MAX_UNIT),
+                   std::min(tiles / (PERSISTENT_WORKGROUPS / 2), r.positions ? MIN_UNIT_STRIDED : MIN_UNIT_CONTIG));
+    }
     if (u < 1) u = 1;
     if (u > r.total) u = r.total;
     r.per_unit = (uint32_t)u;
