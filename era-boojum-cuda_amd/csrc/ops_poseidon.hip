@@ -43,6 +43,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <stddef.h>
 #include <string.h>
 
 #include <mutex>
@@ -606,9 +607,9 @@ __device__ PartialLane pos_partial_lanes[PARTIAL][PT];
 struct CoopLds {
   PosTable t;
   PartialLane partial[PARTIAL][PT];
-  // constants behind Poseidon2's partial rounds, by halves: of element 0 in
-  // round k (k > 0), of element j behind the last at PARTIAL + j, then zeros
-  uint64_t p2_add[PARTIAL + PT + 1][2];
+  // constants behind Poseidon2's partial rounds, by halves (0 but for element 0
+  // and the last round)
+  uint64_t p2_add[PARTIAL][PT][2];
   uint64_t words[COOP_GROUPS][2 * PT];
 };
 
@@ -666,7 +667,7 @@ __device__ __forceinline__ uint64_t coop_sbox(uint64_t x) {
 // after its write), and a wave alone on its SIMD pays a full issue slot for
 // every s_nop that fills such a gap: 27 of 119 slots in a Poseidon2 round.
 // The sum does not depend on the S-box's end, so its instructions stand there
-// (104 slots; a Poseidon2 tree of 2^11 leaves, one permutation each, 122 -> 115
+// (103 slots; a Poseidon2 tree of 2^11 leaves, one permutation each, 122 -> 111
 // us; 128 with the same sum ahead of the S-box).  Poseidon: 168 -> 131 slots,
 // four permutations a leaf 63.9 -> 57.8 us at 2^10 leaves.
 #define BC_ROR(v, n) "v_add_u32_dpp %[" #v "], %[" #v "], %[" #v "] row_ror:" #n " row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
@@ -933,7 +934,7 @@ __device__ __forceinline__ uint64_t add_const(uint64_t a, uint64_t b) {
 struct Coop {
   const PosTable &t;
   const PartialLane (&partial)[PARTIAL][PT];
-  const uint64_t (&p2_add)[PARTIAL + PT + 1][2];
+  const uint64_t (&p2_add)[PARTIAL][PT][2];
   uint64_t *w;      // the row's 2 PT words in LDS
   uint32_t j, jj;   // lane of the row; table row (lanes 12-15 reuse row 11)
   uint32_t keep;    // 22-bit mask, 0 in lanes 12-15
@@ -990,7 +991,8 @@ struct Coop {
   }
 
   // (J + I) (x) M4 on the three tiles: each word plus the sum over the tiles,
-  // then the 4 x 4 row, on limbs, plus the constant k.
+  // then the 4 x 4 row, on limbs, plus the constant k (with 32-bit products, a
+  // quarter of the 24-bit ones' rate, the tree above took 109 us, now 107).
   __device__ __forceinline__ uint64_t m_ext_row(uint64_t x, const uint32_t *m4row, uint64_t k) const {
     Limbs l(x, keep), s = l;
     s.add_ror<8>();
@@ -998,8 +1000,9 @@ struct Coop {
     l.a += s.a;
     l.b += s.b;
     l.c += s.c;
-    auto row = [&](uint32_t v) {  // limbs below 2^25, the row sums to at most 16
-      return m4row[0] * dpp<0x00>(v) + m4row[1] * dpp<0x55>(v) + m4row[2] * dpp<0xAA>(v) + m4row[3] * dpp<0xFF>(v);
+    auto row = [&](uint32_t v) {  // four limbs below 2^22: 24-bit products; the row sums to at most 16
+      return __umul24(m4row[0], dpp<0x00>(v)) + __umul24(m4row[1], dpp<0x55>(v)) + __umul24(m4row[2], dpp<0xAA>(v)) +
+             __umul24(m4row[3], dpp<0xFF>(v));
     };
     l.a = row(l.a);
     l.b = row(l.b);
@@ -1021,19 +1024,21 @@ struct Coop {
 #pragma unroll
     for (int i = 1; i < PT; ++i) mu = jj == (uint32_t)i ? 1u << P2_MU[i] : mu;
     const uint32_t keep_rest = j ? keep : 0u, z_factor = j ? 1u : 1u + (1u << P2_MU[0]);
+    uint32_t s22 = 1u << 22, s12 = 1u << 12;
+    asm volatile("" : "+s"(s22), "+s"(s12));
     // the constants of the next round ride on each matrix
     x = m_ext_row(x, m4row, t.p2_full[0][jj]);
 #pragma unroll 1
     for (int r = 1; r < HALF_FULL; ++r) x = m_ext_row(coop_sbox(x), m4row, t.p2_full[r][jj]);
     x = m_ext_row(coop_sbox(x), m4row, j ? 0ull : t.p2_partial[0]);
 #pragma unroll 1
-    for (int k = 1; k <= PARTIAL; ++k) {
+    for (int k = 0; k < PARTIAL; ++k) {
       // y_0 = rest + (1 + 2^mu_0) z, y_i = rest + mu_i x_i + z
-      const uint64_t *kp = p2_add[k == PARTIAL ? PARTIAL + jj : (j ? PARTIAL + PT : (uint32_t)k)];
+      const uint64_t *kp = p2_add[k][jj];
       RestSum rest;
       const uint64_t z = row_first(coop_sbox_rest(x, keep_rest, mu, kp[0], kp[1], rest));
-      rest.lo += (uint64_t)rest.b * opaque(1u << 22) + (uint64_t)gl::lo32(z) * z_factor;
-      rest.hi += (uint64_t)rest.c * opaque(1u << 12) + (uint64_t)gl::hi32(z) * z_factor;
+      rest.lo += (uint64_t)rest.b * s22 + (uint64_t)gl::lo32(z) * z_factor;
+      rest.hi += (uint64_t)rest.c * s12 + (uint64_t)gl::hi32(z) * z_factor;
       x = coop_join(rest.lo, rest.hi);
     }
 #pragma unroll 1
@@ -1048,21 +1053,22 @@ struct Coop {
 };
 
 template <int H> __device__ __forceinline__ void coop_stage_table(CoopLds &l) {
-  const uint64_t *src = (const uint64_t *)&pos_table;
-  uint64_t *dst = (uint64_t *)&l.t;
-  for (uint32_t i = threadIdx.x; i < sizeof(PosTable) / sizeof(uint64_t); i += blockDim.x) dst[i] = src[i];
   if constexpr (H == 0) {
+    const uint64_t *src = (const uint64_t *)&pos_table;
+    uint64_t *dst = (uint64_t *)&l.t;
+    for (uint32_t i = threadIdx.x; i < offsetof(PosTable, p2_full) / sizeof(uint64_t); i += blockDim.x) dst[i] = src[i];
     src = (const uint64_t *)&pos_partial_lanes;
     dst = (uint64_t *)&l.partial;
     for (uint32_t i = threadIdx.x; i < sizeof l.partial / sizeof(uint64_t); i += blockDim.x) dst[i] = src[i];
     return;
   }
-  if (threadIdx.x <= PARTIAL + PT) {
-    const uint32_t i = threadIdx.x;
-    const uint64_t k = i < PARTIAL ? pos_table.p2_partial[i]
-                                   : (i < PARTIAL + PT ? pos_table.p2_full[HALF_FULL][i - PARTIAL] : 0ull);
-    l.p2_add[i][0] = gl::lo32(k);
-    l.p2_add[i][1] = gl::hi32(k);
+  if (threadIdx.x < 2 * HALF_FULL * PT) (&l.t.p2_full[0][0])[threadIdx.x] = (&pos_table.p2_full[0][0])[threadIdx.x];
+  if (threadIdx.x == 0) l.t.p2_partial[0] = pos_table.p2_partial[0];
+  for (uint32_t i = threadIdx.x; i < PARTIAL * PT; i += blockDim.x) {
+    const uint32_t r = i / PT, j = i % PT;
+    const uint64_t k = r == PARTIAL - 1 ? pos_table.p2_full[HALF_FULL][j] : (j ? 0ull : pos_table.p2_partial[r + 1]);
+    l.p2_add[r][j][0] = gl::lo32(k);
+    l.p2_add[r][j][1] = gl::hi32(k);
   }
 }
 
