@@ -262,23 +262,19 @@ template <uint32_t LPC, uint32_t K, bool PREFETCH> struct EvalShape {
 // Tile shapes per kind, from a sweep on MI355X over 256 columns of 2^20 and
 // 2^16 rows: wide contiguous runs per column (64 lanes x 16 B = 1 KiB per
 // load instruction) read fastest.  `large` serves columns of at least 2^18
-// rows, `mid` shorter ones, `small` columns of 128..(mid rows - 1) rows; below
-// 128 rows one thread per column sums the column directly.
+// rows, `mid` shorter ones above COLUMN_MAX_ROWS.
 template <uint32_t KIND> struct Shapes;
 template <> struct Shapes<BASE_AT_BASE> {
   using large = EvalShape<64, 16, false>;  // 2048-row tiles
   using mid = EvalShape<64, 4, true>;      // 512
-  using small = EvalShape<16, 4, false>;   // 128
 };
 template <> struct Shapes<BASE_AT_EXT> {
   using large = EvalShape<64, 8, false>;  // 1024
   using mid = EvalShape<16, 4, false>;    // 128
-  using small = EvalShape<16, 4, false>;
 };
 template <> struct Shapes<EXT_AT_EXT> {
   using large = EvalShape<64, 4, true>;  // 512
   using mid = EvalShape<64, 4, true>;
-  using small = EvalShape<16, 4, false>;
 };
 constexpr uint64_t BE_LARGE_COUNT = 1ull << 18;
 
@@ -428,7 +424,69 @@ __global__ __launch_bounds__(BE_NT) void bary_eval_final_kernel(const uint64_t *
   }
 }
 
-// N < 128: one thread per column sums its N products directly.
+// Few rows (N >= 2, a power of two): one workgroup per column sums it in one
+// launch, without partial sums in memory.  Bound by the chain of loads, products
+// and the sum over lanes.
+template <uint32_t KIND, bool ALIGNED, uint32_t THREADS>
+__global__ __launch_bounds__(THREADS) void bary_eval_column_kernel(const uint64_t *ys, const uint64_t *coeffs,
+                                                                   uint32_t count, uint64_t *evals) {
+  constexpr bool CEXT = KIND != BASE_AT_BASE;
+  constexpr bool YEXT = KIND == EXT_AT_EXT;
+  constexpr uint32_t WAVES = THREADS / 64;
+  __shared__ uint64_t part[2][WAVES];
+  const uint64_t c = blockIdx.x;
+  const uint64_t *col = ys + c * (YEXT ? 2 : 1) * count;
+  gl::Acc a0, a1, a2;
+  for (uint32_t r = 2 * threadIdx.x; r < count; r += 2 * THREADS) {
+    const U2 l = load2<ALIGNED>(coeffs + r), y = load2<ALIGNED>(col + r);
+    gl::mac(a0, y.x, l.x);
+    gl::mac(a0, y.y, l.y);
+    if constexpr (CEXT) {
+      const U2 m = load2<ALIGNED>(coeffs + count + r);
+      gl::mac(a1, y.x, m.x);
+      gl::mac(a1, y.y, m.y);
+      if constexpr (YEXT) {
+        const U2 z = load2<ALIGNED>(col + count + r);
+        gl::mac(a1, z.x, l.x);
+        gl::mac(a1, z.y, l.y);
+        gl::mac(a2, z.x, m.x);
+        gl::mac(a2, z.y, m.y);
+      }
+    }
+  }
+  uint64_t s0 = gl::acc_reduce(a0), s1 = CEXT ? gl::acc_reduce(a1) : 0ull;
+  if constexpr (YEXT) s0 = gl::add(s0, gl::mul_by_non_residue(gl::acc_reduce(a2)));
+#pragma unroll
+  for (int m = 1; m < 64; m <<= 1) {
+    s0 = gl::add(s0, shfl_xor64(s0, m));
+    if constexpr (CEXT) s1 = gl::add(s1, shfl_xor64(s1, m));
+  }
+  if constexpr (WAVES > 1) {
+    if ((threadIdx.x & 63) == 0) {
+      part[0][threadIdx.x >> 6] = s0;
+      part[1][threadIdx.x >> 6] = s1;
+    }
+    __syncthreads();
+    s0 = part[0][0];
+    s1 = part[1][0];
+#pragma unroll
+    for (uint32_t w = 1; w < WAVES; ++w) {
+      s0 = gl::add(s0, part[0][w]);
+      if constexpr (CEXT) s1 = gl::add(s1, part[1][w]);
+    }
+  }
+  if (threadIdx.x == 0) {
+    if constexpr (CEXT) {
+      evals[2 * c] = s0;
+      evals[2 * c + 1] = s1;
+    } else {
+      evals[c] = s0;
+    }
+  }
+}
+
+// N < 32 (or N < 128 and many columns): one thread per column sums its N
+// products directly.
 template <uint32_t KIND>
 __global__ void bary_eval_small_kernel(const uint64_t *ys, const uint64_t *coeffs, uint32_t count,
                                        uint32_t num_polys, uint64_t *evals) {
@@ -466,13 +524,14 @@ int finish() {
 bool power_of_two(uint64_t v) { return v && !(v & (v - 1)); }
 
 // Tiles of a column (each gives one partial sum) for the shape that serves N
-// rows; 0 selects the one-thread-per-column kernel.
+// rows, and so the partial sums a caller provides room for (short columns,
+// which take none now, keep the room they were given).
+constexpr uint32_t MIN_TILE_ROWS = 128;
 template <uint32_t KIND> uint32_t tile_rows(uint64_t count) {
   using T = Shapes<KIND>;
   if (count >= BE_LARGE_COUNT && count >= T::large::rows) return T::large::rows;
   if (count >= T::mid::rows) return T::mid::rows;
-  if (count >= T::small::rows) return T::small::rows;
-  return 0;
+  return count >= MIN_TILE_ROWS ? MIN_TILE_ROWS : 0;
 }
 
 uint64_t eval_tiles(uint32_t kind, uint64_t count) {
@@ -523,21 +582,45 @@ void launch_tiles(const uint64_t *ys, const uint64_t *coeffs, uint64_t count, ui
   bary_eval_final_kernel<OUT_EXT><<<dim3(num_polys), BE_NT, 0, s>>>(partial, tiles, evals);
 }
 
+// Columns of 32..1024 rows take the column kernel, below 128 rows while the
+// columns are few.  Coefficients and evaluations at an extension point, column
+// kernel against the others: 20 columns of 2^5 / 2^6 / 2^8 / 2^10 / 2^12 rows
+// 18.2 / 18.4 / 18.8 / 19.9 / 23.9 us against 19.8 / 23.9 / 20.4 / 21.2 / 22.0
+// (2^3: 18.6 against 16.6), 40000 columns of 2^7 / 2^8 rows 34 / 40 against 74 /
+// 82 us, of 2^5 32 against 24, 4000 of 2^10 28 against 31.
+constexpr uint64_t COLUMN_MIN_ROWS = 32, COLUMN_MAX_ROWS = 1024;
+constexpr uint32_t COLUMN_FEW = 8192;
+bool column_path(uint64_t count, uint32_t num_polys) {
+  return count >= COLUMN_MIN_ROWS && count <= COLUMN_MAX_ROWS && (count >= 128 || num_polys <= COLUMN_FEW);
+}
+
+template <uint32_t KIND>
+void launch_column(const uint64_t *ys, const uint64_t *coeffs, uint32_t count, uint32_t num_polys, uint64_t *evals,
+                   hipStream_t s) {
+  const bool aligned = !(((uintptr_t)ys | (uintptr_t)coeffs) & 15);
+  auto go = [&](auto threads) {
+    constexpr uint32_t N = decltype(threads)::value;
+    if (aligned) bary_eval_column_kernel<KIND, true, N><<<dim3(num_polys), N, 0, s>>>(ys, coeffs, count, evals);
+    else bary_eval_column_kernel<KIND, false, N><<<dim3(num_polys), N, 0, s>>>(ys, coeffs, count, evals);
+  };
+  if (count <= 512) go(std::integral_constant<uint32_t, 64>{});
+  else go(std::integral_constant<uint32_t, 256>{});
+}
+
 template <uint32_t KIND>
 void launch_eval(const uint64_t *ys, const uint64_t *coeffs, uint64_t count, uint32_t num_polys, uint64_t *partial,
                  uint64_t *evals, hipStream_t s) {
   using T = Shapes<KIND>;
-  const uint32_t rows = tile_rows<KIND>(count);
-  if (rows == 0)
+  if (column_path(count, num_polys))
+    launch_column<KIND>(ys, coeffs, (uint32_t)count, num_polys, evals, s);
+  else if (count < COLUMN_MAX_ROWS)
     bary_eval_small_kernel<KIND><<<dim3((num_polys + 255) / 256), 256, 0, s>>>(ys, coeffs, (uint32_t)count,
                                                                                num_polys, evals);
-  else if (rows == T::large::rows && count >= BE_LARGE_COUNT)  // about three whole rounds of resident workgroups
+  else if (count >= BE_LARGE_COUNT)  // about three whole rounds of resident workgroups
     launch_tiles<KIND, typename T::large>(ys, coeffs, count, num_polys, partial, evals,
                                           3ull * resident_wgs<KIND, typename T::large>(), s);
-  else if (rows == T::mid::rows)
-    launch_tiles<KIND, typename T::mid>(ys, coeffs, count, num_polys, partial, evals, 8192, s);
   else
-    launch_tiles<KIND, typename T::small>(ys, coeffs, count, num_polys, partial, evals, 8192, s);
+    launch_tiles<KIND, typename T::mid>(ys, coeffs, count, num_polys, partial, evals, 8192, s);
 }
 
 }  // namespace
