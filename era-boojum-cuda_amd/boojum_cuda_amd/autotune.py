@@ -27,7 +27,7 @@ from ._lib import lib
 
 MAX_TUNE_ELEMS = 1 << 28  # larger shapes reuse the nearest tuned bucket
 MIN_GAIN = 0.02           # a candidate must beat the incumbent by 2% (timing noise)
-SMALL_LOG_N, SMALL_MAX_COLS = 16, 4  # the built-in latency-path rule (csrc/ntt_internal.hpp)
+SMALL_MIN_LOG_N, SMALL_LOG_N, SMALL_LOG_POINTS = 13, 16, 18  # the built-in latency-path rule (csrc/ntt_internal.hpp)
 
 
 class TuneParams(ctypes.Structure):
@@ -194,13 +194,14 @@ def tune_shape(log_n, log_cols, reps=5, log=print):
     # not pick for this column count); the rest of the search applies to the
     # 4096-point kernels only
     if log_n == SMALL_LOG_N:
-        alt = 12 if num_cols <= SMALL_MAX_COLS else 8
+        alt = 12 if num_cols << log_n <= 1 << SMALL_LOG_POINTS else 8
         p = TuneParams()
         p.tile_log = alt
         ms = trial(p)
         if better(ms, best_ms):
             best, best_ms = p, ms
-    small = best.tile_log == 8 or (log_n == SMALL_LOG_N and best.tile_log == 0 and num_cols <= SMALL_MAX_COLS)
+    small = best.tile_log == 8 or (SMALL_MIN_LOG_N <= log_n <= SMALL_LOG_N and best.tile_log == 0
+                                   and num_cols << log_n <= 1 << SMALL_LOG_POINTS)
     # 1. pass split (the built-in split itself is not a candidate: an entry
     # that repeats it could only record timing noise)
     for c, k in ([] if small else splits(log_n)):

@@ -174,7 +174,7 @@ extern "C" int bc_batch_ntt_internal(const uint64_t *inputs, uint64_t *outputs, 
 
   const TuneParams tp = tuned(log_n, num_ntts);
   if (small_path_applies(log_n, num_ntts, log_ext, tp))
-    return launch_small(ctx->tab, inputs, outputs, num_ntts, stride_in, stride_out, bitrev_inputs, inverse, s);
+    return launch_small(ctx->tab, inputs, outputs, log_n, num_ntts, stride_in, stride_out, bitrev_inputs, inverse, s);
 
   PassDesc passes[8];
   const int np = describe_fast_passes(ctx->tab, inputs, outputs, log_n, num_ntts, stride_in, stride_out,
@@ -383,19 +383,19 @@ extern "C" int bc_ntt_describe_plan(uint32_t log_n, uint32_t num_ntts, bool bitr
   *num_passes = 0;
   if (log_n < 8 || num_ntts == 0) return BC_SUCCESS;
   if (small_path_applies(log_n, num_ntts, log_ext, tuned(log_n, num_ntts))) {
-    // two one-wave passes of 8 bits: the top one (stride 256, pass twist,
-    // n^-1 for inverses) and the bottom one; b2n runs them in reverse
+    // two one-wave passes: the top one (stride 256, pass twist, n^-1 for
+    // inverses) and the bottom one of 8 bits; b2n runs them in reverse
     if (!passes || max_passes < 2) return BC_ERROR_INVALID_VALUE;
     for (int k = 0; k < 2; ++k) {
       const bool top = (k == 0) != bitrev_inputs;
       bc_pass_info &o = passes[k];
       o = bc_pass_info{};
       o.contiguous = top ? 0u : 1u;
-      o.log_h = 8;
-      o.log_block = top ? SMALL_LOG_N : 8;
+      o.log_h = top ? log_n - 8 : 8;
+      o.log_block = top ? log_n : 8;
       o.mode = top && inverse ? (uint32_t)MODE_NINV : (uint32_t)MODE_NONE;
-      o.work_items = (uint64_t)num_ntts << 8;
-      o.positions = top ? 256 : 0;
+      o.work_items = (uint64_t)num_ntts << (top ? 8 : log_n - 8);
+      o.positions = top ? 1u << (log_n - 8) : 0;
       o.groups = top ? num_ntts : 0;
       o.pairs_per_workgroup = top ? 1 : 0;
       o.workgroup_threads = 64;

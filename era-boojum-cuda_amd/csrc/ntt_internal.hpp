@@ -128,14 +128,19 @@ void tune_autoload();
 constexpr uint32_t TILE_LOG = 12;
 constexpr uint32_t TILE = 1u << TILE_LOG;
 
-// Latency path (ntt_small.hip): 1..SMALL_MAX_COLS columns of 2^SMALL_LOG_N
-// points with no coset, as two launches of one-wave workgroups.
-constexpr uint32_t SMALL_LOG_N = 16;
-constexpr uint32_t SMALL_MAX_COLS = 4;
+// Latency path (ntt_small.hip): columns of 2^SMALL_MIN_LOG_N .. 2^SMALL_LOG_N
+// points with no coset, at most 2^SMALL_LOG_POINTS points in all, as two
+// launches of one-wave workgroups: four waves a SIMD, one round.  Against the
+// 4096-point passes, at half, all and twice that: 2^13 8.6, 8.9, 13.0 us
+// against 12.7, 13.2, 13.9; 2^15 8.6, 9.6, 14.2 against 13.0, 13.6, 14.6; 2^16
+// 9.2, 10.8, 16.8, the last against 14.1.
+constexpr uint32_t SMALL_MIN_LOG_N = 13, SMALL_LOG_N = 16;
+constexpr uint32_t SMALL_LOG_POINTS = 18;
 // Whether a call of this shape takes the latency path under tuned params tp.
 bool small_path_applies(uint32_t log_n, uint32_t num_cols, uint32_t log_ext, const TuneParams &tp);
-hipError_t launch_small(const Tables &tab, const uint64_t *inputs, uint64_t *outputs, uint32_t num_cols,
-                        uint64_t stride_in, uint64_t stride_out, bool bitrev_inputs, bool inverse, hipStream_t s);
+hipError_t launch_small(const Tables &tab, const uint64_t *inputs, uint64_t *outputs, uint32_t log_n,
+                        uint32_t num_cols, uint64_t stride_in, uint64_t stride_out, bool bitrev_inputs, bool inverse,
+                        hipStream_t s);
 
 // log_n 1..7 (ntt_small.hip): a.coset_exp, a.log_ext and a.n_inv as for the
 // fast passes.

@@ -1,15 +1,15 @@
 // Transforms of one wave, 4 values per lane: columns of 2..128 points
-// (ntt_short_kernel, below), and the latency path for a few columns of 2^16
-// points (the single-column case of the reference's benches) as two launches
-// of one-wave workgroups, each wave holding one 256-point sub-DFT.
+// (ntt_short_kernel, below), and the latency path for a few columns of
+// 2^13..2^16 points (the single-column case of the reference's benches) as two
+// launches of one-wave workgroups, each wave holding 256 values.
 //
 // The pass kernels of ntt_fast.hip give each thread 16 values of a 4096-point
 // tile, so one 2^16 column is 16 workgroups per pass and the call takes one
-// workgroup's serial work.  Here a 2^16 transform is split 8 + 8: the top pass
-// runs 256 sub-DFTs over the top index bits (stride 256, with the pass twist
-// omega_n^(r * brev(j))), the bottom pass 256 sub-DFTs over consecutive
-// points; 256 one-wave workgroups per column per pass, and each lane does four
-// values' work.
+// workgroup's serial work.  Here the transform is split h + 8: the top pass
+// runs 256 2^h-point sub-DFTs over the top index bits (stride 256, with the
+// pass twist omega_n^(r * brev(j))), 2^(8-h) to a wave, the bottom pass
+// 256-point sub-DFTs over consecutive points, one to a wave; each lane does
+// four values' work.
 //
 // One wave's 256-point DIF, point j = 64 i + l at lane l, register i:
 //   stage 1: radix 4 over j bits 7..6 (registers), twist omega_256^(l k1);
@@ -80,93 +80,118 @@ struct WaveLds {
   uint64_t ex3[4 * SW];
 };
 
-// Stage twiddles of lane l: tw[3 (s - 1) + i - 1] for stage s = 1..3 and
-// register i = 1..3 (register 0 has k = 0).
-__device__ __forceinline__ void stage_twiddles(const Tables &tab, uint32_t l, bool inv, uint64_t *tw) {
+// The lower LN levels of a wave's 256-point transform: 2^(8-LN) transforms of
+// 2^LN points.  Position p of the wave's 256 values is point p mod 2^LN of
+// transform p / 2^LN; at stage s register i of lane l holds the position with
+// register bits at B = 6 - 2s, and the stages above the transforms' length
+// (and the exchanges behind them) fall away.  With odd LN the first stage is
+// radix 2 over its lower bit.
+template <int LN, bool INV, bool DIT> struct WaveDft {
+  static constexpr int S0 = 4 - (LN + 1) / 2;
+  static constexpr int FIRST = DIT ? 3 : S0, LAST = DIT ? S0 : 3;  // stages of the inputs and the outputs
+  uint32_t l;
+  uint64_t tw[3][3];  // twists of registers 1..3 behind (DIT: before) the stages
+  __device__ __forceinline__ WaveDft(const Tables &tab, uint32_t lane) : l(lane) {
+    static_for<3 - S0>([&](auto k) {
+      constexpr int S = S0 + decltype(k)::value, B = 6 - 2 * S;
+      const uint32_t rp = l & ((1u << B) - 1u);
+      if constexpr (S == S0 && LN % 2) {
+        tw[S][0] = root(tab, B + 1, rp, INV);
+      } else {
 #pragma unroll
-  for (int i = 1; i < 4; ++i) {
-    const uint32_t k = brev2((uint32_t)i);
-    tw[i - 1] = root(tab, 8, l * k, inv);
-    tw[3 + i - 1] = root(tab, 6, (l & 15u) * k, inv);
-    tw[6 + i - 1] = root(tab, 4, (l & 3u) * k, inv);
+        for (int i = 1; i < 4; ++i) tw[S][i - 1] = root(tab, B + 2, rp * brev2((uint32_t)i), INV);
+      }
+    });
   }
-}
+  __device__ __forceinline__ uint32_t pos(int s, int i) const {
+    const int b = 6 - 2 * s;
+    return ((l >> b) << (b + 2)) | ((uint32_t)i << b) | (l & ((1u << b) - 1u));
+  }
+  template <int S> __device__ __forceinline__ void twist(uint64_t *x) const {
+    if constexpr (S == 3) return;
+    else if constexpr (S == S0 && LN % 2) {
+      x[1] = gl::mul(x[1], tw[S][0]);
+      x[3] = gl::mul(x[3], tw[S][0]);
+    } else {
+#pragma unroll
+      for (int i = 1; i < 4; ++i) x[i] = gl::mul(x[i], tw[S][i - 1]);
+    }
+  }
+  template <int S> __device__ __forceinline__ static void dft(uint64_t *x) {
+    constexpr int A = S == S0 && LN % 2 ? 1 : 2;
+#pragma unroll
+    for (int g = 0; g < 4; g += 1 << A) {
+      if constexpr (DIT) dft_dit<A, INV>(x + g);
+      else dft_dif<A, INV>(x + g);
+    }
+  }
+  // between stages S and S + 1, either way
+  template <int S> __device__ __forceinline__ void exchange(uint64_t *x, WaveLds &sh) const {
+    if constexpr (S == 0) swap_lane45(x);
+    else if constexpr (S == 1) swap_lanes_lds<2>(x, sh.ex2, l);
+    else if constexpr (S == 2) swap_lanes_lds<0>(x, sh.ex3, l);
+  }
+  // canonical values in, canonical values out
+  __device__ __forceinline__ void run(uint64_t *x, WaveLds &sh) const {
+    static_for<4 - S0>([&](auto k) {
+      constexpr int K = decltype(k)::value, S = DIT ? 3 - K : S0 + K;
+      if constexpr (DIT) {
+        if constexpr (K > 0) exchange<S>(x, sh);
+        twist<S>(x);
+        dft<S>(x);
+      } else {
+        dft<S>(x);
+        twist<S>(x);
+        if constexpr (S < 3) exchange<S>(x, sh);
+      }
+    });
+  }
+};
 
-template <bool INV> __device__ __forceinline__ void wave_dif256(uint64_t *x, const uint64_t *tw, WaveLds &sh, uint32_t l) {
-  dft_dif<2, INV>(x);
-#pragma unroll
-  for (int i = 1; i < 4; ++i) x[i] = gl::mul(x[i], tw[i - 1]);
-  swap_lane45(x);
-  dft_dif<2, INV>(x);
-#pragma unroll
-  for (int i = 1; i < 4; ++i) x[i] = gl::mul(x[i], tw[3 + i - 1]);
-  swap_lanes_lds<2>(x, sh.ex2, l);
-  dft_dif<2, INV>(x);
-#pragma unroll
-  for (int i = 1; i < 4; ++i) x[i] = gl::mul(x[i], tw[6 + i - 1]);
-  swap_lanes_lds<0>(x, sh.ex3, l);
-  dft_dif<2, INV>(x);
-}
-
-template <bool INV> __device__ __forceinline__ void wave_dit256(uint64_t *x, const uint64_t *tw, WaveLds &sh, uint32_t l) {
-  dft_dit<2, INV>(x);
-  swap_lanes_lds<0>(x, sh.ex3, l);
-#pragma unroll
-  for (int i = 1; i < 4; ++i) x[i] = gl::mul(x[i], tw[6 + i - 1]);
-  dft_dit<2, INV>(x);
-  swap_lanes_lds<2>(x, sh.ex2, l);
-#pragma unroll
-  for (int i = 1; i < 4; ++i) x[i] = gl::mul(x[i], tw[3 + i - 1]);
-  dft_dit<2, INV>(x);
-  swap_lane45(x);
-#pragma unroll
-  for (int i = 1; i < 4; ++i) x[i] = gl::mul(x[i], tw[i - 1]);
-  dft_dit<2, INV>(x);
-}
-
-// Top pass (sub-DFTs over index bits 15..8, stride 256): workgroup (r, column).
-// DIF loads natural points (64 i + l) 256 + r and stores position 4 l + i with
-// the pass twist omega_65536^(r brev8(4 l + i)) (n^-1 folded in for inverse
-// transforms); DIT is the transpose.
-template <bool INV, bool DIT>
+// Top pass of a 2^(LH+8)-point column: workgroup (group of 2^(8-LH)
+// consecutive r, column), a 2^LH-point sub-DFT over the points j 256 + r for
+// each r, with the pass twist omega_n^(r brev(j)) (n^-1 folded in for inverse
+// transforms) behind it (DIT: before).
+template <int LH, bool INV, bool DIT>
 __global__ __launch_bounds__(SW) void ntt_small_top_kernel(FastArgs a) {
   __shared__ WaveLds sh;
-  const uint32_t l = threadIdx.x;
-  // workgroups are dispatched round-robin over the 8 XCDs: keep the 16
+  // workgroups are dispatched round-robin over the 8 XCDs: keep the
   // workgroups whose r share a 128-byte line on one XCD (one L2)
-  const uint32_t r = ((blockIdx.x & 7u) << 5) | (blockIdx.x >> 3);
+  const uint32_t r0 = (((blockIdx.x & 7u) << (LH - 3)) | (blockIdx.x >> 3)) << (8 - LH);
   const uint64_t c = blockIdx.y;
-  const uint64_t *in = a.in + c * a.stride_in + r;
-  uint64_t *out = a.out + c * a.stride_out + r;
-  uint64_t tw[9];
-  stage_twiddles(a.tab, l, INV, tw);
+  const uint64_t *in = a.in + c * a.stride_in + r0;
+  uint64_t *out = a.out + c * a.stride_out + r0;
+  using W = WaveDft<LH, INV, DIT>;
+  const W w(a.tab, threadIdx.x);
+  auto at = [&](int s, int i) -> uint64_t {
+    const uint32_t p = w.pos(s, i);
+    return ((uint64_t)(p & ((1u << LH) - 1u)) << 8) + (p >> LH);
+  };
+  constexpr int TS = 3;  // the stage at the twisted end
   uint64_t pt[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const uint32_t k = brev_bits(4u * l + (uint32_t)i, 8);
-    uint32_t e = (r * k) << 16;
+    const uint32_t p = w.pos(TS, i), k = brev_bits(p & ((1u << LH) - 1u), LH);
+    uint32_t e = ((r0 + (p >> LH)) * k) << (24 - LH);
     if (INV) e = 0u - e;
     pt[i] = pow_w(a.tab, e);
     if (INV) pt[i] = gl::mul(pt[i], a.n_inv);
   }
   uint64_t x[4];
-  if constexpr (!DIT) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) x[i] = in[(uint64_t)(64u * i + l) << 8];
+  for (int i = 0; i < 4; ++i) x[i] = in[at(W::FIRST, i)];
+  if constexpr (!DIT) {
     if (a.first) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) x[i] = gl::canon(x[i]);
     }
-    wave_dif256<INV>(x, tw, sh, l);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) out[(uint64_t)(4u * l + i) << 8] = gl::mul(x[i], pt[i]);
   } else {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) x[i] = gl::mul(in[(uint64_t)(4u * l + i) << 8], pt[i]);
-    wave_dit256<INV>(x, tw, sh, l);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) out[(uint64_t)(64u * i + l) << 8] = x[i];
+    for (int i = 0; i < 4; ++i) x[i] = gl::mul(x[i], pt[i]);
   }
+  w.run(x, sh);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) out[at(W::LAST, i)] = DIT ? x[i] : gl::mul(x[i], pt[i]);
 }
 
 // Bottom pass (sub-DFTs over index bits 7..0): workgroup (block, column),
@@ -174,36 +199,27 @@ __global__ __launch_bounds__(SW) void ntt_small_top_kernel(FastArgs a) {
 template <bool INV, bool DIT>
 __global__ __launch_bounds__(SW) void ntt_small_bottom_kernel(FastArgs a) {
   __shared__ WaveLds sh;
-  const uint32_t l = threadIdx.x;
   const uint64_t c = blockIdx.y, b = blockIdx.x;
   const uint64_t *in = a.in + c * a.stride_in + (b << 8);
   uint64_t *out = a.out + c * a.stride_out + (b << 8);
-  uint64_t tw[9];
-  stage_twiddles(a.tab, l, INV, tw);
+  using W = WaveDft<8, INV, DIT>;
+  const W w(a.tab, threadIdx.x);
   uint64_t x[4];
-  if constexpr (!DIT) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) x[i] = in[64u * i + l];
-    wave_dif256<INV>(x, tw, sh, l);
+  for (int i = 0; i < 4; ++i) x[i] = in[w.pos(W::FIRST, i)];
+  if (a.first) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) out[4u * l + i] = x[i];
-  } else {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) x[i] = in[4u * l + i];
-    if (a.first) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) x[i] = gl::canon(x[i]);
-    }
-    wave_dit256<INV>(x, tw, sh, l);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) out[64u * i + l] = x[i];
+    for (int i = 0; i < 4; ++i) x[i] = gl::canon(x[i]);
   }
+  w.run(x, sh);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) out[w.pos(W::LAST, i)] = x[i];
 }
 
-template <bool INV, bool DIT> hipError_t launch_pair(const FastArgs &top, const FastArgs &bottom, hipStream_t s) {
-  const dim3 grid(256, top.num_cols);
+template <int LH, bool INV, bool DIT> hipError_t launch_pair(const FastArgs &top, const FastArgs &bottom, hipStream_t s) {
+  const dim3 grid(1u << LH, top.num_cols);
   if constexpr (!DIT) {
-    ntt_small_top_kernel<INV, false><<<grid, SW, 0, s>>>(top);
+    ntt_small_top_kernel<LH, INV, false><<<grid, SW, 0, s>>>(top);
     hipError_t err = hipGetLastError();
     if (err != hipSuccess) return err;
     ntt_small_bottom_kernel<INV, false><<<grid, SW, 0, s>>>(bottom);
@@ -211,17 +227,21 @@ template <bool INV, bool DIT> hipError_t launch_pair(const FastArgs &top, const 
     ntt_small_bottom_kernel<INV, true><<<grid, SW, 0, s>>>(bottom);
     hipError_t err = hipGetLastError();
     if (err != hipSuccess) return err;
-    ntt_small_top_kernel<INV, true><<<grid, SW, 0, s>>>(top);
+    ntt_small_top_kernel<LH, INV, true><<<grid, SW, 0, s>>>(top);
   }
   return hipGetLastError();
 }
 
-// Columns of 2^LN points, LN = 1..7: the lower LN bits of a wave's 256-point
-// transform, 2^(8-LN) columns to a wave.  Position p of the wave's 256 values
-// is point p mod 2^LN of its column p / 2^LN; at stage s register i of lane l
-// holds the position with register bits at B = 6 - 2s, and the stages above
-// the columns' length (and the exchanges behind them) fall away.  With odd LN
-// the first stage is radix 2 over its lower bit.
+// `first` reads the caller's input, `second` works in place on the output.
+template <int LH>
+hipError_t launch_small_h(const FastArgs &first, const FastArgs &second, bool bitrev_inputs, bool inverse,
+                          hipStream_t s) {
+  if (!bitrev_inputs)
+    return inverse ? launch_pair<LH, true, false>(first, second, s) : launch_pair<LH, false, false>(first, second, s);
+  return inverse ? launch_pair<LH, true, true>(second, first, s) : launch_pair<LH, false, true>(second, first, s);
+}
+
+// Columns of 2^LN points, LN = 1..7, 2^(8-LN) columns to a wave.
 //
 // A small call is bound by one wave's serial work behind the launch: 256
 // columns of 2^4 / 2^7 points took 8.7-14 / 12-17 us as 4096-point tiles of
@@ -231,84 +251,28 @@ template <bool INV, bool DIT> hipError_t launch_pair(const FastArgs &top, const 
 constexpr uint32_t SHORT_WAVES = 4;  // waves a workgroup of many-column calls has
 template <int LN, bool INV, bool DIT>
 __global__ __launch_bounds__(SHORT_WAVES * SW) void ntt_short_kernel(FastArgs a) {
-  constexpr int S0 = 4 - (LN + 1) / 2;
-  __shared__ WaveLds sh_all[SHORT_WAVES];
-  const uint32_t l = threadIdx.x % SW;
-  WaveLds &sh = sh_all[threadIdx.x / SW];
+  __shared__ WaveLds sh[SHORT_WAVES];
   const uint64_t col0 = ((uint64_t)blockIdx.x * (blockDim.x / SW) + threadIdx.x / SW) << (8 - LN);
-  auto pos = [&](int s, int i) -> uint32_t {
-    const int b = 6 - 2 * s;
-    return ((l >> b) << (b + 2)) | ((uint32_t)i << b) | (l & ((1u << b) - 1u));
-  };
-  // twist of register i behind (DIT: before) stage s
-  uint64_t tw[3][3];
-  static_for<3 - S0>([&](auto k) {
-    constexpr int S = S0 + decltype(k)::value, B = 6 - 2 * S;
-    constexpr bool ODD = S == S0 && LN % 2;
-    const uint32_t rp = l & ((1u << B) - 1u);
-    if constexpr (ODD) {
-      tw[S][0] = root(a.tab, B + 1, rp, INV);
-    } else {
-#pragma unroll
-      for (int i = 1; i < 4; ++i) tw[S][i - 1] = root(a.tab, B + 2, rp * brev2((uint32_t)i), INV);
-    }
-  });
-  auto twist = [&](auto s, uint64_t *x) {
-    constexpr int S = decltype(s)::value;
-    if constexpr (S == 3) return;
-    else if constexpr (S == S0 && LN % 2) {
-      x[1] = gl::mul(x[1], tw[S][0]);
-      x[3] = gl::mul(x[3], tw[S][0]);
-    } else {
-#pragma unroll
-      for (int i = 1; i < 4; ++i) x[i] = gl::mul(x[i], tw[S][i - 1]);
-    }
-  };
-  auto dft = [&](auto s, uint64_t *x) {
-    constexpr int A = decltype(s)::value == S0 && LN % 2 ? 1 : 2;
-#pragma unroll
-    for (int g = 0; g < 4; g += 1 << A) {
-      if constexpr (DIT) dft_dit<A, INV>(x + g);
-      else dft_dif<A, INV>(x + g);
-    }
-  };
-  auto exchange = [&](auto s, uint64_t *x) {  // between stages S and S + 1, either way
-    constexpr int S = decltype(s)::value;
-    if constexpr (S == 0) swap_lane45(x);
-    else if constexpr (S == 1) swap_lanes_lds<2>(x, sh.ex2, l);
-    else if constexpr (S == 2) swap_lanes_lds<0>(x, sh.ex3, l);
-  };
+  using W = WaveDft<LN, INV, DIT>;
+  const W w(a.tab, threadIdx.x % SW);
   uint64_t x[4];
-  constexpr int FIRST = DIT ? 3 : S0, LAST = DIT ? S0 : 3;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const uint32_t p = pos(FIRST, i), j = p & ((1u << LN) - 1u);
+    const uint32_t p = w.pos(W::FIRST, i), j = p & ((1u << LN) - 1u);
     const uint64_t c = col0 + (p >> LN);
     x[i] = c < a.num_cols ? gl::canon(a.in[c * a.stride_in + j]) : 0ull;
   }
   if (!INV && a.log_ext) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const uint32_t j = pos(FIRST, i) & ((1u << LN) - 1u);
+      const uint32_t j = w.pos(W::FIRST, i) & ((1u << LN) - 1u);
       x[i] = gl::mul(x[i], coset_pow(a.tab, a.coset_exp, DIT ? brev_bits(j, LN) : j, false));
     }
   }
-  static_for<4 - S0>([&](auto k) {
-    constexpr int K = decltype(k)::value, S = DIT ? 3 - K : S0 + K;
-    constexpr std::integral_constant<int, S> s{};
-    if constexpr (DIT) {
-      if constexpr (K > 0) exchange(s, x);
-      twist(s, x);
-      dft(s, x);
-    } else {
-      dft(s, x);
-      twist(s, x);
-      if constexpr (S < 3) exchange(s, x);
-    }
-  });
+  w.run(x, sh[threadIdx.x / SW]);
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const uint32_t p = pos(LAST, i), j = p & ((1u << LN) - 1u);
+    const uint32_t p = w.pos(W::LAST, i), j = p & ((1u << LN) - 1u);
     const uint64_t c = col0 + (p >> LN);
     if (c >= a.num_cols) continue;
     uint64_t v = x[i];
@@ -351,18 +315,18 @@ hipError_t launch_short(const FastArgs &a, bool inverse, bool bitrev_inputs, hip
 }
 
 bool small_path_applies(uint32_t log_n, uint32_t num_cols, uint32_t log_ext, const TuneParams &tp) {
-  if (log_n != SMALL_LOG_N || log_ext != 0 || num_cols < 1 || num_cols > 65535) return false;
-  return tp.tile_log == 8 || (tp.tile_log == 0 && num_cols <= SMALL_MAX_COLS);
+  if (log_n < SMALL_MIN_LOG_N || log_n > SMALL_LOG_N || log_ext != 0 || num_cols < 1 || num_cols > 65535) return false;
+  return tp.tile_log == 8 || (tp.tile_log == 0 && num_cols <= (1u << SMALL_LOG_POINTS) >> log_n);
 }
 
-hipError_t launch_small(const Tables &tab, const uint64_t *inputs, uint64_t *outputs, uint32_t num_cols,
-                        uint64_t stride_in, uint64_t stride_out, bool bitrev_inputs, bool inverse, hipStream_t s) {
+hipError_t launch_small(const Tables &tab, const uint64_t *inputs, uint64_t *outputs, uint32_t log_n,
+                        uint32_t num_cols, uint64_t stride_in, uint64_t stride_out, bool bitrev_inputs, bool inverse,
+                        hipStream_t s) {
   FastArgs a{};
   a.tab = tab;
   a.num_cols = num_cols;
-  a.log_n = SMALL_LOG_N;
-  a.n_inv = gl::inv((1ull << SMALL_LOG_N) % gl::P);
-  // the first launch reads the caller's input, the second works in place on the output
+  a.log_n = log_n;
+  a.n_inv = gl::inv((1ull << log_n) % gl::P);
   FastArgs first = a, second = a;
   first.in = inputs;
   first.stride_in = stride_in;
@@ -374,9 +338,13 @@ hipError_t launch_small(const Tables &tab, const uint64_t *inputs, uint64_t *out
   second.out = outputs;
   second.stride_out = stride_out;
   second.first = 0;
-  if (!bitrev_inputs)
-    return inverse ? launch_pair<true, false>(first, second, s) : launch_pair<false, false>(first, second, s);
-  return inverse ? launch_pair<true, true>(second, first, s) : launch_pair<false, true>(second, first, s);
+  switch (log_n) {
+  case 13: return launch_small_h<5>(first, second, bitrev_inputs, inverse, s);
+  case 14: return launch_small_h<6>(first, second, bitrev_inputs, inverse, s);
+  case 15: return launch_small_h<7>(first, second, bitrev_inputs, inverse, s);
+  case 16: return launch_small_h<8>(first, second, bitrev_inputs, inverse, s);
+  default: return hipErrorInvalidValue;
+  }
 }
 
 }  // namespace bc
