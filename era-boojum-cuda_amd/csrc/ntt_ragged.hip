@@ -3,21 +3,23 @@
 //
 // Planning (host).  Every job becomes a chain of passes (describe_fast_passes):
 // an LDE is an inverse transform followed by 2^k coset transforms that all
-// depend on it.  Each (job, stage, pass) is a segment of independent work
-// units (groups of contiguous tiles, or (r-range, pair group) units of a
-// strided pass).  A segment's dependency level is its pass index along its
-// job's chain, and every segment depends only on segments of lower levels.
-// Segments are ordered by level, then by kernel variant, then by job, so the
-// units of one level are one contiguous range of the queue and concurrently
-// running workgroups mostly share code.
+// depend on it.  Equal transforms of several jobs are one group, and each pass
+// of a group is a segment of independent work units (contiguous tiles, or
+// (column, block) pairs at one r-range of a strided pass).  A segment's
+// dependency level is its pass index along its jobs' chain, and every segment
+// depends only on segments of lower levels.  Segments are ordered by level,
+// then by kernel variant, then by group, so the units of one level are one
+// contiguous range of the queue and concurrently running workgroups mostly
+// share code.
 //
-// Execution (device).  The persistent kernel is launched once per level (at
-// most 16 launches for any batch).  Its workgroups pop unit indices from the
-// level's atomic counter, find the unit's segment by binary search and run it
-// with the same pass bodies as the standalone kernels.  Units of one level
-// never wait for each other, so there are no spins and no device-scope
-// fences inside a launch: on gfx950 an agent-scope fence writes back and
-// invalidates the L2 of the XCD, which per unit costs more than the unit.
+// Execution (device).  One persistent launch runs all levels, its workgroups
+// waiting for each other between them (ntt_ragged_all_kernel); where such a
+// launch does not fit, one launch per level (ntt_ragged_kernel).  Workgroups
+// pop unit indices from the level's atomic counter, find the unit's segment
+// through the chunk index and run it with the same pass bodies as the
+// standalone kernels.  Units of one level never wait for each other: on gfx950
+// an agent-scope fence writes back and invalidates the L2 of the XCD, which
+// per unit costs more than the unit.
 #include "ntt_ragged.hpp"
 #include "ntt_passes.hpp"
 

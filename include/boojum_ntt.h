@@ -391,8 +391,8 @@ typedef struct {
   uint32_t ragged_unit_contig;  /* ragged work unit: tiles, <= 64 */
   uint32_t ragged_unit_strided; /* ragged work unit: (column, block) pairs, <= 64 */
   uint32_t tile_log;            /* workgroup tile: 8 = one-wave 256-point passes (log_n 16, no coset, up to 65535
-                                   columns), 12 = 4096-point pass kernels; 0: built-in (256-point for 1..4
-                                   columns of 2^16) */
+                                   columns), 12 = 4096-point pass kernels; 0: built-in (one-wave passes for
+                                   at most 2^18 points in columns of 2^13..2^16) */
 } bc_tune_params;
 
 /* One HBM pass of a planned transform, as bc_batch_ntt_internal would launch
@@ -406,11 +406,11 @@ typedef struct {
   uint64_t positions;           /* strided: r-ranges (grid.x) */
   uint64_t groups;              /* strided: pair groups (grid.y, <= 65535) */
   uint32_t pairs_per_workgroup; /* strided */
-  uint32_t workgroup_threads;   /* 256, or 64 for the one-wave 256-point passes */
+  uint32_t workgroup_threads;   /* 256, or 64 for the one-wave passes */
 } bc_pass_info;
 
 /* The pass plan of bc_batch_ntt_internal for this shape (log_n >= 8; below
- * that one generic pass runs and *num_passes is 0).  Arguments are checked as
+ * that one launch does it all and *num_passes is 0).  Arguments are checked as
  * bc_batch_ntt_internal checks them.  No reference counterpart (the
  * reference's plan is the static PLANS table, src/ntt.rs:74-169). */
 int bc_ntt_describe_plan(uint32_t log_n, uint32_t num_ntts, bool bitrev_inputs, bool inverse,
