@@ -41,10 +41,10 @@ bc_context *current_context() {
 
 // Fixes a strided pass's launch shape for `positions` r-ranges; false if it
 // cannot be launched.
-bool strided_shape(PassDesc &pd, uint64_t positions, uint32_t tuned_bpw, uint32_t *groups) {
+bool strided_shape(PassDesc &pd, uint64_t positions, bool dit, uint32_t tuned_bpw, uint32_t *groups) {
   if (positions > 0x7FFFFFFFull) return false;
   pd.positions = positions;
-  *groups = strided_groups(pd.pairs, positions, tuned_bpw, &pd.a.blocks_per_wg);
+  *groups = strided_groups(pd.pairs, positions, (uint32_t)pd.log_h, dit, tuned_bpw, &pd.a.blocks_per_wg);
   return true;
 }
 
@@ -186,7 +186,7 @@ extern "C" int bc_batch_ntt_internal(const uint64_t *inputs, uint64_t *outputs, 
   uint32_t groups[8] = {};
   for (int k = 0; k < np; ++k) {
     PassDesc &pd = passes[k];
-    if (!pd.contig && !strided_shape(pd, pd.positions, tp.strided_bpw, &groups[k])) return BC_ERROR_INVALID_VALUE;
+    if (!pd.contig && !strided_shape(pd, pd.positions, bitrev_inputs, tp.strided_bpw, &groups[k])) return BC_ERROR_INVALID_VALUE;
   }
   for (int k = 0; k < np; ++k) {
     const PassDesc &pd = passes[k];
@@ -269,7 +269,7 @@ int lde_cosets(bc_context *ctx, const uint64_t *coeffs, uint64_t *outputs, uint3
       pd.a.tiles <<= log_blowup;
       pd.pairs <<= log_blowup;
     }
-    if (!pd.contig && !strided_shape(pd, positions, tp.strided_bpw, &groups[k])) return NOT_BATCHED;
+    if (!pd.contig && !strided_shape(pd, positions, bitrev_coeffs, tp.strided_bpw, &groups[k])) return NOT_BATCHED;
   }
   for (int k = 0; k < np; ++k) {
     const PassDesc &pd = passes[k];
@@ -423,7 +423,8 @@ extern "C" int bc_ntt_describe_plan(uint32_t log_n, uint32_t num_ntts, bool bitr
       if (pd[k].positions > 0x7FFFFFFFull) return BC_ERROR_INVALID_VALUE;
       o.work_items = pd[k].pairs;
       o.positions = pd[k].positions;
-      o.groups = strided_groups(pd[k].pairs, pd[k].positions, tp.strided_bpw, &o.pairs_per_workgroup);
+      o.groups = strided_groups(pd[k].pairs, pd[k].positions, (uint32_t)pd[k].log_h, bitrev_inputs, tp.strided_bpw,
+                                &o.pairs_per_workgroup);
     }
   }
   *num_passes = (uint32_t)np;

@@ -102,7 +102,8 @@ int describe_fast_passes(const Tables &tab, const uint64_t *inputs, uint64_t *ou
 // STRIDED_MAX_GROUPS) and stores the pairs per workgroup in *bpw.  tuned_bpw
 // (0: built-in) is raised when the groups would not fit the grid.
 constexpr uint64_t STRIDED_MAX_GROUPS = 65535;
-uint32_t strided_groups(uint64_t pairs, uint64_t positions, uint32_t tuned_bpw, uint32_t *bpw);
+uint32_t strided_groups(uint64_t pairs, uint64_t positions, uint32_t log_h, bool dit, uint32_t tuned_bpw,
+                        uint32_t *bpw);
 
 // max_wgs: grid cap of a contiguous pass (0: built-in, whole rounds of resident workgroups).
 hipError_t launch_contig(const FastArgs &a, int log_h, bool inverse, bool dit, int mode, uint32_t max_wgs,

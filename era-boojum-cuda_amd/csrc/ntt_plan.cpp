@@ -57,10 +57,25 @@ void make_fast_plan(uint32_t log_n, const TuneParams &tp, FastPlan &pl) {
 
 }  // namespace
 
-uint32_t strided_groups(uint64_t pairs, uint64_t positions, uint32_t tuned_bpw, uint32_t *bpw_out) {
-  // about 2048 (r-range, pair group) workgroups, 1..16 pairs each, unless tuned
+uint32_t strided_groups(uint64_t pairs, uint64_t positions, uint32_t log_h, bool dit, uint32_t tuned_bpw,
+                        uint32_t *bpw_out) {
+  // about 2048 (r-range, pair group) workgroups, 1..16 pairs each, unless
+  // tuned.  Passes of at least 5 bits, whose setup (level and pass twists) costs
+  // more than a pair, take one round of resident workgroups instead (256 CUs x
+  // the kernels' register bounds) where that is at most ONE_ROUND pairs each
+  // and fills the round: 100 coset columns of 2^17 103 -> 96 us (7 pairs; 113 at
+  // the rule's 1), 40 of 2^18 94 -> 78, 30 of 2^18 68 -> 63; part-filled it
+  // loses (6 of 2^19: 28.4 -> 30.2; 32 of 2^19 with the last group a third full:
+  // 111 -> 115).
+  constexpr uint64_t ONE_ROUND = 8;
+  const uint64_t resident = log_h >= 7 && !dit ? 768 : 512;
   uint64_t bpw = pairs * positions / 2048;
   bpw = bpw < 1 ? 1 : (bpw > 16 ? 16 : bpw);
+  const uint64_t round = (pairs * positions + resident - 1) / resident;
+  if (log_h >= 5 && round >= 1 && round <= ONE_ROUND) {
+    const uint64_t groups = (pairs + round - 1) / round, wgs = groups * positions;
+    if (wgs <= resident && wgs * 8 >= resident * 7 && groups * round * 12 <= pairs * 13) bpw = round;
+  }
   if (tuned_bpw) bpw = tuned_bpw;
   // grid.y is at most 65535: larger batches take more pairs per workgroup
   const uint64_t min_bpw = (pairs + STRIDED_MAX_GROUPS - 1) / STRIDED_MAX_GROUPS;
