@@ -259,7 +259,7 @@ struct MatMul {
 };
 
 // A dot product of state words with table constants: six 64-bit sums, one
-// multiply-add per word half and limb.  At most 22 terms, so the sums stay
+// multiply-add per word half and limb.  At most BLOCK terms, so the sums stay
 // below 2^61 (limbs of 24 bits) and 2^53 (16 bits).
 struct Dot {
   uint64_t p0, p1 = 0, p2 = 0, q0, q1 = 0, q2 = 0;
