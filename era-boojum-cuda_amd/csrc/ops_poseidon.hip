@@ -1072,11 +1072,37 @@ template <int H> __device__ __forceinline__ void coop_stage_table(CoopLds &l) {
   }
 }
 
+// Climbs `layers` node layers from a workgroup's COOP_GROUPS digests in LDS,
+// the first of `count` nodes (digests past a short layer's end are not read).
+// Layer l's digests go to its place behind the layers before it.
+template <int H>
+__device__ __forceinline__ void coop_climb(const Coop &c, uint64_t (&digest)[COOP_GROUPS][CAP], uint64_t *results,
+                                           uint32_t count, uint32_t layers, uint32_t group, uint32_t j) {
+  uint32_t active = COOP_GROUPS;
+  for (; layers; --layers) {
+    __syncthreads();
+    active /= 2;
+    const uint64_t g = (uint64_t)blockIdx.x * active + group;
+    uint64_t x = 0;
+    if (j < 2 * CAP && group < active) x = digest[2 * group + (j >> 2)][j & 3u];
+    __syncthreads();
+    if (group < active && g < count) {
+      c.permute_h<H>(x);
+      if (j < CAP) {
+        const uint64_t d = gl::canon(x);
+        results[g + (uint64_t)j * count] = d;
+        digest[group][j] = d;
+      }
+    }
+    results += (uint64_t)CAP * count;
+    count /= 2;
+  }
+}
+
 // `layers` consecutive node layers, the first of `count` nodes: a workgroup
-// hashes COOP_GROUPS nodes of the first layer and keeps their digests in LDS
-// for the next, so one launch climbs up to log2(COOP_GROUPS) + 1 layers
-// (count is a multiple of COOP_GROUPS or below it and a power of two when
-// layers > 1).  Layer l's digests go to its place behind the layers before it.
+// hashes COOP_GROUPS nodes of the first layer and climbs from their digests, so
+// one launch takes up to log2(COOP_GROUPS) + 1 layers (count is a multiple of
+// COOP_GROUPS or below it and a power of two when layers > 1).
 constexpr uint32_t COOP_MAX_LAYERS = 6;
 static_assert(COOP_GROUPS == 1u << (COOP_MAX_LAYERS - 1), "");
 template <int H>
@@ -1087,46 +1113,35 @@ __global__ __launch_bounds__(COOP_NT) void poseidon_nodes_coop_kernel(const uint
   __shared__ uint64_t digest[COOP_GROUPS][CAP];
   coop_stage_table<H>(lds);
   const uint32_t group = threadIdx.x / COOP_LANES, j = threadIdx.x % COOP_LANES;
-  uint64_t g = (uint64_t)blockIdx.x * COOP_GROUPS + group;
+  const uint64_t g = (uint64_t)blockIdx.x * COOP_GROUPS + group;
   // element j: left[j] (j < 4), right[j - 4] (4 <= j < 8), capacity 0
   uint64_t x = 0;
   if (j < 2 * CAP && g < count) x = values[2 * (g + (uint64_t)(j & 3u) * count) + (j >> 2)];
   __syncthreads();
   const Coop c(lds, j, group);
-  uint32_t active = COOP_GROUPS;
-  for (uint32_t l = 0; l < layers; ++l) {
-    const bool on = group < active && g < count;
-    if (on) {
-      c.permute_h<H>(x);
-      if (j < CAP) {
-        const uint64_t d = gl::canon(x);
-        results[g + (uint64_t)j * count] = d;
-        digest[group][j] = d;
-      }
+  if (g < count) {
+    c.permute_h<H>(x);
+    if (j < CAP) {
+      const uint64_t d = gl::canon(x);
+      results[g + (uint64_t)j * count] = d;
+      digest[group][j] = d;
     }
-    if (l + 1 == layers) return;
-    __syncthreads();
-    results += (uint64_t)CAP * count;
-    count /= 2;
-    active /= 2;
-    g = (uint64_t)blockIdx.x * active + group;
-    x = 0;
-    if (j < 2 * CAP && group < active) x = digest[2 * group + (j >> 2)][j & 3u];
-    __syncthreads();
   }
+  coop_climb<H>(c, digest, results + (uint64_t)CAP * count, count / 2, layers - 1, group, j);
 }
 
 // Cooperative leaves (src/poseidon.rs:194-216): the absorption of
 // poseidon_leaves_kernel with one state over a 16-lane row; for each chunk,
 // lane j < 8 takes position off + j (= c rows + r) into state element j, read
-// one chunk ahead.
+// one chunk ahead.  Then up to log2(COOP_GROUPS) node layers (count as above).
 template <int H>
 __global__ __launch_bounds__(COOP_NT) void poseidon_leaves_coop_kernel(const uint64_t *__restrict__ values,
                                                                        uint64_t *__restrict__ results,
                                                                        uint32_t log_rows, uint32_t cols, uint32_t count,
                                                                        bool load_intermediate,
-                                                                       bool store_intermediate) {
+                                                                       bool store_intermediate, uint32_t layers) {
   __shared__ CoopLds lds;
+  __shared__ uint64_t digest[COOP_GROUPS][CAP];
   coop_stage_table<H>(lds);
   const uint32_t group = threadIdx.x / COOP_LANES, j = threadIdx.x % COOP_LANES;
   const uint64_t g = (uint64_t)blockIdx.x * COOP_GROUPS + group;
@@ -1142,20 +1157,23 @@ __global__ __launch_bounds__(COOP_NT) void poseidon_leaves_coop_kernel(const uin
   uint64_t x = 0, next = chunk(0);
   if (on && load_intermediate && j >= RATE && j < PT) x = results[g + (uint64_t)(j - RATE) * count];
   __syncthreads();
-  if (!on) return;  // whole rows leave together, and no barrier follows
   const Coop c(lds, j, group);
-  for (uint64_t off = 0; off < total; off += RATE) {
-    if (j < RATE) x = next;
-    next = chunk(off + RATE);
-    c.permute_h<H>(x);
+  if (on) {  // whole rows together
+    for (uint64_t off = 0; off < total; off += RATE) {
+      if (j < RATE) x = next;
+      next = chunk(off + RATE);
+      c.permute_h<H>(x);
+    }
+    // the digest is state[0..4], the stored capacity state[8..12]
+    x = gl::canon(x);
+    if (store_intermediate) {
+      if (j >= RATE && j < PT) results[g + (uint64_t)(j - RATE) * count] = x;
+    } else if (j < CAP) {
+      results[g + (uint64_t)j * count] = x;
+      digest[group][j] = x;
+    }
   }
-  // the digest is state[0..4], the stored capacity state[8..12]
-  x = gl::canon(x);
-  if (store_intermediate) {
-    if (j >= RATE && j < PT) results[g + (uint64_t)(j - RATE) * count] = x;
-  } else if (j < CAP) {
-    results[g + (uint64_t)j * count] = x;
-  }
+  coop_climb<H>(c, digest, results + (uint64_t)CAP * count, count / 2, layers, group, j);
 }
 
 // ---- Merkle openings: row and path gathers (native/poseidon_common.cu:9-37) --
@@ -1429,7 +1447,7 @@ int launch_leaves(const uint64_t *values, uint64_t *results, uint32_t log_rows, 
   if (count == 0) return BC_SUCCESS;
   if (COOP || count <= COOP_MAX) {
     poseidon_leaves_coop_kernel<H><<<dim3((count + COOP_GROUPS - 1) / COOP_GROUPS), dim3(COOP_NT), 0, s>>>(
-        values, results, log_rows, cols, count, load, store);
+        values, results, log_rows, cols, count, load, store, 0);
   } else {
     poseidon_leaves_kernel<H><<<dim3((count + 255) / 256), dim3(256), 0, s>>>(values, results, 1u << log_rows, cols,
                                                                              count, load, store);
@@ -1527,6 +1545,30 @@ int tree_impl(const uint64_t *values, uint64_t values_len, uint64_t *results, ui
       values_len % leaves != 0)
     return BC_ERROR_INVALID_VALUE;
   const uint64_t half = results_len / 2;
+  // few leaves: their launch also takes the first node layers, one launch and
+  // one staging of the tables less.  Trees of one permutation a leaf, Poseidon /
+  // Poseidon2, with and without: 2^9 leaves 116 / 85 and 121 / 90 us, 2^11 141 /
+  // 103 and 143 / 106, 2^13 167 / 123 and 170 / 126; at 2^14 the workgroups of
+  // the leaves no longer start at once and hold the climb up: 196 / 150 and 191 /
+  // 144 (five permutations 298 / 228 and 283 / 215).
+  const uint64_t rows = 1ull << (log_rows_per_hash & 31u), total = values_len / leaves;
+  if (layers_count > 1 && leaves >= 2 && leaves <= COOP_MAX / 2 && (leaves & (leaves - 1)) == 0 && values && results &&
+      log_rows_per_hash < 32 && total % rows == 0 && total <= 0xFFFFFFFFull) {
+    const int rc = require_table();
+    if (rc != BC_SUCCESS) return rc;
+    constexpr uint32_t MAX_CLIMB = COOP_MAX_LAYERS - 1;
+    const uint32_t climb = layers_count - 1 < MAX_CLIMB ? layers_count - 1 : MAX_CLIMB;
+    const uint32_t count = (uint32_t)leaves;
+    poseidon_leaves_coop_kernel<H>
+        <<<dim3((count + COOP_GROUPS - 1) / COOP_GROUPS), dim3(COOP_NT), 0, (hipStream_t)stream>>>(
+            values, results, log_rows_per_hash, (uint32_t)(total >> log_rows_per_hash), count, false, false, climb);
+    const hipError_t err = hipGetLastError();
+    if (err != hipSuccess) return err;
+    // layer l (l = 0: the leaves) has count >> l digests behind the layers before it
+    for (uint32_t l = 0; l < climb; ++l) results += (uint64_t)CAP * (count >> l);
+    return launch_nodes<H>(results, results + (uint64_t)CAP * (count >> climb), count >> (climb + 1),
+                           layers_count - 1 - climb, (hipStream_t)stream);
+  }
   const int e = leaves_impl<H>(values, values_len, results, half, log_rows_per_hash, false, false, stream);
   if (e != BC_SUCCESS) return e;
   return tree_nodes_impl<H>(results, half, results + half, half, layers_count - 1, stream);

@@ -73,3 +73,24 @@ def test_fused_node_layers(consts, p, log_children, layers):  # noqa: F811
         assert np.array_equal(got[at:at + 4 * count], layer), f"layer {l}"
         at += 4 * count
     assert (got[at:] == guard).all()
+
+
+@pytest.mark.parametrize("log_leaves", [1, 4, 5, 6, 11, 13, 14, 15])
+@pytest.mark.parametrize("p", [0, 1])
+def test_tree_equals_leaves_and_nodes(gpu_ctx, p, log_leaves):
+    """build_merkle_tree (whose leaves' launch climbs the first node layers when
+    they are few) against the leaves and nodes entry points, for every number
+    of layers."""
+    import torch
+    from boojum_cuda_amd import poseidon
+    kind = (poseidon.POSEIDON, poseidon.POSEIDON2)[p]
+    leaves = 1 << log_leaves
+    g = torch.Generator(device="cuda").manual_seed(log_leaves)
+    values = torch.randint(-2**63, 2**63 - 1, (leaves * 2 * 9,), dtype=torch.int64, device="cuda", generator=g)
+    for layers in range(1, log_leaves + 2):
+        want = torch.full((8 * leaves,), -1, dtype=torch.int64, device="cuda")
+        got = want.clone()
+        poseidon.build_merkle_tree_leaves(values, want[:4 * leaves], 1, p=kind)
+        poseidon.build_merkle_tree_nodes(want[:4 * leaves], want[4 * leaves:], layers - 1, p=kind)
+        poseidon.build_merkle_tree(values, got, 1, layers_count=layers, p=kind)
+        assert torch.equal(got, want), layers
