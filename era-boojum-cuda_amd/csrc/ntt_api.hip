@@ -282,6 +282,20 @@ int lde_cosets(bc_context *ctx, const uint64_t *coeffs, uint64_t *outputs, uint3
   return BC_SUCCESS;
 }
 
+// Whether coefficients and outputs of an LDE share memory.  Columns of one
+// stride may also lie between each other's.
+bool lde_overlap(const uint64_t *coeffs, const uint64_t *outputs, uint64_t n, uint64_t num_cols, uint64_t stride_coeffs,
+                 uint64_t stride_out, uint32_t log_blowup) {
+  const uint64_t c0 = (uint64_t)coeffs, o0 = (uint64_t)outputs, out_len = n << log_blowup;
+  if (num_cols == 0 || c0 >= o0 + 8 * ((num_cols - 1) * stride_out + out_len) ||
+      o0 >= c0 + 8 * ((num_cols - 1) * stride_coeffs + n))
+    return false;
+  if (stride_coeffs != stride_out) return true;
+  const uint64_t row = 8 * stride_out;
+  const uint64_t at = c0 >= o0 ? (c0 - o0) % row : (row - (o0 - c0) % row) % row;  // of coefficients in an output row
+  return at < 8 * out_len || at + 8 * n > row;
+}
+
 uint32_t brev_small(uint32_t x, uint32_t bits) {
   uint32_t r = 0;
   for (uint32_t i = 0; i < bits; ++i) r |= ((x >> i) & 1u) << (bits - 1 - i);
@@ -307,7 +321,9 @@ extern "C" int bc_batch_lde(const uint64_t *inputs, uint64_t *coeffs, uint64_t *
   //    bit-reversed evaluations (n2b) and vice versa (b2n)
   bc_context *ctx = current_context();
   if (!ctx) return BC_ERROR_NOT_INITIALIZED;
-  if (n <= stride_coeffs) {
+  // coefficients inside the outputs (a column's last block may hold them) are
+  // overwritten by the coset of their block: that one has to come last
+  if (n <= stride_coeffs && !lde_overlap(coeffs, outputs, n, num_cols, stride_coeffs, stride_out, log_blowup)) {
     rc = lde_cosets(ctx, coeffs, outputs, log_n, num_cols, stride_coeffs, (uint32_t)stride_out, log_blowup,
                     !bitrev_inputs, (hipStream_t)stream);
     if (rc != NOT_BATCHED) return rc;

@@ -87,7 +87,9 @@ int bc_batch_ntt_in_place(uint64_t *inputs_matrix, size_t inputs_len, uint32_t l
  *   inputs:  evaluations, column i at inputs + i * stride_in (n values,
  *            bit-reversed order if bitrev_inputs, else natural)
  *   coeffs:  receives the coefficients (n per column, stride stride_coeffs);
- *            may equal inputs (then the inputs are overwritten)
+ *            may equal inputs (then the inputs are overwritten), or be the
+ *            last of the outputs' blocks (stride_coeffs == stride_out; the
+ *            cosets then run one after the other instead of together)
  *   outputs: column i at outputs + i * stride_out holds 2^log_blowup blocks
  *            of n values.  With bitrev_inputs, block brev(c) holds coset c in
  *            bit-reversed order, so the column is the bit-reversed LDE over
