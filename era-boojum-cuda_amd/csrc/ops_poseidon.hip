@@ -1439,6 +1439,12 @@ int require_table() {
 
 using TableUse = std::shared_lock<std::shared_mutex>;
 
+// Whether a layer's inputs share memory with what the layers above it write.
+// They then have to be read before those layers start, in a launch of their own.
+bool overlap(const uint64_t *a, uint64_t a_len, const uint64_t *b, uint64_t b_len) {
+  return (uintptr_t)a < (uintptr_t)(b + b_len) && (uintptr_t)b < (uintptr_t)(a + a_len);
+}
+
 // COOP: always the cooperative kernel; otherwise the cooperative kernel for
 // at most COOP_MAX leaves and one thread per leaf above.
 template <int H, bool COOP>
@@ -1466,6 +1472,7 @@ int launch_nodes(const uint64_t *values, uint64_t *results, uint32_t count, uint
     uint32_t n = 1;
     if (COOP || count <= COOP_MAX) {
       n = layers < COOP_MAX_LAYERS ? layers : COOP_MAX_LAYERS;
+      if (overlap(values, 2ull * CAP * count, results + (uint64_t)CAP * count, (uint64_t)CAP * count)) n = 1;
       poseidon_nodes_coop_kernel<H>
           <<<dim3((count + COOP_GROUPS - 1) / COOP_GROUPS), dim3(COOP_NT), 0, s>>>(values, results, count, n);
     } else {
@@ -1553,7 +1560,8 @@ int tree_impl(const uint64_t *values, uint64_t values_len, uint64_t *results, ui
   // 144 (five permutations 298 / 228 and 283 / 215).
   const uint64_t rows = 1ull << (log_rows_per_hash & 31u), total = values_len / leaves;
   if (layers_count > 1 && leaves >= 2 && leaves <= COOP_MAX / 2 && (leaves & (leaves - 1)) == 0 && values && results &&
-      log_rows_per_hash < 32 && total % rows == 0 && total <= 0xFFFFFFFFull) {
+      log_rows_per_hash < 32 && total % rows == 0 && total <= 0xFFFFFFFFull &&
+      !overlap(values, values_len, results + half, half)) {
     const int rc = require_table();
     if (rc != BC_SUCCESS) return rc;
     constexpr uint32_t MAX_CLIMB = COOP_MAX_LAYERS - 1;
