@@ -594,17 +594,29 @@ bool column_path(uint64_t count, uint32_t num_polys) {
   return count >= COLUMN_MIN_ROWS && count <= COLUMN_MAX_ROWS && (count >= 128 || num_polys <= COLUMN_FEW);
 }
 
+bool overlap(const uint64_t *a, uint64_t a_len, const uint64_t *b, uint64_t b_len) {
+  return (uintptr_t)a < (uintptr_t)(b + b_len) && (uintptr_t)b < (uintptr_t)(a + a_len);
+}
+
+// Evaluations that go over columns or coefficients other workgroups still read
+// are kept in the partial sums, one to a column, until all have been read
+// (from MIN_TILE_ROWS on, where callers provide these).
 template <uint32_t KIND>
-void launch_column(const uint64_t *ys, const uint64_t *coeffs, uint32_t count, uint32_t num_polys, uint64_t *evals,
-                   hipStream_t s) {
+void launch_column(const uint64_t *ys, const uint64_t *coeffs, uint32_t count, uint32_t num_polys, uint64_t *partial,
+                   uint64_t *evals, hipStream_t s) {
+  constexpr uint64_t YW = KIND == EXT_AT_EXT ? 2 : 1, W = KIND == BASE_AT_BASE ? 1 : 2;
+  const bool hold = count >= MIN_TILE_ROWS && (overlap(evals, W * num_polys, ys, YW * count * num_polys) ||
+                                               overlap(evals, W * num_polys, coeffs, W * count));
+  uint64_t *sums = hold ? partial : evals;
   const bool aligned = !(((uintptr_t)ys | (uintptr_t)coeffs) & 15);
   auto go = [&](auto threads) {
     constexpr uint32_t N = decltype(threads)::value;
-    if (aligned) bary_eval_column_kernel<KIND, true, N><<<dim3(num_polys), N, 0, s>>>(ys, coeffs, count, evals);
-    else bary_eval_column_kernel<KIND, false, N><<<dim3(num_polys), N, 0, s>>>(ys, coeffs, count, evals);
+    if (aligned) bary_eval_column_kernel<KIND, true, N><<<dim3(num_polys), N, 0, s>>>(ys, coeffs, count, sums);
+    else bary_eval_column_kernel<KIND, false, N><<<dim3(num_polys), N, 0, s>>>(ys, coeffs, count, sums);
   };
   if (count <= 512) go(std::integral_constant<uint32_t, 64>{});
   else go(std::integral_constant<uint32_t, 256>{});
+  if (hold) bary_eval_final_kernel<KIND != BASE_AT_BASE><<<dim3(num_polys), BE_NT, 0, s>>>(sums, 1, evals);
 }
 
 template <uint32_t KIND>
@@ -612,7 +624,7 @@ void launch_eval(const uint64_t *ys, const uint64_t *coeffs, uint64_t count, uin
                  uint64_t *evals, hipStream_t s) {
   using T = Shapes<KIND>;
   if (column_path(count, num_polys))
-    launch_column<KIND>(ys, coeffs, (uint32_t)count, num_polys, evals, s);
+    launch_column<KIND>(ys, coeffs, (uint32_t)count, num_polys, partial, evals, s);
   else if (count < COLUMN_MAX_ROWS)
     bary_eval_small_kernel<KIND><<<dim3((num_polys + 255) / 256), 256, 0, s>>>(ys, coeffs, (uint32_t)count,
                                                                                num_polys, evals);
