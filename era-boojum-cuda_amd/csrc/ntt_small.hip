@@ -284,19 +284,30 @@ __global__ __launch_bounds__(SHORT_WAVES * SW) void ntt_short_kernel(FastArgs a)
   }
 }
 
-template <int LN> hipError_t launch_short_ln(const FastArgs &a, bool inverse, bool dit, hipStream_t s) {
-  // one-wave workgroups until the chip has four on every SIMD
-  const uint64_t waves = ((uint64_t)a.num_cols + (1u << (8 - LN)) - 1) >> (8 - LN);
-  const uint32_t per_wg = waves > 4096 ? SHORT_WAVES : 1;
-  const dim3 grid((uint32_t)((waves + per_wg - 1) / per_wg)), block(per_wg * SW);
-  if (inverse) {
-    if (dit) ntt_short_kernel<LN, true, true><<<grid, block, 0, s>>>(a);
-    else ntt_short_kernel<LN, true, false><<<grid, block, 0, s>>>(a);
-  } else {
-    if (dit) ntt_short_kernel<LN, false, true><<<grid, block, 0, s>>>(a);
-    else ntt_short_kernel<LN, false, false><<<grid, block, 0, s>>>(a);
+template <int LN> hipError_t launch_short_ln(const FastArgs &all, bool inverse, bool dit, hipStream_t s) {
+  // A launch takes fewer than 2^32 threads: 2^33 values at a time, a whole
+  // number of workgroups of SHORT_WAVES waves.
+  constexpr uint64_t MAX_COLS = 1ull << (33 - LN);
+  for (uint64_t col = 0; col < all.num_cols; col += MAX_COLS) {
+    FastArgs a = all;
+    a.in += col * a.stride_in;
+    a.out += col * a.stride_out;
+    a.num_cols = (uint32_t)(all.num_cols - col < MAX_COLS ? all.num_cols - col : MAX_COLS);
+    // one-wave workgroups until the chip has four on every SIMD
+    const uint64_t waves = ((uint64_t)a.num_cols + (1u << (8 - LN)) - 1) >> (8 - LN);
+    const uint32_t per_wg = waves > 4096 ? SHORT_WAVES : 1;
+    const dim3 grid((uint32_t)((waves + per_wg - 1) / per_wg)), block(per_wg * SW);
+    if (inverse) {
+      if (dit) ntt_short_kernel<LN, true, true><<<grid, block, 0, s>>>(a);
+      else ntt_short_kernel<LN, true, false><<<grid, block, 0, s>>>(a);
+    } else {
+      if (dit) ntt_short_kernel<LN, false, true><<<grid, block, 0, s>>>(a);
+      else ntt_short_kernel<LN, false, false><<<grid, block, 0, s>>>(a);
+    }
+    const hipError_t err = hipGetLastError();
+    if (err != hipSuccess) return err;
   }
-  return hipGetLastError();
+  return hipSuccess;
 }
 
 }  // namespace
