@@ -81,9 +81,9 @@ GL_FN uint64_t reduce_limbs(uint32_t l0, uint32_t l1, uint32_t l2, uint32_t l3) 
 #if defined(__HIP_DEVICE_COMPILE__)
 // gfx950 building blocks whose carries stay in lane masks (SGPR pairs).  A
 // VALU instruction that reads a lane mask written by another VALU
-// instruction needs two wait states; every block below that consumes such a
-// mask as a carry-in starts with s_nop 1, and masks read by SALU first need
-// none.  The blocks hold no memory operations.
+// instruction needs two wait states: s_nop 1, or two instructions that are sure
+// to stand between.  Masks read by SALU first need none.  The blocks hold no
+// memory operations.
 namespace dev {
 
 // a * b + c as 65 bits: the low 64 bits, and bit 64 in `carry`
@@ -94,10 +94,16 @@ __device__ __forceinline__ uint64_t mad_carry(uint32_t a, uint32_t b, uint64_t c
   return r;
 }
 
+// The wait states of a product's carry c (out of t2) before sub_fold.  The
+// widening of t2 and the multiply-add t3 = a1 b1 + hi(t2) stand there, but for
+// an a1 b1 that is known when compiling (a factor below 2^32, say).  Nothing is
+// emitted otherwise.
+__device__ __forceinline__ void wait_if_known(uint64_t a1b1, uint64_t &c) {
+  if (__builtin_constant_p(a1b1)) asm("s_nop 1" : "+s"(c));
+}
+
 // Y = x - h - cin (cin a lane mask), and n = l less Y's borrow, with n's own
-// borrow in b2.  cin is read without wait states: in a product it comes from
-// the multiply-add t2, and h and l from a widening move and a multiply-add
-// that both follow it.
+// borrow in b2.  cin is read without wait states (wait_if_known).
 __device__ __forceinline__ uint64_t sub_fold(uint32_t x0, uint32_t x1, uint32_t h, uint32_t l, uint64_t cin,
                                              uint32_t &n, uint64_t &b2) {
   uint32_t lo, hi;
@@ -201,6 +207,7 @@ GL_FN uint64_t mul(uint64_t a, uint64_t b) {
   uint32_t n;
   const uint64_t t2 = dev::mad_carry(a1, b0, t1, c);
   const uint64_t t3 = (uint64_t)a1 * b1 + (t2 >> 32);
+  dev::wait_if_known((uint64_t)a1 * b1, c);
   const uint64_t y = dev::sub_fold((uint32_t)t0, (uint32_t)t2, (uint32_t)(t3 >> 32), (uint32_t)t3, c, n, b2);
   const uint64_t z = dev::mad_carry(n, 0xFFFFFFFFu, y, c2);
   return dev::fold_carry(z, c2, b2);

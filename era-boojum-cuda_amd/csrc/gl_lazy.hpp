@@ -17,8 +17,9 @@
 // one instruction and would add wait states between two of them, and it does
 // not know the masks a block writes, so a block that starts by reading one
 // spends the states itself when N < 3 (sub_fold and sub_borrow need not: the
-// mask they read comes from the multiply-add t2, and between the two lie, for
-// every N, the move that widens t2's high word and the multiply-add t3).
+// mask they read comes from the multiply-add t2, and between the two lie the
+// move that widens t2's high word and the multiply-add t3, or, where these are
+// known when compiling and N < 3, dev::wait_if_known).
 //
 // Lazy values.  Inside a DFT a value is V = x + e 2^64 with x any u64 and e a
 // small signed integer: a sum or difference is three carry instructions
@@ -371,6 +372,9 @@ GL_FN void mul_row(uint64_t *o, const uint64_t *a, const uint64_t *b, int32_t *e
     x1[i] = lo32(t2[i]);
     l[i] = lo32(t3);
     h[i] = hi32(t3);
+#if defined(__HIP_DEVICE_COMPILE__)
+    if constexpr (N < 3) dev::wait_if_known((uint64_t)a1[i] * b1[i], c[i]);
+#endif
   });
   uint32_t y0[N], y1[N];
   uint64_t y[N], z[N];
