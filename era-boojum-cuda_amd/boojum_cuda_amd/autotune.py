@@ -189,19 +189,19 @@ def tune_shape(log_n, log_cols, reps=5, log=print):
     def better(ms, incumbent):
         return ms < incumbent * (1.0 - MIN_GAIN)
 
-    # 0. workgroup tile: for 2^16 columns, the one-wave 256-point passes
-    # against the 4096-point pass kernels (whichever the built-in rule does
-    # not pick for this column count); the rest of the search applies to the
-    # 4096-point kernels only
-    if log_n == SMALL_LOG_N:
-        alt = 12 if num_cols << log_n <= 1 << SMALL_LOG_POINTS else 8
+    # 0. workgroup tile: the one-wave passes against the 4096-point pass
+    # kernels (whichever the built-in rule does not pick for this column
+    # count; the one-wave passes can be asked for at 2^16 only).  The rest of
+    # the search applies to the 4096-point kernels, which a shaped entry
+    # selects below 2^16.
+    few = num_cols << log_n <= 1 << SMALL_LOG_POINTS
+    if log_n == SMALL_LOG_N or (SMALL_MIN_LOG_N <= log_n < SMALL_LOG_N and few):
         p = TuneParams()
-        p.tile_log = alt
+        p.tile_log = 12 if few else 8
         ms = trial(p)
         if better(ms, best_ms):
             best, best_ms = p, ms
-    small = best.tile_log == 8 or (SMALL_MIN_LOG_N <= log_n <= SMALL_LOG_N and best.tile_log == 0
-                                   and num_cols << log_n <= 1 << SMALL_LOG_POINTS)
+    small = best.tile_log == 8 or (log_n == SMALL_LOG_N and best.tile_log == 0 and few)
     # 1. pass split (the built-in split itself is not a candidate: an entry
     # that repeats it could only record timing noise)
     for c, k in ([] if small else splits(log_n)):
@@ -219,8 +219,8 @@ def tune_shape(log_n, log_cols, reps=5, log=print):
             ms = trial(p)
             if better(ms, best_ms):
                 best, best_ms = p, ms
-    # 3. contiguous grid cap (the built-in default is two rounds of resident
-    # workgroups; 768 and 2304 are one and three rounds on 256 CUs x 3)
+    # 3. contiguous grid cap (the built-in default is eight rounds of resident
+    # workgroups, 6144 on 256 CUs x 3; 768 and 2304 are one and three rounds)
     for grid in (() if small else (512, 768, 1024, 2304, 4096, 8192)):
         p = TuneParams(*best.key())
         p.contig_grid = grid

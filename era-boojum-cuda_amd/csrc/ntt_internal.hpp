@@ -137,7 +137,9 @@ constexpr uint32_t TILE = 1u << TILE_LOG;
 // 9.2, 10.8, 16.8, the last against 14.1.
 constexpr uint32_t SMALL_MIN_LOG_N = 13, SMALL_LOG_N = 16;
 constexpr uint32_t SMALL_LOG_POINTS = 18;
-// Whether a call of this shape takes the latency path under tuned params tp.
+// Whether a call of this shape takes the latency path under tuned params tp
+// (whose split, pairs and grid take a column shorter than 2^SMALL_LOG_N to the
+// 4096-point passes they are for).
 bool small_path_applies(uint32_t log_n, uint32_t num_cols, uint32_t log_ext, const TuneParams &tp);
 hipError_t launch_small(const Tables &tab, const uint64_t *inputs, uint64_t *outputs, uint32_t log_n,
                         uint32_t num_cols, uint64_t stride_in, uint64_t stride_out, bool bitrev_inputs, bool inverse,

@@ -327,7 +327,9 @@ hipError_t launch_short(const FastArgs &a, bool inverse, bool bitrev_inputs, hip
 
 bool small_path_applies(uint32_t log_n, uint32_t num_cols, uint32_t log_ext, const TuneParams &tp) {
   if (log_n < SMALL_MIN_LOG_N || log_n > SMALL_LOG_N || log_ext != 0 || num_cols < 1 || num_cols > 65535) return false;
-  return tp.tile_log == 8 || (tp.tile_log == 0 && num_cols <= (1u << SMALL_LOG_POINTS) >> log_n);
+  // an entry that shapes the 4096-point passes of a shorter column asks for them
+  const bool shaped = log_n != SMALL_LOG_N && (tp.contig_log || tp.strided_bpw || tp.contig_grid);
+  return tp.tile_log == 8 || (tp.tile_log == 0 && !shaped && num_cols <= (1u << SMALL_LOG_POINTS) >> log_n);
 }
 
 hipError_t launch_small(const Tables &tab, const uint64_t *inputs, uint64_t *outputs, uint32_t log_n,

@@ -394,7 +394,9 @@ typedef struct {
   uint32_t ragged_unit_strided; /* ragged work unit: (column, block) pairs, <= 64 */
   uint32_t tile_log;            /* workgroup tile: 8 = one-wave 256-point passes (log_n 16, no coset, up to 65535
                                    columns), 12 = 4096-point pass kernels; 0: built-in (one-wave passes for
-                                   at most 2^18 points in columns of 2^13..2^16) */
+                                   at most 2^18 points in columns of 2^13..2^16, and for columns
+                                   below 2^16 only if no field above that shapes the 4096-point
+                                   passes, contig_log to contig_grid, is set) */
 } bc_tune_params;
 
 /* One HBM pass of a planned transform, as bc_batch_ntt_internal would launch
