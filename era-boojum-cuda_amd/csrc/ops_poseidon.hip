@@ -1608,6 +1608,7 @@ extern "C" int bc_poseidon_set_round_constants(const uint64_t *round_constants) 
   // while the lock is held)
   err = hipDeviceSynchronize();
   if (err != hipSuccess) return err;
+  pos_ready[dev] = false;  // until all tables are new
   err = hipMemcpyToSymbol(HIP_SYMBOL(pos_table), &t, sizeof t, 0, hipMemcpyHostToDevice);
   if (err != hipSuccess) return err;
   err = hipMemcpyToSymbol(HIP_SYMBOL(pos_fast), &f, sizeof f, 0, hipMemcpyHostToDevice);

@@ -272,7 +272,8 @@ int bc_batch_eval(uint32_t kind, const uint64_t *ys, uint64_t stride, uint32_t n
  * table lock exclusively (hashing calls on other threads wait for it), waits
  * for all work queued on the device (hashing kernels read the table), then
  * replaces the table.  Every hashing call on a device returns
- * BC_ERROR_NOT_INITIALIZED until this has been called there. */
+ * BC_ERROR_NOT_INITIALIZED until this has been called there, and again after
+ * a call that failed while it replaced the table. */
 int bc_poseidon_set_round_constants(const uint64_t *round_constants);
 
 /* Host only (no device call): the per-device table derived from 360
