@@ -27,9 +27,6 @@ __device__ __forceinline__ uint64_t pow_w(const Tables &t, uint32_t e) {
   return f ? gl::mul(c, t.w_fine[f]) : c;
 }
 
-// omega_{2^32}^E for E a multiple of 2^16.
-__device__ __forceinline__ uint64_t pow_w_coarse(const Tables &t, uint32_t e) { return t.w_coarse[e >> TABLE_LOG]; }
-
 __device__ __forceinline__ uint64_t pow_g(const Tables &t, uint32_t i, bool inverse) {
   const uint64_t *fine = inverse ? t.gi_fine : t.g_fine;
   const uint64_t *coarse = inverse ? t.gi_coarse : t.g_coarse;

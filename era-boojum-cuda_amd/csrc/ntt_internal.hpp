@@ -61,7 +61,6 @@ struct FastArgs {
   uint32_t log_ext;
   uint32_t coset_exp;
   uint32_t first;          // pass reads the caller's (possibly non-canonical) input
-  uint32_t last;           // pass writes the final (canonical) output
   uint32_t tiles;          // contiguous passes: number of 4096-point tiles
   uint32_t blocks_per_wg;  // strided passes: (column, block) pairs per workgroup
   const ColPtrs *cols;     // column-table addressing (ragged): column c at cols[c], in/out/strides unused

@@ -111,7 +111,6 @@ int describe_fast_passes(const Tables &tab, const uint64_t *inputs, uint64_t *ou
     pd.a.out = outputs;
     pd.a.stride_out = stride_out;
     pd.a.first = first;
-    pd.a.last = last;
     pd.positions = pd.pairs = 0;
     if (p == np - 1) {
       int mode = MODE_NONE;
