@@ -447,7 +447,10 @@ extern "C" int bc_ragged_run_plain(const bc_ragged_job *jobs, uint32_t num_jobs,
 // hipGetSymbolAddress returns (each GPU holds its own copy).
 namespace bc {
 namespace {
-constexpr size_t NOALLOC_SCRATCH_BYTES = (size_t)8 << 20;
+// 8 MiB, and room for the chunk index of smaller work units than 32 tiles,
+// which all but the largest levels are split into: a few thousand more units a
+// level, 4 bytes for every 64.
+constexpr size_t NOALLOC_SCRATCH_BYTES = ((size_t)8 << 20) + ((size_t)64 << 10);
 constexpr int NOALLOC_MAX_DEVICES = 64;
 }  // namespace
 }  // namespace bc

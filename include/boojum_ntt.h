@@ -171,8 +171,9 @@ int bc_ragged_run_plain(const bc_ragged_job *jobs, uint32_t num_jobs, void *stre
  * hipMalloc/hipFree, no allocator of any library.  No counterpart in the
  * reference; it is for callers that cannot allocate (tight serving loops,
  * harnesses that forbid it).  The packed plan table and the queue state go to
- * a static 8 MiB device array that every GPU running the library keeps until
- * the process ends; a plan that needs more returns BC_ERROR_OUT_OF_MEMORY
+ * a static device array (8 MiB + 64 KiB) that every GPU running the library
+ * keeps until the process ends; a plan that needs more returns
+ * BC_ERROR_OUT_OF_MEMORY
  * before anything is launched (the 1000-job ragged benchmark batch takes
  * about 0.12 MiB).  The table is uploaded from pageable host memory, which HIP
  * copies synchronously, then the plan is launched on `stream` once per
