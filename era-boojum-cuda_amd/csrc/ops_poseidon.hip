@@ -887,7 +887,10 @@ __device__ __forceinline__ uint64_t coop_sbox_terms(uint64_t x, uint64_t vx, uin
 }
 #undef BC_ROR
 
-// a b + lo + hi 2^32 (lo, hi < 2^52), any u64.
+// a b + lo + hi 2^32, any u64, for the sums of a partial round: in a lane of
+// words 1..11 lo, hi <= 2^33 - 2 (two 32-bit terms) and the low word of a is
+// below 2^32 - 1 (derive_lanes), so a0 b0 + lo and a0 b1 + hi + (a0 b0 + lo) / 2^32
+// stay below 2^64; in lane 0 a = 1 and lo, hi < 2^52.
 __device__ __forceinline__ uint64_t coop_mul_add(uint64_t a, uint64_t b, uint64_t lo, uint64_t hi) {
   const uint64_t p = (uint64_t)gl::lo32(a) * gl::lo32(b) + lo;
   uint64_t t = (uint64_t)gl::lo32(a) * gl::hi32(b) + (hi + gl::hi32(p));
@@ -1358,16 +1361,20 @@ void set_mat(PosMat &m, int mat, uint64_t (*kout)[2], int outputs, const uint64_
   }
 }
 
-void derive_lanes(const PosTable &t, PartialLane (*lanes)[PT]) {
+// False if a column entry does not suit coop_mul_add (the MDS matrix alone
+// decides that, not the round constants).
+bool derive_lanes(const PosTable &t, PartialLane (*lanes)[PT]) {
   for (int k = 0; k < PARTIAL; ++k)
     for (int j = 0; j < PT; ++j) {
       PartialLane &l = lanes[k][j];
       l.v = j ? t.vs[k][j - 1] : 0;
       l.w = j ? t.w_hats[k][j - 1] : 1;
+      if ((uint32_t)l.w == 0xFFFFFFFFu) return false;
       const uint64_t c = gl::mul(l.w, t.sbox_c[k]);
       l.k[0] = (uint32_t)c;
       l.k[1] = c >> 32;
     }
+  return true;
 }
 
 // The one-lane forms' tables from the fused one.
@@ -1601,7 +1608,7 @@ extern "C" int bc_poseidon_set_round_constants(const uint64_t *round_constants) 
   std::vector<PosMat> m(1);
   derive_fast(t, f, m[0]);
   PartialLane lanes[PARTIAL][PT];
-  derive_lanes(t, lanes);
+  if (!derive_lanes(t, lanes)) return BC_ERROR_INVALID_VALUE;
   std::unique_lock<std::shared_mutex> lk(pos_mu);
   // hashing kernels already queued on any stream of this device read the
   // table: let them finish before it changes (no new ones can be queued
