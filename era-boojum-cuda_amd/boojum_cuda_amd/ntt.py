@@ -79,7 +79,7 @@ class _PassInfo(ctypes.Structure):
 
 def describe_plan(log_n, num_ntts, bitrev_inputs=False, inverse=False, log_extension_degree=0, coset_index=0):
     """The HBM passes batch_ntt_internal launches for this shape, as dicts
-    (host only, no device needed).  Empty for log_n < 8 (one generic pass)."""
+    (host only, no device needed).  Empty for log_n < 8 (one launch does it all)."""
     arr = (_PassInfo * 8)()
     n = ctypes.c_uint32()
     rc = lib().bc_ntt_describe_plan(log_n, num_ntts, bool(bitrev_inputs), bool(inverse), log_extension_degree,

@@ -9,9 +9,10 @@ namespace {
 using namespace pass;
 
 // Register bounds: three workgroups per CU for the n2b variants and the
-// 12-bit b2n ones (160-168 VGPRs, no spills in the plain forms), two for the
-// shorter b2n ones, some of which need more.  Four per CU spills 18-20 dwords
-// in the 12-bit kernels and ran 4-5% slower.
+// 12-bit b2n ones, two for the shorter b2n ones, some of which need more (up to
+// 204 VGPRs).  The 12-bit kernels take 150-168 VGPRs without spills; n2b ones
+// of 10 and 11 bits spill up to 6 dwords.  Four per CU spills 18-20 dwords in
+// the 12-bit kernels and ran 4-5% slower.
 template <int LH, bool INV, bool DIT, int MODE, bool MC>
 __global__ __launch_bounds__(NT, DIT && LH != 12 ? 2 : 3) void
     ntt_contig_kernel(FastArgs a) {
@@ -26,9 +27,11 @@ __global__ __launch_bounds__(NT, DIT && LH != 12 ? 2 : 3) void
   contig_run<LH, INV, DIT, MODE, MC>(a, sh, wg, a.tiles, wgs);
 }
 
-// Three workgroups per CU for n2b h = 7 and 8 (2-6 spilled dwords; two per CU
-// was 5-6% slower on 256 x 2^20), two for the others, which spill 10-84 dwords
-// at three (b2n h = 8 runs the same at both: 0.97 ms on 256 x 2^20).
+// No form spills VGPRs.  n2b h = 7 and 8 take 155-166 and are bounded to three
+// workgroups per CU (at two the compiler takes more: 5-6% slower on 256 x
+// 2^20).  The others are bounded to two: h = 5 and 6 and the inverse coset forms
+// need 171-196 and run two, plain h = 4 (139-147) and plain b2n h = 7 and 8 (167
+// and 163) run three under that bound as well.
 template <int LH, bool INV, bool DIT, int MODE>
 __global__ __launch_bounds__(NT, LH >= 7 && !DIT ? 3 : 2) void ntt_strided_kernel(FastArgs a) {
   __shared__ PassLds sh;

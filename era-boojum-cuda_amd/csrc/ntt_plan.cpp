@@ -61,12 +61,16 @@ uint32_t strided_groups(uint64_t pairs, uint64_t positions, uint32_t log_h, bool
                         uint32_t *bpw_out) {
   // about 2048 (r-range, pair group) workgroups, 1..16 pairs each, unless
   // tuned.  Passes of at least 5 bits, whose setup (level and pass twists) costs
-  // more than a pair, take one round of resident workgroups instead (256 CUs x
-  // the kernels' register bounds) where that is at most ONE_ROUND pairs each
-  // and fills the round: 100 coset columns of 2^17 103 -> 96 us (7 pairs; 113 at
-  // the rule's 1), 40 of 2^18 94 -> 78, 30 of 2^18 68 -> 63; part-filled it
-  // loses (6 of 2^19: 28.4 -> 30.2; 32 of 2^19 with the last group a third full:
-  // 111 -> 115).
+  // more than a pair, take one round of workgroups instead (256 CUs x the
+  // kernels' register bounds) where that is at most ONE_ROUND pairs each and
+  // fills the round: 100 coset columns of 2^17 103 -> 96 us (7 pairs; 113 at the
+  // rule's 1), 40 of 2^18 94 -> 78, 30 of 2^18 68 -> 63; part-filled it loses (6
+  // of 2^19: 28.4 -> 30.2; 32 of 2^19 with the last group a third full: 111 ->
+  // 115).  Plain b2n h = 7 and 8 run three workgroups per CU, but 512 is the
+  // better round for them too: 8, 12 and 16 inverse columns of 2^19 take 34.9,
+  // 47.8 and 64.0 us in it (2, 3, 4 pairs), 36.5, 49.9 and 64.0 with the pairs of
+  // a round of 768 (1, 2, 3); 4, 6, 8 and 12 of 2^20 36.6, 50.4, 65.8 and 92.4
+  // against 38.8, 49.9, 65.2 and 93.0.
   constexpr uint64_t ONE_ROUND = 8;
   const uint64_t resident = log_h >= 7 && !dit ? 768 : 512;
   uint64_t bpw = pairs * positions / 2048;

@@ -587,7 +587,10 @@ void launch_tiles(const uint64_t *ys, const uint64_t *coeffs, uint64_t count, ui
 // kernel against the others: 20 columns of 2^5 / 2^6 / 2^8 / 2^10 / 2^12 rows
 // 18.2 / 18.4 / 18.8 / 19.9 / 23.9 us against 19.8 / 23.9 / 20.4 / 21.2 / 22.0
 // (2^3: 18.6 against 16.6), 40000 columns of 2^7 / 2^8 rows 34 / 40 against 74 /
-// 82 us, of 2^5 32 against 24, 4000 of 2^10 28 against 31.
+// 82 us, of 2^5 32 against 24, 4000 of 2^10 28 against 31.  Evaluations alone,
+// base columns at base points / extension columns: 20 columns of 2^6 and 2^10
+// rows 7.0 and 7.1 / 7.1 and 7.0 us against 8.0 and 10.3 / 14.1 and 10.4, 4000 of
+// 2^10 7.3 / 16.8 against 10.3 / 22.8, 40000 of 2^7 11.6 / 24 against 32.6 / 68.
 constexpr uint64_t COLUMN_MIN_ROWS = 32, COLUMN_MAX_ROWS = 1024;
 constexpr uint32_t COLUMN_FEW = 8192;
 bool column_path(uint64_t count, uint32_t num_polys) {

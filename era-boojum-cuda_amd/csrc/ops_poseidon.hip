@@ -29,15 +29,15 @@
 // 1..11 pass that S-box untouched.
 //
 // One lane hashes one leaf or node: the permutation is a serial chain of field
-// products with no data shared between hashes, and 12 state words fit in 128
-// registers, four waves per SIMD.  A wave's 64 states take Poseidon's matrix
+// products with no data shared between hashes, at four waves per SIMD (122-128
+// registers for Poseidon, 8 more spilled by its leaves; 76 for Poseidon2).  A wave's 64 states take Poseidon's matrix
 // products to the matrix cores together (MatMul).  Bound: vector issue slots:
 // about 10.3k vector instructions per Poseidon permutation, 60% of them S-box
-// products, and 11.9k (cheaper ones) per Poseidon2 permutation, against 64
+// products, and 10.4k (cheaper ones) per Poseidon2 permutation, against 64
 // bytes absorbed.  With every word reduced to [0, p) in every step, products
 // one at a time and sparse partial rounds it was 24.8k and 16.4k; 128 columns
 // x 2^20 rows: 10.7 -> 5.5 ms a Poseidon tree, 2^18 leaves of 2 x 93 values:
-// 3.30 -> 1.97 ms a Poseidon2 tree.
+// 3.28 -> 1.82 ms a Poseidon2 tree.
 #include "../../include/boojum_ntt.h"
 #include "gl_lazy.hpp"
 
